@@ -4,12 +4,14 @@
 // layer but the last.  Activations, gradients and the optimiser state are FP32; every matrix
 // product runs on v_mfma_f32_16x16x16bf16_1k with BF16 operands and FP32 accumulation.
 //
-// One GEMM kernel serves every product: C[m][n] = sum_k A(m,k) B(k,n) with arbitrary element
-// strides for A and B (so X W^T, dZ^T H and dZ W are the same kernel), a 64x64 block tile,
-// 16-deep K steps staged through LDS as BF16, four wavefronts each owning a 32x32 sub-tile
-// (2x2 MFMA tiles).  Long reductions (the weight gradient sums over all nodes) are split over
-// grid.z into FP32 partials that a second kernel adds in split order, so every result is
-// bitwise reproducible.
+// Networks of width <= 128 (every width of the nodal predictors) run in four launches: the whole
+// forward pass, the whole chain of hidden gradients, every weight gradient, and the reduction of
+// the partial sums (see "Narrow networks" below).  Wider ones take one GEMM launch per product:
+// C[m][n] = sum_k A(m,k) B(k,n) with arbitrary element strides for A and B (so X W^T, dZ^T H and
+// dZ W are the same kernel), a 64x64 block tile, 16-deep K steps staged through LDS as BF16, four
+// wavefronts each owning a 32x32 sub-tile (2x2 MFMA tiles).  Long reductions (the weight and bias
+// gradients sum over all nodes) are split into FP32 partials that a second kernel adds in a fixed
+// order, so every result is bitwise reproducible.
 #include "fne_common.h"
 
 namespace {
@@ -135,16 +137,27 @@ __global__ __launch_bounds__(256) void mlp_split_reduce_kernel(const float* __re
   out[i] = s;
 }
 
-// column sums of X [rows][cols] over row chunks of 1024 -> part[chunk][cols]
+// column sums of X [rows][cols] over row chunks of kColsumRows -> part[chunk][cols].  A thread
+// sums kColsumRows / 4 rows of one column (64 neighbouring columns per wavefront, so loads
+// coalesce), the four wavefronts' sums are added in order.
+constexpr int kColsumRows = 256;
+
 __global__ __launch_bounds__(256) void mlp_colsum_kernel(const float* __restrict__ X, long rows, int cols,
                                                          float* __restrict__ part) {
-  const int c = blockIdx.y * blockDim.x + threadIdx.x;
-  if (c >= cols) return;
-  const long r0 = long(blockIdx.x) * 1024;
-  const long r1 = r0 + 1024 < rows ? r0 + 1024 : rows;
+  __shared__ float sums[4][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c = blockIdx.y * 64 + lane;
+  const long r0 = long(blockIdx.x) * kColsumRows;
   float s = 0.f;
-  for (long r = r0; r < r1; ++r) s += X[size_t(r) * cols + c];
-  part[size_t(blockIdx.x) * cols + c] = s;
+  if (c < cols) {
+#pragma unroll 8
+    for (int r = wave; r < kColsumRows; r += 4)
+      if (r0 + r < rows) s += X[size_t(r0 + r) * cols + c];
+  }
+  sums[wave][lane] = s;
+  __syncthreads();
+  if (wave == 0 && c < cols)
+    part[size_t(blockIdx.x) * cols + c] = (sums[0][lane] + sums[1][lane]) + (sums[2][lane] + sums[3][lane]);
 }
 
 __global__ __launch_bounds__(256) void mlp_adam_kernel(long n, float* __restrict__ w, unsigned short* __restrict__ wb,
@@ -167,6 +180,356 @@ __global__ __launch_bounds__(256) void mlp_to_bf16_kernel(long n, const float* _
                                                           unsigned short* __restrict__ wb) {
   const long i = long(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i < n) wb[i] = f2bf(w[i]);
+}
+
+// ---------------------------------------------------------------------------------------------
+// Narrow networks (every width <= kNarrow = 128).
+//
+// A 10-128x4-3 network on 16,384 rows is 5 GFLOP and 8 MB per hidden activation: one launch per
+// product (25 of them, 64x64 tiles read and written through memory, a bias-gradient column sum of
+// 1,024 serial loads per thread) took 1,475 us on an MI355X for forward + backward, of which the
+// arithmetic needs under 10.  Here a workgroup keeps its R rows in LDS (BF16) through all
+// layers; a wavefront holds the weight fragments of its 32 columns in registers, so a layer costs
+// one LDS read per 16x16 input tile and two MFMAs.  The order of every accumulation (16-deep
+// steps, k ascending, then bias, tanh) is that of the GEMM kernel: activations and hidden
+// gradients have the same bits in both forms.  Measured (forward + backward of 10-128x4-3, 16,384
+// rows): 1,475 -> 113 us, of which forward 37.6 (tanhf and 34 MB of activations written), chain
+// 34.3, weight gradients 34.2 (67 MB read at 2 TB/s), reduction 5.7.
+// ---------------------------------------------------------------------------------------------
+constexpr int kNarrow = 128;
+constexpr int kNarrowStride = kNarrow + 8;  // LDS row of BF16: 272 B, so 16 rows start in 16 bank groups
+
+typedef __bf16 mlp_b8 __attribute__((ext_vector_type(8)));
+typedef unsigned short mlp_u8 __attribute__((ext_vector_type(8)));
+
+// FP32 -> BF16 by the conversion instruction (round to nearest even, as f2bf; a NaN stays a NaN)
+__device__ __forceinline__ unsigned short cvt_bf(float f) {
+  return __builtin_bit_cast(unsigned short, static_cast<__bf16>(f));
+}
+
+// rows per workgroup: 32 put two workgroups on every CU at 16,384 rows (forward + chain 71.8 us;
+// 16 rows 80.7: the weights are loaded twice as often; 64 rows 94.9: one workgroup per CU)
+constexpr int kNarrowRows = 32;
+
+// layer l's 16x16x16 products over the workgroup's rows: acc[mt][j] for column tiles 2 wave + j
+template <int R>
+__device__ __forceinline__ void narrow_products(const unsigned short (*sA)[kNarrowStride], const mlp_s4 (*bf)[8],
+                                                int ksteps, int lane, mlp_f4 (*acc)[2]) {
+#pragma unroll
+  for (int mt = 0; mt < R / 16; ++mt) acc[mt][0] = acc[mt][1] = mlp_f4{0.f, 0.f, 0.f, 0.f};
+  const int kq = 4 * (lane >> 4);
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    if (s < ksteps) {
+#pragma unroll
+      for (int mt = 0; mt < R / 16; ++mt) {
+        const mlp_s4 a = *reinterpret_cast<const mlp_s4*>(&sA[mt * 16 + (lane & 15)][16 * s + kq]);
+        acc[mt][0] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bf[0][s], acc[mt][0], 0, 0, 0);
+        acc[mt][1] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bf[1][s], acc[mt][1], 0, 0, 0);
+      }
+    }
+  }
+}
+
+// the workgroup's rows of X [n][cols] as BF16, columns padded with zeros to a multiple of 16
+template <int R>
+__device__ __forceinline__ void narrow_load_rows(const float* __restrict__ X, long n, long row0, int cols,
+                                                 unsigned short (*sA)[kNarrowStride]) {
+  const int kp = (cols + 15) & ~15;
+  for (int i = threadIdx.x; i < R * kp; i += 256) {
+    const int r = i / kp, k = i - r * kp;
+    sA[r][k] = (row0 + r < n && k < cols) ? cvt_bf(X[size_t(row0 + r) * cols + k]) : 0;
+  }
+}
+
+template <int R>
+__global__ __launch_bounds__(256) void mlp_narrow_forward_kernel(fne_mlp_desc net, long n, const float* __restrict__ x,
+                                                                 float* __restrict__ y, float* __restrict__ acts) {
+  __shared__ unsigned short sA[R][kNarrowStride];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c15 = lane & 15, kq = 4 * (lane >> 4);
+  const long row0 = long(blockIdx.x) * R;
+  narrow_load_rows<R>(x, n, row0, net.dims[0], sA);
+  size_t off = 0;
+  for (int l = 0; l < net.n_layers; ++l) {
+    const int din = net.dims[l], dout = net.dims[l + 1];
+    const bool last = l == net.n_layers - 1;
+    const unsigned short* W = net.w[l];
+    const int ksteps = (din + 15) >> 4;
+    const bool vec = (din & 3) == 0 && (reinterpret_cast<uintptr_t>(W) & 7u) == 0;  // 8-byte fragments
+    mlp_s4 bf[2][8];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int col = (2 * wave + j) * 16 + c15;
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        mlp_s4 b = {0, 0, 0, 0};
+        const int k = 16 * s + kq;
+        if (s < ksteps && col < dout) {
+          const unsigned short* w = W + size_t(col) * din + k;  // B(k, col) = W[col][k]
+          if (vec) {
+            if (k < din) b = *reinterpret_cast<const mlp_s4*>(w);
+          } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              if (k + q < din) b[q] = (short)w[q];
+          }
+        }
+        bf[j][s] = b;
+      }
+    }
+    __syncthreads();  // the rows are in LDS
+    mlp_f4 acc[R / 16][2];
+    narrow_products<R>(sA, bf, ksteps, lane, acc);
+    __syncthreads();  // every read of the rows is done
+    float* out = last ? y : acts + off;
+    const float* bias = net.b[l];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int col = (2 * wave + j) * 16 + c15;
+      if (col >= ((dout + 15) & ~15)) continue;
+      const float bj = col < dout ? bias[col] : 0.f;
+#pragma unroll
+      for (int mt = 0; mt < R / 16; ++mt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int row = mt * 16 + kq + r;
+          float v = 0.f;
+          if (col < dout) {
+            v = acc[mt][j][r] + bj;
+            if (!last) v = tanhf(v);
+            if (row0 + row < n) out[size_t(row0 + row) * dout + col] = v;
+          }
+          if (!last) sA[row][col] = cvt_bf(v);
+        }
+    }
+    if (!last) off += size_t(n) * dout;
+  }
+}
+
+// hidden gradients dz_{l-1} = (dz_l W_l) (1 - h_{l-1}^2) for l = L-1 .. 1, written back to back in
+// acts' layout, and the column sums of every dz over the workgroup's rows (cpart [blocks][sum of
+// widths], layer l at the sum of the widths before it)
+template <int R>
+__global__ __launch_bounds__(256) void mlp_narrow_chain_kernel(fne_mlp_desc net, long n,
+                                                               const float* __restrict__ acts,
+                                                               const float* __restrict__ dy, float* __restrict__ dz,
+                                                               float* __restrict__ cpart, int widths) {
+  __shared__ unsigned short sA[R][kNarrowStride];
+  __shared__ unsigned short sW[kNarrow][kNarrowStride];  // W_l transposed: [input][output]
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int c15 = lane & 15, kq = 4 * (lane >> 4);
+  const long row0 = long(blockIdx.x) * R;
+  const int L = net.n_layers;
+  float* cp = cpart + size_t(blockIdx.x) * widths;
+  size_t off = 0;  // of dz_{L-2} in acts' layout
+  int coff = widths - net.dims[L];
+  for (int l = 0; l + 2 < L; ++l) off += size_t(n) * net.dims[l + 1];
+  narrow_load_rows<R>(dy, n, row0, net.dims[L], sA);
+  for (int c = threadIdx.x; c < net.dims[L]; c += 256) {
+    float s = 0.f;
+    for (int r = 0; r < R; ++r)
+      if (row0 + r < n) s += dy[size_t(row0 + r) * net.dims[L] + c];
+    cp[coff + c] = s;
+  }
+  for (int l = L - 1; l > 0; --l) {
+    const int din = net.dims[l], dout = net.dims[l + 1];
+    const unsigned short* W = net.w[l];
+    const int ksteps = (dout + 15) >> 4;
+    // four rows by eight columns of W at a time (16-byte loads where the rows allow), zero-padded
+    // to whole K steps
+    const int kp = 16 * ksteps;
+    const bool vec = (din & 7) == 0 && (reinterpret_cast<uintptr_t>(W) & 15u) == 0;
+    const int cg = (din + 7) >> 3;
+    for (int u = threadIdx.x; u < (kp >> 2) * cg; u += 256) {
+      const int k0 = (u / cg) * 4, col0 = (u % cg) * 8;
+      mlp_u8 w[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        w[q] = mlp_u8{0, 0, 0, 0, 0, 0, 0, 0};
+        if (k0 + q < dout) {
+          const unsigned short* src = W + size_t(k0 + q) * din + col0;
+          if (vec) {
+            w[q] = *reinterpret_cast<const mlp_u8*>(src);
+          } else {
+#pragma unroll
+            for (int t = 0; t < 8; ++t)
+              if (col0 + t < din) w[q][t] = src[t];
+          }
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < 8; ++t)
+        *reinterpret_cast<mlp_s4*>(&sW[col0 + t][k0]) =
+            mlp_s4{short(w[0][t]), short(w[1][t]), short(w[2][t]), short(w[3][t])};
+    }
+    const float* H = acts + off;
+    float hv[2][R / 16][4];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int mt = 0; mt < R / 16; ++mt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int col = (2 * wave + j) * 16 + c15;
+          const long row = row0 + mt * 16 + kq + r;
+          hv[j][mt][r] = (col < din && row < n) ? H[size_t(row) * din + col] : 0.f;
+        }
+    __syncthreads();  // rows and weights are in LDS
+    mlp_s4 bf[2][8];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int s = 0; s < 8; ++s)
+        if (s < ksteps) bf[j][s] = *reinterpret_cast<const mlp_s4*>(&sW[(2 * wave + j) * 16 + c15][16 * s + kq]);
+    mlp_f4 acc[R / 16][2];
+    narrow_products<R>(sA, bf, ksteps, lane, acc);
+    __syncthreads();  // every read of the rows and weights is done
+    coff -= din;
+    float* out = dz + off;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int col = (2 * wave + j) * 16 + c15;
+      if (col >= ((din + 15) & ~15)) continue;
+      float s = 0.f;
+#pragma unroll
+      for (int mt = 0; mt < R / 16; ++mt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int row = mt * 16 + kq + r;
+          float v = 0.f;
+          if (col < din && row0 + row < n) {
+            const float h = hv[j][mt][r];
+            v = acc[mt][j][r] * (1.0f - h * h);
+            out[size_t(row0 + row) * din + col] = v;
+            s += v;
+          }
+          if (l > 1) sA[row][col] = cvt_bf(v);
+        }
+      s += __shfl_xor(s, 16, 64);
+      s += __shfl_xor(s, 32, 64);
+      if (lane < 16 && col < din) cp[coff + col] = s;
+    }
+    if (l > 1) off -= size_t(n) * net.dims[l - 1];
+  }
+}
+
+// weight gradients dW_l = dz_l^T h_{l-1}, all layers in one launch: blockIdx.y is the layer,
+// blockIdx.x a chunk of rows; a workgroup reads its rows of both factors once and holds the whole
+// dout x din product (four wavefronts of 64x64).  Rows are transposed into LDS as BF16, 32 at a
+// time (one K step of the 16x16x32 MFMA), the next 32 being loaded meanwhile.
+constexpr int kWgStride = 40;  // LDS row of 32 BF16: 80 B, 16-byte aligned fragments in 16 bank groups
+
+struct MlpWgradArgs {
+  const float* dz[FNE_MLP_MAX_LAYERS];  // [n][dims[l+1]]
+  const float* h[FNE_MLP_MAX_LAYERS];   // [n][dims[l]]
+  int dims[FNE_MLP_MAX_LAYERS + 1];
+  long woff[FNE_MLP_MAX_LAYERS];  // layer l's weights within a slice of partials
+  long weights;                   // length of a slice
+};
+
+__global__ __launch_bounds__(256) void mlp_narrow_wgrad_kernel(MlpWgradArgs g, long n, long chunk,
+                                                               float* __restrict__ part) {
+  __shared__ unsigned short sD[kNarrow][kWgStride];
+  __shared__ unsigned short sH[kNarrow][kWgStride];
+  const int l = blockIdx.y;
+  const int M = g.dims[l + 1], N = g.dims[l];
+  const float* D = g.dz[l];
+  const float* H = g.h[l];
+  const long r0 = long(blockIdx.x) * chunk, r1 = r0 + chunk < n ? r0 + chunk : n;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+  const int c = tid & 127, rb = (tid >> 7) * 16;  // this thread's column and 16 of the 32 rows
+  mlp_f4 acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = mlp_f4{0.f, 0.f, 0.f, 0.f};
+  float fd[16], fh[16];
+  auto load = [&](long base) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const long r = base + rb + i;
+      fd[i] = (r < r1 && c < M) ? D[size_t(r) * M + c] : 0.f;
+      fh[i] = (r < r1 && c < N) ? H[size_t(r) * N + c] : 0.f;
+    }
+  };
+  load(r0);
+  for (long base = r0; base < r1; base += 32) {
+    mlp_u8 d0, d1, h0, h1;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      d0[i] = cvt_bf(fd[i]);
+      d1[i] = cvt_bf(fd[8 + i]);
+      h0[i] = cvt_bf(fh[i]);
+      h1[i] = cvt_bf(fh[8 + i]);
+    }
+    __syncthreads();  // the previous step's fragments have been read
+    *reinterpret_cast<mlp_u8*>(&sD[c][rb]) = d0;
+    *reinterpret_cast<mlp_u8*>(&sD[c][rb + 8]) = d1;
+    *reinterpret_cast<mlp_u8*>(&sH[c][rb]) = h0;
+    *reinterpret_cast<mlp_u8*>(&sH[c][rb + 8]) = h1;
+    if (base + 32 < r1) load(base + 32);
+    __syncthreads();
+    mlp_b8 a[4], b[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (wm + 16 * i < M) a[i] = *reinterpret_cast<const mlp_b8*>(&sD[wm + 16 * i + (lane & 15)][8 * (lane >> 4)]);
+      if (wn + 16 * i < N) b[i] = *reinterpret_cast<const mlp_b8*>(&sH[wn + 16 * i + (lane & 15)][8 * (lane >> 4)]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (wm + 16 * i < M && wn + 16 * j < N)  // uniform over the wavefront
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+  }
+  float* out = part + size_t(blockIdx.x) * g.weights + g.woff[l];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int m = wm + 16 * i + 4 * (lane >> 4) + r, k = wn + 16 * j + (lane & 15);
+        if (m < M && k < N) out[size_t(m) * N + k] = acc[i][j][r];
+      }
+}
+
+// sums of the partial weight gradients over the row chunks (blocks [0, wblocks)) and of the partial
+// column sums over the chain's workgroups (one wavefront per column), both in index order per thread
+struct MlpGrads {
+  float* dw[FNE_MLP_MAX_LAYERS];
+  float* db[FNE_MLP_MAX_LAYERS];
+};
+
+__global__ __launch_bounds__(256) void mlp_narrow_reduce_kernel(MlpWgradArgs g, int layers, MlpGrads out, int wblocks,
+                                                                const float* __restrict__ part, int splits,
+                                                                const float* __restrict__ cpart, int cblocks,
+                                                                int widths) {
+  if (int(blockIdx.x) < wblocks) {
+    const long i = long(blockIdx.x) * 256 + threadIdx.x;
+    if (i >= g.weights) return;
+    float s = 0.f;
+#pragma unroll 8
+    for (int k = 0; k < splits; ++k) s += part[size_t(k) * g.weights + i];
+    int l = 0;
+    while (l + 1 < layers && i >= g.woff[l + 1]) ++l;
+    out.dw[l][i - g.woff[l]] = s;
+    return;
+  }
+  const int col = (int(blockIdx.x) - wblocks) * 4 + int(threadIdx.x >> 6);
+  if (col >= widths) return;
+  const int lane = threadIdx.x & 63;
+  float s = 0.f;
+  for (int k = lane; k < cblocks; k += 64) s += cpart[size_t(k) * widths + col];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  if (lane == 0) {
+    int l = 0, c = col;
+    while (c >= g.dims[l + 1]) c -= g.dims[++l];
+    out.db[l][c] = s;
+  }
 }
 
 template <typename TA, typename TB>
@@ -200,14 +563,76 @@ long max_width(const fne_mlp_desc* net) {
 
 constexpr int kWgradSplits = 64;
 
+bool narrow(const fne_mlp_desc* net) { return max_width(net) <= kNarrow; }
+
+// widths of all layer outputs, weights of all layers, row chunks of the weight gradients
+struct NarrowSizes {
+  long hidden = 0, widths = 0, weights = 0, blocks = 0, chunk = 0, splits = 0;
+};
+
+NarrowSizes narrow_sizes(const fne_mlp_desc* net, int64_t n) {
+  NarrowSizes z;
+  for (int l = 0; l < net->n_layers; ++l) {
+    z.widths += net->dims[l + 1];
+    z.weights += long(net->dims[l]) * net->dims[l + 1];
+  }
+  z.hidden = z.widths - net->dims[net->n_layers];
+  z.blocks = (n + kNarrowRows - 1) / kNarrowRows;
+  // whole 32-row steps, at most kWgradSplits chunks of at least 128 rows: 64 chunks x 5 layers give
+  // every CU a workgroup (39.9 us with the reduction at 16,384 rows; 128 chunks 41.6: more partial
+  // sums to reduce)
+  z.chunk = ((n + kWgradSplits - 1) / kWgradSplits + 31) / 32 * 32;
+  if (z.chunk < 128) z.chunk = 128;
+  z.splits = (n + z.chunk - 1) / z.chunk;
+  return z;
+}
+
+int narrow_backward(const fne_mlp_desc* net, long n, const float* x, const float* acts, const float* dy,
+                    float* const* dw, float* const* db, void* workspace, hipStream_t s) {
+  const NarrowSizes z = narrow_sizes(net, n);
+  const int L = net->n_layers;
+  float* dz = reinterpret_cast<float*>(workspace);
+  float* part = dz + size_t(n) * z.hidden;
+  float* cpart = part + size_t(z.splits) * z.weights;
+  hipLaunchKernelGGL(mlp_narrow_chain_kernel<kNarrowRows>, dim3(z.blocks), dim3(256), 0, s, *net, n, acts, dy, dz,
+                     cpart, int(z.widths));
+  FNE_LAUNCH_CHECK();
+  MlpWgradArgs g{};
+  MlpGrads out{};
+  size_t off = 0;
+  for (int l = 0; l < L; ++l) {
+    g.dims[l] = net->dims[l];
+    g.h[l] = l == 0 ? x : acts + off - size_t(n) * net->dims[l];
+    g.dz[l] = l == L - 1 ? dy : dz + off;
+    g.woff[l] = g.weights;
+    g.weights += long(net->dims[l]) * net->dims[l + 1];
+    if (l < L - 1) off += size_t(n) * net->dims[l + 1];
+    out.dw[l] = dw[l];
+    out.db[l] = db[l];
+  }
+  g.dims[L] = net->dims[L];
+  hipLaunchKernelGGL(mlp_narrow_wgrad_kernel, dim3(z.splits, L), dim3(256), 0, s, g, n, z.chunk, part);
+  FNE_LAUNCH_CHECK();
+  const int wblocks = int((z.weights + 255) / 256), cb = int((z.widths + 3) / 4);
+  hipLaunchKernelGGL(mlp_narrow_reduce_kernel, dim3(wblocks + cb), dim3(256), 0, s, g, L, out, wblocks, part,
+                     int(z.splits), cpart, int(z.blocks), int(z.widths));
+  FNE_LAUNCH_CHECK();
+  return FNE_OK;
+}
+
 }  // namespace
 
 extern "C" {
 
 int64_t fne_mlp_workspace_bytes(const fne_mlp_desc* net, int64_t n) {
   if (!net_ok(net) || n < 0) return FNE_EINVAL;
+  if (narrow(net)) {
+    // every hidden gradient, the weight gradients' partials, the column sums' partials
+    const NarrowSizes z = narrow_sizes(net, n);
+    return int64_t(sizeof(float)) * (n * z.hidden + z.splits * z.weights + z.blocks * z.widths);
+  }
   const long w = max_width(net);
-  const long chunks = (n + 1023) / 1024;
+  const long chunks = (n + kColsumRows - 1) / kColsumRows;
   // two dZ buffers, weight-gradient split partials, bias-gradient chunk partials
   return int64_t(sizeof(float)) * (2 * n * w + long(kWgradSplits) * w * w + chunks * w);
 }
@@ -219,6 +644,17 @@ int fne_mlp_forward(const fne_mlp_desc* net, int64_t n, const float* x, float* y
     return FNE_EINVAL;
   }
   hipStream_t s = (hipStream_t)stream;
+  if (narrow(net)) {
+    if (net->n_layers > 1 && !acts) {
+      fne_set_error("fne_mlp_forward: activation buffer required");
+      return FNE_EINVAL;
+    }
+    if (n == 0) return FNE_OK;
+    hipLaunchKernelGGL(mlp_narrow_forward_kernel<kNarrowRows>, dim3((n + kNarrowRows - 1) / kNarrowRows), dim3(256), 0,
+                       s, *net, long(n), x, y, acts);
+    FNE_LAUNCH_CHECK();
+    return FNE_OK;
+  }
   const float* in = x;
   size_t off = 0;
   for (int l = 0; l < net->n_layers; ++l) {
@@ -266,12 +702,13 @@ int fne_mlp_backward(const fne_mlp_desc* net, int64_t n, const float* x, const f
     return FNE_EINVAL;
   }
   hipStream_t s = (hipStream_t)stream;
+  if (narrow(net)) return narrow_backward(net, n, x, acts, dy, dw, db, workspace, s);
   const long w = max_width(net);
   float* dz0 = reinterpret_cast<float*>(workspace);
   float* dz1 = dz0 + size_t(n) * w;
   float* part = dz1 + size_t(n) * w;
   float* cpart = part + size_t(kWgradSplits) * w * w;
-  const long chunks = (n + 1023) / 1024;
+  const long chunks = (n + kColsumRows - 1) / kColsumRows;
   // offsets of each hidden activation in acts
   size_t offs[FNE_MLP_MAX_LAYERS + 1];
   offs[0] = 0;
@@ -302,7 +739,7 @@ int fne_mlp_backward(const fne_mlp_desc* net, int64_t n, const float* x, const f
     hipLaunchKernelGGL(mlp_split_reduce_kernel, dim3((nw + 255) / 256), dim3(256), 0, s, part, splits, nw, dw[l]);
     FNE_LAUNCH_CHECK();
     // db[j] = sum_i dz[i][j]
-    hipLaunchKernelGGL(mlp_colsum_kernel, dim3(chunks, (dout + 255) / 256), dim3(256), 0, s, dz, long(n), dout,
+    hipLaunchKernelGGL(mlp_colsum_kernel, dim3(chunks, (dout + 63) / 64), dim3(256), 0, s, dz, long(n), dout,
                        cpart);
     FNE_LAUNCH_CHECK();
     hipLaunchKernelGGL(mlp_split_reduce_kernel, dim3((dout + 255) / 256), dim3(256), 0, s, cpart, int(chunks),

@@ -65,3 +65,36 @@ def test_training_reduces_loss(require_gpu):
     net = NodeMLP(DIMS, seed=11)
     losses = net.train_mse(torch.as_tensor(x), torch.as_tensor(t), epochs=40, batch=4096, lr=2e-3)
     assert losses[-1] < 0.05 * losses[0], losses[::8]
+
+
+@pytest.mark.parametrize("dims,n", [
+    ([10, 128, 128, 128, 128, 3], 1),  # one row of the only workgroup
+    ([7, 64, 96, 2], 31),
+    ([7, 96, 2], 33),  # a row past a workgroup's 32
+    ([5, 33, 17, 4], 129),  # widths off the 4- and 16-column fragments, one row past a chunk's 128
+    ([1, 1, 1], 64),
+    ([13, 6], 257),  # a single layer: no hidden gradient
+    ([128, 128], 40),
+    ([16, 127, 128, 1], 8193),  # more than 64 chunks of 128 rows
+    ([10, 129, 3], 700),  # wider than 128: one launch per product
+    ([10, 160, 144, 3], 1025),
+])
+def test_layer_widths_and_row_counts(require_gpu, dims, n):
+    """Edges of the narrow form (every width <= 128) and of the per-product form, against the oracle
+    with the bound of the tests above (products of BF16 operands)."""
+    net = NodeMLP(dims, seed=n)
+    rng = np.random.default_rng(n + 1)
+    x = rng.standard_normal((n, dims[0])).astype(np.float32)
+    dy = rng.standard_normal((n, dims[-1])).astype(np.float32)
+    for b in net.b32:
+        b.copy_(torch.as_tensor(rng.standard_normal(b.numel()).astype(np.float32) * 0.1))
+    ws = [w.cpu().numpy().astype(np.float64) for w in net.weights_bf16_values()]
+    bs = [b.cpu().numpy().astype(np.float64) for b in net.b32]
+    y = net.forward(torch.as_tensor(x), keep=True).cpu().numpy()
+    dw, db = net.backward(torch.as_tensor(dy))
+    yo, acts = omlp.forward(ws, bs, x)
+    dwo, dbo = omlp.backward(ws, bs, x, acts, dy)
+    assert _rel(y, yo) < 5e-3
+    for l in range(len(ws)):
+        assert _rel(dw[l].cpu().numpy(), dwo[l]) < 5e-3, l
+        assert _rel(db[l].cpu().numpy(), dbo[l]) < 5e-3, l
