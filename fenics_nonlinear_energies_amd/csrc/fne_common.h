@@ -27,6 +27,41 @@ void fne_set_error(const std::string& msg);
 // ---------------------------------------------------------------------------------------------
 // plan object
 // ---------------------------------------------------------------------------------------------
+// Node-patch schedule of the tetrahedral assembly (fne_plan_build_node_patches): a patch is a run of
+// consecutive free nodes and every element that touches one of them.  Device arrays, owned by the
+// plan (one allocation).  Items name an element by its slot in the patch.
+struct FneNodePatches {
+  int n_patch = 0;
+  const int32_t* pnode = nullptr;      // [n_patch + 1] first node
+  const int32_t* pelem_ptr = nullptr;  // [n_patch + 1] offsets into pelem / pelem_node
+  const int32_t* pelem = nullptr;      // element ids, the patch's own first
+  const int4* pelem_node = nullptr;    // their four nodes: free node, or n_nodes + total node
+  const int32_t* pown = nullptr;       // [n_patch] own elements (their energy is summed here)
+  const int32_t* pair_ptr = nullptr;   // [n_patch + 1] offsets into pair / pair_items
+  // off-diagonal 3x3 blocks (i, j) of the CSR rows, those with both nodes in the patch once for
+  // (i, j) and (j, i), in row order.  x: local node i [0:6) | position of j in its row [6:14) |
+  // items in pair_items [14:18) | further item blocks [18:22) at extra_ptr[p] + [22:32);
+  // y: local node j [0:6) | position of i in its row [6:14), or kNodePatchNone
+  const uint2* pair = nullptr;
+  const uint4* pair_items = nullptr;   // 8 x (slot [0:9) | a [9:11) | b [11:13) | index of (a,b) [13:16))
+  const int32_t* extra_ptr = nullptr;  // [n_patch] offsets into extra
+  const uint4* extra = nullptr;        // blocks of 8 items
+  const uint2* diag_items = nullptr;   // [n_nodes][8] blocks of 4 x (slot [0:9) | a [9:11))
+  // [n_nodes] block position of the diagonal [0:8) | further blocks of 8 items [8:16) at extra_ptr[p] + [16:32)
+  const uint32_t* diag = nullptr;
+  void* storage = nullptr;
+};
+// threads per workgroup; elements (at most one per thread) and nodes per patch.  240 element states
+// are 50 KB of LDS, so three workgroups share a CU: the fused FP32 assembly of the 320x16x16 beam
+// takes 69.8 us; 256 elements (two workgroups) 81.6, 192 of 192 threads 78.9, 128 of 128 81.0 (more
+// elements evaluated twice)
+constexpr int kNodePatchThreads = 256;
+constexpr int kNodePatchElems = 240;
+constexpr int kNodePatchNodes = 32;
+constexpr uint32_t kNodePatchNone = 0xFFFFFFFFu;
+// unused items name a slot of zeros behind the elements
+constexpr uint16_t kNodePatchZero = kNodePatchElems;
+
 struct fne_plan {
   fne_plan_desc d;
   double2* partials = nullptr;  // per-block (sum, compensation) pairs for energy reductions
@@ -38,6 +73,7 @@ struct fne_plan {
   // [n_elem][n_loc][n_loc] (FP64 or FP32), written by the element kernel, read by the row gather
   double* mc_g = nullptr;
   void* mc_h = nullptr;
+  FneNodePatches np;  // tetrahedra: n_patch = 0 until fne_plan_build_node_patches
 };
 
 constexpr int kEnergyBlocks = 2048;  // fixed grid => fixed reduction order => deterministic

@@ -310,6 +310,7 @@ int fne_plan_destroy(fne_plan* plan) {
   if (plan->partials) (void)hipFree(plan->partials);
   if (plan->mc_h) (void)hipFree(plan->mc_h);
   if (plan->mc_g) (void)hipFree(plan->mc_g);
+  if (plan->np.storage) (void)hipFree(plan->np.storage);
   delete plan;
   return FNE_OK;
 }

@@ -81,6 +81,7 @@ class FnePlanDesc(C.Structure):
 _SIGNATURES = [
     ("fne_plan_create", C.c_int, [C.POINTER(FnePlanDesc), C.POINTER(C.c_void_p)]),
     ("fne_plan_destroy", C.c_int, [C.c_void_p]),
+    ("fne_plan_build_node_patches", C.c_int, [C.c_void_p, _i32p, _i32p, _i32p]),
     ("fne_plan_set_params", C.c_int, [C.c_void_p, _f64p]),
     ("fne_plan_set_mode", C.c_int, [C.c_void_p, C.c_int32]),
     ("fne_energy", C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]),

@@ -15,6 +15,7 @@ from __future__ import annotations
 import numpy as np
 import scipy.sparse as sp
 
+from .. import native
 from ..assembler import ReorderedElementAssemblerBase
 from ..native import FNE_FLAG_ABS_DET, FNE_FLAG_ROW_GATHER, FNE_KIND_NEOHOOKEAN
 from ..patches import build_block_plan, build_row_incidence_plan
@@ -185,6 +186,22 @@ class HEReorderedElementAssembler(ReorderedElementAssemblerBase):
         B[0::3, 4], B[2::3, 4] = X[:, 2], -X[:, 0]
         B[0::3, 5], B[1::3, 5] = -X[:, 1], X[:, 0]
         return B
+
+    # row-gather plans get the node-patch schedule where the mesh allows it
+    node_patches = True
+
+    def _upload_plan(self) -> None:
+        super()._upload_plan()
+        if self.assembly_mode != "rowgather" or not self.node_patches:
+            return
+        import ctypes
+
+        i32 = ctypes.POINTER(ctypes.c_int32)
+        host = [np.ascontiguousarray(a, dtype=np.int32)
+                for a in (self._host_codes.T, self.layout.indptr, self.layout.indices)]
+        rc = native.lib().fne_plan_build_node_patches(self._plan, *(a.ctypes.data_as(i32) for a in host))
+        if rc != native.FNE_EUNSUPPORTED:
+            native.check(rc, "fne_plan_build_node_patches")
 
     def _element_geometry(self) -> np.ndarray:
         p = self.params

@@ -122,6 +122,19 @@ typedef struct fne_plan fne_plan;
  * (core/petsc/reordered_element_base.py:803-819). */
 int fne_plan_create(const fne_plan_desc* desc, fne_plan** out);
 int fne_plan_destroy(fne_plan* plan);
+/*
+ * Tetrahedral plans with FNE_FLAG_ROW_GATHER: add the node-patch schedule, with which gradient,
+ * Hessian and fused assembly run in one launch without element matrices in memory (fne_hvp keeps
+ * the row gather).  HOST pointers, the same values as the descriptor's device arrays: edof
+ * [12][n_elem], indptr, indices; read during the call only.  Needs nodes whose three components are
+ * free together or constrained together, consecutive and aligned, and CSR rows made of 3x3 node
+ * blocks with a symmetric pattern; otherwise FNE_EUNSUPPORTED, and the plan goes on with the row
+ * gather.  Allocates the schedule once (freed by fne_plan_destroy) and gives the plan's element
+ * matrices back.  Not while work on the plan is in flight.
+ * Stands in for the scatter build (core/petsc/reordered_element_base.py:1464-1534).
+ */
+int fne_plan_build_node_patches(fne_plan* plan, const int32_t* edof, const int32_t* indptr,
+                                const int32_t* indices);
 /* Replaces update of model parameters between continuation steps (e.g. Davis-B reduced
  * cohesion/friction, slope_stability/jax_petsc/solver.py:600-603). */
 int fne_plan_set_params(fne_plan* plan, const double* param8);

@@ -7,6 +7,7 @@ import torch
 from fenics_nonlinear_energies_amd.problems.hyperelasticity import (
     HEReorderedElementAssembler,
     build_beam_problem,
+    problem_from_mesh,
     rotate_right_face_from_reference,
 )
 from oracle import assembly
@@ -81,3 +82,79 @@ def test_he_nonpositive_jacobian_gives_nan_energy(require_gpu):
     u[0::3] *= -1.0  # mirror x: inverts every free-node element orientation
     E = asm.energy_fn(asm.create_vec(u[asm.layout.perm]))
     assert not np.isfinite(E)
+
+
+class _RowGather(HEReorderedElementAssembler):
+    node_patches = False
+
+
+def _node_permutation(p, seed):
+    """Free nodes in random order, components together: patches whose nodes share few elements."""
+    n = p["freedofs"].size // 3
+    return (3 * np.random.default_rng(seed).permutation(n)[:, None] + np.arange(3)).ravel()
+
+
+def _fan(n):
+    """Three axis edges joined to a ring of n vertices: edges with n tetrahedra (more than one
+    block of items), axis nodes with 2 n."""
+    t = 2 * np.pi * np.arange(n) / n
+    axis = np.stack((np.zeros(4), np.zeros(4), np.arange(4.0)), 1)
+    nodes = np.concatenate((axis, np.stack((np.cos(t), np.sin(t), 1.5 + 0 * t), 1)))
+    k = np.arange(n)
+    tets = [np.stack((0 * k + j, 0 * k + j + 1, 4 + k, 4 + (k + 1) % n), 1) for j in range(3)]
+    return problem_from_mesh(nodes, np.concatenate(tets), 1.0, 2.0)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("dims,order,absdet", [
+    ("fan", "block_morton", False),
+    ((2, 1, 1), "block_morton", False),  # four free nodes, one patch
+    ((6, 1, 1), "none", True),
+    ((16, 3, 3), "random", False),
+    ((30, 5, 4), "block_xyz", False),
+    ((40, 9, 7), "block_morton", True),  # patches cut by their elements and by their nodes
+])
+def test_node_patches_match_row_gather(require_gpu, dims, order, absdet, precision):
+    """The node-patch schedule against the row gather on the same plan arrays.  Both evaluate the same
+    FP64 element formulas: a CSR value sums at most ~30 element values, so 1e-12 of the largest entry
+    (2e-6 where the row gather sums in FP32); the energy 1e-12; the gradient's terms cancel, 1e-10 of
+    its largest entry as against the oracle."""
+    p, adj, u0 = _fan(30) if dims == "fan" else build_beam_problem(*dims)
+    kw = dict(use_abs_det=absdet, hessian_precision=precision)
+    kw.update({"perm_override": _node_permutation(p, 3)} if order == "random" else {"reorder_mode": order})
+    u = _state(p, u0, 5, amp=0.05 if dims == "fan" else 2e-3 / max(dims[1:]))
+    out = []
+    for cls in (HEReorderedElementAssembler, _RowGather):
+        asm = cls(p, None, adj, **kw)
+        x = asm.create_vec(u[asm.layout.perm])
+        asm._f_dev = torch.as_tensor(np.random.default_rng(7).standard_normal(u.size)).cuda()  # a load
+        g, g2 = x.duplicate(), x.duplicate()
+        asm.A.data.fill_(float("nan"))  # every entry is written
+        e = float(asm.energy_grad_hessian_device(x.t, g.t).item())
+        h = asm.A.data.clone()
+        asm.gradient_fn(x, g2)
+        assert torch.equal(g.t, g2.t)
+        asm.A.data.fill_(float("nan"))
+        asm.assemble_hessian(x)
+        assert torch.equal(asm.A.data, h)
+        out.append((e, g.t.cpu().numpy(), h.double().cpu().numpy()))
+        asm.cleanup()
+    (e, g, h), (e0, g0, h0) = out
+    # an inverted element's energy is NaN (ln J) in either form
+    assert abs(e - e0) <= 1e-12 * abs(e0) if np.isfinite(e0) else np.isnan(e) == np.isnan(e0)
+    assert np.abs(g - g0).max() <= 1e-10 * np.abs(g0).max()
+    assert np.abs(h - h0).max() <= (1e-12 if precision == "fp64" else 2e-6) * np.abs(h0).max()
+
+
+def test_node_patches_leave_mixed_orders_to_the_row_gather(require_gpu):
+    """Components of one node apart: no 3x3 blocks in the CSR rows, the plan keeps the row gather."""
+    p, adj, u0 = build_beam_problem(8, 2, 2)
+    perm = np.random.default_rng(2).permutation(u0.size)
+    out = []
+    for cls in (HEReorderedElementAssembler, _RowGather):
+        asm = cls(p, None, adj, perm_override=perm)
+        x = asm.create_vec(_state(p, u0, 4)[perm])
+        asm.assemble_hessian(x)
+        out.append(asm.A.data.clone())
+        asm.cleanup()
+    assert torch.equal(*out)
