@@ -62,6 +62,18 @@ constexpr uint32_t kNodePatchNone = 0xFFFFFFFFu;
 // unused items name a slot of zeros behind the elements
 constexpr uint16_t kNodePatchZero = kNodePatchElems;
 
+// Row units of the Mohr-Coulomb assembly (fne_plan_build_row_units): a CSR row, or the x and y rows of
+// a node with the same columns and elements.  x: first CSR entry, y: first item, z: row, w: row length
+// [0:8) | two rows [8] | items [9:31).  The items of all
+// units have incidences and positions of their own, once per unit: half of the plan's.
+struct FneRowUnits {
+  int n_unit = 0;
+  const int4* unit = nullptr;           // device arrays, one allocation owned by the plan
+  const uint32_t* inc = nullptr;        // [items] element * 32 + local row
+  const unsigned char* pos = nullptr;   // [items][16 for P2, 32 for P4] positions as in pitem
+  void* storage = nullptr;
+};
+
 struct fne_plan {
   fne_plan_desc d;
   double2* partials = nullptr;  // per-block (sum, compensation) pairs for energy reductions
@@ -73,6 +85,7 @@ struct fne_plan {
   // [n_elem][n_loc][n_loc] (FP64 or FP32), written by the element kernel, read by the row gather
   double* mc_g = nullptr;
   void* mc_h = nullptr;
+  FneRowUnits units;  // Mohr-Coulomb: n_unit = 0 (every row by itself) until fne_plan_build_row_units
   FneNodePatches np;  // tetrahedra: n_patch = 0 until fne_plan_build_node_patches
 };
 
@@ -360,7 +373,7 @@ int fne_finalize_energy(fne_plan* plan, int nblocks, double* out, hipStream_t st
 // bytes of the element-matrix scratch (and, via gbytes, of the gradient scratch) used by the
 // row-gather assembly (Mohr-Coulomb always, tetrahedra with FNE_FLAG_ROW_GATHER)
 size_t fne_mc_scratch_bytes(const fne_plan_desc& d, size_t* gbytes);
-// CSR rows gather their incident element rows from the scratch (n_loc 12 or 30)
+// CSR rows of tetrahedral plans gather their incident element rows from the scratch
 int fne_launch_row_gather(fne_plan* plan, bool want_g, bool want_h, const FneCall& c);
 // Hessian-vector products of the P1 (staged plans) and tetrahedral (row-gather plans) families
 int fne_hvp_p1(fne_plan* plan, const double* x, const double* dvals, const double* v, double* y, hipStream_t s);

@@ -311,6 +311,7 @@ int fne_plan_destroy(fne_plan* plan) {
   if (plan->mc_h) (void)hipFree(plan->mc_h);
   if (plan->mc_g) (void)hipFree(plan->mc_g);
   if (plan->np.storage) (void)hipFree(plan->np.storage);
+  if (plan->units.storage) (void)hipFree(plan->units.storage);
   delete plan;
   return FNE_OK;
 }

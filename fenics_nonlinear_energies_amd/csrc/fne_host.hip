@@ -105,6 +105,40 @@ extern "C" int fne_color_distance2(int32_t n, const int32_t* indptr, const int32
 // ---------------------------------------------------------------------------------------------
 namespace {
 
+// host arrays to be placed in one device allocation, each at a multiple of 256 bytes
+struct HostParts {
+  struct Part {
+    const void* src;
+    size_t n, at;
+  };
+  std::vector<Part> parts;
+  size_t bytes = 0;
+
+  template <typename T>
+  size_t add(const std::vector<T>& v) {
+    const size_t n = v.size() * sizeof(T), at = bytes;
+    parts.push_back(Part{v.data(), n, at});
+    bytes += (n + 255) / 256 * 256;
+    return at;
+  }
+
+  int upload(char** out, const char* name) const {
+    char* base = nullptr;
+    if (hipMalloc(&base, std::max<size_t>(bytes, 256)) != hipSuccess) {
+      fne_set_error(std::string(name) + ": hipMalloc of the schedule failed");
+      return FNE_ENOMEM;
+    }
+    for (const Part& p : parts)
+      if (p.n && hipMemcpy(base + p.at, p.src, p.n, hipMemcpyHostToDevice) != hipSuccess) {
+        (void)hipFree(base);
+        fne_set_error(std::string(name) + ": upload of the schedule failed");
+        return FNE_EHIP;
+      }
+    *out = base;
+    return FNE_OK;
+  }
+};
+
 struct NodePatchHost {
   std::vector<int32_t> pnode, pelem_ptr, pelem, pelem_node, pown, pair_ptr, extra_ptr;
   std::vector<uint32_t> pair, diag;  // pair: two words per unit
@@ -286,67 +320,22 @@ int build_node_patches(const fne_plan_desc& d, const int32_t* edof, const int32_
   return FNE_OK;
 }
 
-}  // namespace
-
-extern "C" int fne_plan_build_node_patches(fne_plan* plan, const int32_t* edof, const int32_t* indptr,
-                                           const int32_t* indices) {
-  if (!plan || !edof || !indptr || !indices) {
-    fne_set_error("fne_plan_build_node_patches: null pointer");
-    return FNE_EINVAL;
-  }
-  const fne_plan_desc& d = plan->d;
-  if (d.kind != FNE_KIND_NEOHOOKEAN || !(d.flags & FNE_FLAG_ROW_GATHER) || plan->np.storage)
-    return node_patch_unsupported("needs a tetrahedral row-gather plan without node patches");
-  if (d.n_elem <= 0 || d.n_free <= 0) return node_patch_unsupported("empty mesh");
-  NodePatchHost h;
-  try {
-    const int rc = build_node_patches(d, edof, indptr, indices, h);
-    if (rc != FNE_OK) return rc;
-  } catch (const std::bad_alloc&) {
-    fne_set_error("fne_plan_build_node_patches: out of host memory");
-    return FNE_ENOMEM;
-  }
+int upload_node_patches(fne_plan* plan, const NodePatchHost& h) {
   FneNodePatches np;
   np.n_patch = int(h.pnode.size()) - 1;
-  size_t bytes = 0;
-  auto place = [&](size_t n) {
-    const size_t at = bytes;
-    bytes += (n + 255) / 256 * 256;
-    return at;
-  };
-  struct Part {
-    const void* src;
-    size_t n, at;
-  };
-  Part parts[12];
-  int np_parts = 0;
-  auto add = [&](const auto& v) {
-    const size_t n = v.size() * sizeof(v[0]);
-    parts[np_parts] = Part{v.data(), n, place(n)};
-    return parts[np_parts++].at;
-  };
-  const size_t o_pnode = add(h.pnode), o_pep = add(h.pelem_ptr), o_pe = add(h.pelem), o_pn = add(h.pelem_node),
-               o_po = add(h.pown), o_pp = add(h.pair_ptr), o_pr = add(h.pair), o_pi = add(h.pair_items),
-               o_xp = add(h.extra_ptr), o_x = add(h.extra), o_di = add(h.diag_items), o_dg = add(h.diag);
+  HostParts parts;
+  const size_t o_pnode = parts.add(h.pnode), o_pep = parts.add(h.pelem_ptr), o_pe = parts.add(h.pelem),
+               o_pn = parts.add(h.pelem_node), o_po = parts.add(h.pown), o_pp = parts.add(h.pair_ptr),
+               o_pr = parts.add(h.pair), o_pi = parts.add(h.pair_items), o_xp = parts.add(h.extra_ptr),
+               o_x = parts.add(h.extra), o_di = parts.add(h.diag_items), o_dg = parts.add(h.diag);
   char* base = nullptr;
-  if (hipMalloc(&base, bytes) != hipSuccess) {
-    fne_set_error("hipMalloc of the node patches failed");
-    return FNE_ENOMEM;
-  }
+  const int up = parts.upload(&base, "fne_plan_build_node_patches");
+  if (up != FNE_OK) return up;
   double2* partials = nullptr;
   if (np.n_patch > plan->n_partials && hipMalloc(&partials, sizeof(double2) * np.n_patch) != hipSuccess) {
     (void)hipFree(base);
     fne_set_error("hipMalloc of reduction scratch failed");
     return FNE_ENOMEM;
-  }
-  for (int i = 0; i < np_parts; ++i) {
-    if (parts[i].n == 0) continue;
-    if (hipMemcpy(base + parts[i].at, parts[i].src, parts[i].n, hipMemcpyHostToDevice) != hipSuccess) {
-      (void)hipFree(base);
-      if (partials) (void)hipFree(partials);
-      fne_set_error("upload of the node patches failed");
-      return FNE_EHIP;
-    }
   }
   if (partials) {
     (void)hipFree(plan->partials);
@@ -370,5 +359,112 @@ extern "C" int fne_plan_build_node_patches(fne_plan* plan, const int32_t* edof, 
   np.diag_items = reinterpret_cast<uint2*>(base + o_di);
   np.diag = reinterpret_cast<uint32_t*>(base + o_dg);
   plan->np = np;
+  return FNE_OK;
+}
+
+}  // namespace
+
+extern "C" int fne_plan_build_node_patches(fne_plan* plan, const int32_t* edof, const int32_t* indptr,
+                                           const int32_t* indices) {
+  if (!plan || !edof || !indptr || !indices) {
+    fne_set_error("fne_plan_build_node_patches: null pointer");
+    return FNE_EINVAL;
+  }
+  const fne_plan_desc& d = plan->d;
+  if (d.kind != FNE_KIND_NEOHOOKEAN || !(d.flags & FNE_FLAG_ROW_GATHER) || plan->np.storage)
+    return node_patch_unsupported("needs a tetrahedral row-gather plan without node patches");
+  if (d.n_elem <= 0 || d.n_free <= 0) return node_patch_unsupported("empty mesh");
+  NodePatchHost h;
+  try {
+    const int rc = build_node_patches(d, edof, indptr, indices, h);
+    if (rc != FNE_OK) return rc;
+    return upload_node_patches(plan, h);
+  } catch (const std::bad_alloc&) {
+    fne_set_error("fne_plan_build_node_patches: out of host memory");
+    return FNE_ENOMEM;
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
+// Row units of the Mohr-Coulomb assembly (FneRowUnits), from the plan's row incidences.
+// ---------------------------------------------------------------------------------------------
+constexpr size_t kUnitWindow = 256;
+
+extern "C" int fne_plan_build_row_units(fne_plan* plan, const int32_t* inc_ptr, const uint32_t* inc,
+                                        const unsigned char* pos, const int32_t* indptr,
+                                        const int32_t* indices) {
+  if (!plan || !inc_ptr || !inc || !pos || !indptr || !indices) {
+    fne_set_error("fne_plan_build_row_units: null pointer");
+    return FNE_EINVAL;
+  }
+  const fne_plan_desc& d = plan->d;
+  auto unsupported = [](const char* why) {
+    fne_set_error(std::string("fne_plan_build_row_units: ") + why);
+    return FNE_EUNSUPPORTED;
+  };
+  if (d.kind != FNE_KIND_MOHR_COULOMB || plan->units.unit || d.n_elem <= 0 || d.n_free <= 0 || !d.inc_ptr || !d.inc || !d.pitem)
+    return unsupported("needs a Mohr-Coulomb plan with row incidences and without units");
+  const int32_t nf = d.n_free;
+  auto items_of = [&](int32_t r) { return inc_ptr[r + 1] - inc_ptr[r]; };
+  auto len_of = [&](int32_t r) { return indptr[r + 1] - indptr[r]; };
+  for (int32_t r = 0; r < nf; ++r) {
+    if (items_of(r) < 0 || items_of(r) >= (1 << 22) || len_of(r) < 0 || len_of(r) > 254)
+      return unsupported("row or incidence list too long");
+    for (int32_t k = inc_ptr[r]; k < inc_ptr[r + 1]; ++k)
+      if (int32_t(inc[k] >> 5) >= d.n_elem || int32_t(inc[k] & 31u) >= d.n_loc)
+        return unsupported("incidence item out of range");
+  }
+  // rows r, r + 1 are the x and y rows of a node with the same columns and elements
+  auto paired = [&](int32_t r) {
+    if (r + 1 >= nf || items_of(r) != items_of(r + 1) || items_of(r) == 0 || len_of(r) != len_of(r + 1)) return false;
+    for (int32_t k = 0; k < items_of(r); ++k) {
+      const uint32_t a = inc[inc_ptr[r] + k];
+      if ((a & 1u) || inc[inc_ptr[r + 1] + k] != a + 1u) return false;
+    }
+    const unsigned char *p = pos + size_t(inc_ptr[r]) * 32, *p1 = pos + size_t(inc_ptr[r + 1]) * 32;
+    if (!std::equal(p, p1, p1)) return false;
+    return std::equal(indices + indptr[r], indices + indptr[r + 1], indices + indptr[r + 1]);
+  };
+  try {
+    std::vector<int4> unit;
+    unit.reserve(size_t(nf) / 2 + 1);
+    for (int32_t r = 0; r < nf;) {
+      const bool two = paired(r);
+      unit.push_back(make_int4(indptr[r], inc_ptr[r], r, len_of(r) | (int(two) << 8) | (items_of(r) << 9)));
+      r += two ? 2 : 1;
+    }
+    // units with the same number of elements side by side: the lane groups of a wavefront then take
+    // the same branches; in windows, so that neighbouring rows keep sharing element matrices
+    for (size_t i = 0; i < unit.size(); i += kUnitWindow)
+      std::stable_sort(unit.begin() + i, unit.begin() + std::min(unit.size(), i + kUnitWindow),
+                       [](const int4& a, const int4& b) { return (a.w >> 9) < (b.w >> 9); });
+    const size_t width = d.n_loc == 30 ? 32 : 16;
+    size_t items = 0;
+    for (const int4& w : unit) items += size_t(w.w >> 9);
+    std::vector<uint32_t> uinc(items);
+    std::vector<unsigned char> upos(items * width);
+    items = 0;
+    for (int4& w : unit) {
+      const int from = w.y, n = w.w >> 9;
+      w.y = int(items);
+      for (int k = 0; k < n; ++k, ++items) {
+        uinc[items] = inc[from + k];
+        std::copy_n(pos + size_t(from + k) * 32, width, &upos[items * width]);
+      }
+    }
+    HostParts parts;
+    const size_t o_u = parts.add(unit), o_i = parts.add(uinc), o_p = parts.add(upos);
+    char* base = nullptr;
+    const int up = parts.upload(&base, "fne_plan_build_row_units");
+    if (up != FNE_OK) return up;
+    plan->units.storage = base;
+    plan->units.unit = reinterpret_cast<int4*>(base + o_u);
+    plan->units.inc = reinterpret_cast<uint32_t*>(base + o_i);
+    plan->units.pos = reinterpret_cast<unsigned char*>(base + o_p);
+    plan->units.n_unit = int(unit.size());
+  } catch (const std::bad_alloc&) {
+    fne_set_error("fne_plan_build_row_units: out of host memory");
+    return FNE_ENOMEM;
+  }
   return FNE_OK;
 }

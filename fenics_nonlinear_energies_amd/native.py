@@ -34,6 +34,7 @@ FNE_PCG_NOALLOC_MAX_BYTES = 16 << 20
 
 _i32p = C.POINTER(C.c_int32)
 _u32p = C.POINTER(C.c_uint32)
+_u8p = C.POINTER(C.c_uint8)
 _f64p = C.POINTER(C.c_double)
 
 
@@ -82,6 +83,7 @@ _SIGNATURES = [
     ("fne_plan_create", C.c_int, [C.POINTER(FnePlanDesc), C.POINTER(C.c_void_p)]),
     ("fne_plan_destroy", C.c_int, [C.c_void_p]),
     ("fne_plan_build_node_patches", C.c_int, [C.c_void_p, _i32p, _i32p, _i32p]),
+    ("fne_plan_build_row_units", C.c_int, [C.c_void_p, _i32p, _u32p, _u8p, _i32p, _i32p]),
     ("fne_plan_set_params", C.c_int, [C.c_void_p, _f64p]),
     ("fne_plan_set_mode", C.c_int, [C.c_void_p, C.c_int32]),
     ("fne_energy", C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]),

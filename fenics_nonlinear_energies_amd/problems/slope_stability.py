@@ -332,6 +332,27 @@ class SlopeStabilityReorderedElementAssembler(ReorderedElementAssemblerBase):
         lay = self.layout
         return build_row_incidence_plan(elem_free, lay.indptr, lay.indices, lay.n_free)
 
+    # plans list the rows of a node together where the ordering allows it
+    row_units = True
+
+    def _upload_plan(self) -> None:
+        super()._upload_plan()
+        if not self.row_units:
+            return
+        import ctypes
+
+        from .. import native
+
+        plan, lay = self.patch_plan, self.layout
+        ptr = {np.int32: ctypes.c_int32, np.uint32: ctypes.c_uint32, np.uint8: ctypes.c_uint8}
+        host = [np.ascontiguousarray(a, dtype=t) for a, t in (
+            (plan.inc_ptr, np.int32), (plan.inc, np.uint32), (plan.pitem, np.uint8), (lay.indptr, np.int32),
+            (lay.indices, np.int32))]
+        rc = native.lib().fne_plan_build_row_units(
+            self._plan, *(a.ctypes.data_as(ctypes.POINTER(ptr[a.dtype.type])) for a in host))
+        if rc != native.FNE_EUNSUPPORTED:
+            native.check(rc, "fne_plan_build_row_units")
+
     def _build_rhs_owned(self) -> np.ndarray:
         f = np.asarray(self.params["force"], dtype=np.float64)
         return np.asarray(f[np.asarray(self.params["freedofs"], dtype=np.int64)][self.layout.perm], dtype=np.float64)

@@ -98,3 +98,43 @@ def test_elastic_mode_matches_elastic_stiffness(require_gpu):
     Eref = assembly.assemble("mc", p, u, want=("e",))["e"]
     assert abs(Ee - Eref) <= 1e-12 * abs(Eref)
     asm.cleanup()
+
+
+class _SingleRows(SlopeStabilityReorderedElementAssembler):
+    row_units = False
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("degree,h,order", [
+    (4, 10.0, "block_morton"),  # fewer elements than a block's wavefronts take
+    (4, 4.0, "block_morton"),
+    (4, 2.2, "block_xyz"),  # rows of a node together
+    (4, 3.0, "random"),  # components of a node apart: single-row units
+    (2, 1.1, "block_morton"),
+    (2, 1.6, "random"),
+])
+def test_row_units_match_single_rows(require_gpu, degree, h, order, precision):
+    """Node rows assembled together against every row by itself on the same plan arrays, with a load and
+    the tolerances of the tests above (an FP32 entry: both forms within 3e-5 of the largest)."""
+    p, adj = mc_params(h=h, degree=degree, lam=1.5)
+    n = p["freedofs"].size
+    kw = {"perm_override": np.random.default_rng(4).permutation(n)} if order == "random" else {"reorder_mode": order}
+    out = []
+    for cls in (SlopeStabilityReorderedElementAssembler, _SingleRows):
+        asm = cls(p, None, adj, hessian_precision=precision, **kw)
+        x = asm.create_vec(_state(p, asm.layout, 5)[asm.layout.perm])
+        g, g2 = x.duplicate(), x.duplicate()
+        asm.A.data.fill_(float("nan"))  # every entry is written
+        e = float(asm.energy_grad_hessian_device(x.t, g.t).item())
+        v = asm.A.data.clone()
+        asm.gradient_device(x.t, g2.t)
+        assert float(asm.energy_device(x.t).item()) == e and torch.equal(g.t, g2.t)
+        asm.A.data.fill_(float("nan"))
+        asm.hessian_device(x.t)
+        assert torch.equal(asm.A.data, v)
+        out.append((e, g.t.cpu().numpy(), v.double().cpu().numpy()))
+        asm.cleanup()
+    (e, g, v), (e0, g0, v0) = out
+    assert abs(e - e0) <= 1e-12 * abs(e0)
+    assert np.abs(g - g0).max() <= 1e-11 * np.abs(g0).max()
+    assert np.abs(v - v0).max() <= (1e-10 if precision == "fp64" else 3e-5) * np.abs(v0).max()
