@@ -114,10 +114,20 @@ class _DevMat:
         )
 
 
+def _spgemm_lanes(avg_b_row: float) -> int:
+    """Lanes per result row: the smallest group (8 to 64) that takes 1.5 times B's average row at
+    once, so that few rows need a second, unpipelined pass; more lanes only idle."""
+    for lanes in (8, 16, 32):
+        if 1.5 * avg_b_row <= lanes:
+            return lanes
+    return 64
+
+
 def _spgemm(a_indptr, a_indices, a_data, b: _DevMat, b_data: torch.Tensor, c: _DevMat, c_data: torch.Tensor):
     """c_data <- (A B) on C's pattern (fne_spgemm_numeric); A given by its CSR arrays."""
     n_rows = int(a_indptr.numel() - 1)
     prec = native.FNE_FP32 if a_data.dtype == torch.float32 else native.FNE_FP64
+    prec |= _spgemm_lanes(b.nnz / max(1, b.n_rows)) << 8
     native.check(
         native.lib().fne_spgemm_numeric(n_rows, native.ptr(a_indptr), native.ptr(a_indices), native.ptr(a_data), prec,
                                         native.ptr(b.indptr), native.ptr(b.indices), native.ptr(b_data),

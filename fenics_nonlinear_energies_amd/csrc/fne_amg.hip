@@ -8,95 +8,124 @@
 //
 // C = A B restricted to C's pattern, which must hold every column a product of the row
 // reaches (columns outside it are dropped; pattern entries no product reaches become 0).
-// One 64-lane workgroup per row.  The row's result columns are staged in LDS in chunks of
-// kChunk, and A's row with the bounds of the B rows it selects in chunks of kStage; for each
-// nonzero a_ip of A's row, in order, the lanes take the entries of B's row p (distinct columns,
-// so distinct accumulator slots), binary-search their slot in the staged columns and add
-// a_ip * b_pj, while the first entries of the next B row are already on their way.  A barrier
-// closes every p, so each result entry is the sum of its products in the order of A's row: the
-// product is deterministic.
+// G lanes per row, 256 / G rows per workgroup.  The row's result columns are staged in LDS, 8 G at a
+// time.  Lane l holds entry l of A's row and the bounds of the B row it selects; the first G entries
+// of eight B rows are loaded and their slots in the staged columns searched together, then for each
+// nonzero a_ip of A's row, in order, the lanes add a_ip * b_pj of B's row p (distinct columns, so
+// distinct slots) with LDS additions that return nothing.  LDS operations of a wavefront stay in
+// order, so each result entry is the sum of its products in the order of A's row: the product is
+// deterministic, and the same for every G.  Bound by the latency of that chain; G follows B's rows
+// (caller's choice), because one 64-lane workgroup per row left most lanes idle on the 1 to 16
+// entries of the scalar problems' rows, and binary searches one after the other were
+// most of the chain (383^2 p-Laplace hierarchy, nine products of three levels: 1004 -> 352 us).
 #include "fne_common.h"
 
 namespace {
 
-constexpr int kChunk = 512;   // result columns staged per pass
-constexpr int kStage = 256;   // entries of A's row staged per pass
-constexpr int kLanes = 64;
-
-template <typename TA>
-__global__ __launch_bounds__(kLanes) void spgemm_numeric_kernel(
+template <typename TA, int G>
+__global__ __launch_bounds__(256) void spgemm_numeric_kernel(
     int n_rows, const int32_t* __restrict__ a_ptr, const int32_t* __restrict__ a_idx, const TA* __restrict__ a_val,
     const int32_t* __restrict__ b_ptr, const int32_t* __restrict__ b_idx, const double* __restrict__ b_val,
     const int32_t* __restrict__ c_ptr, const int32_t* __restrict__ c_idx, double* __restrict__ c_val) {
-  __shared__ int32_t s_col[kChunk];
-  __shared__ double s_acc[kChunk];
-  __shared__ double s_a[kStage];    // A's row (values) ...
-  __shared__ int32_t s_b0[kStage];  // ... and the bounds of the B rows its columns select
-  __shared__ int32_t s_b1[kStage];
-  const int row = xcd_remap(blockIdx.x, gridDim.x);
-  if (row >= n_rows) return;  // the whole (single-wave) block leaves together
-  const int lane = threadIdx.x;
+  constexpr int kRows = 256 / G, kChunk = 8 * G;
+  constexpr int W = G == 64 ? 2 : 1, kPf = 8 / W;  // entries of a B row per lane, B rows in flight
+  __shared__ int32_t s_cols[kRows][kChunk];
+  __shared__ double s_accs[kRows][kChunk];
+  const int lane = threadIdx.x & (G - 1), grp = threadIdx.x / G;
+  int32_t* s_col = s_cols[grp];
+  double* s_acc = s_accs[grp];
+  const int row = xcd_remap(blockIdx.x, gridDim.x) * kRows + grp;
+  if (row >= n_rows) return;  // the whole lane group; no block-level barrier below
   const int c0 = c_ptr[row], c1 = c_ptr[row + 1];
   const int a0 = a_ptr[row], a1 = a_ptr[row + 1];
   for (int cs = c0; cs < c1; cs += kChunk) {
     const int len = min(kChunk, c1 - cs);
-    for (int t = lane; t < len; t += kLanes) {
+    for (int t = lane; t < len; t += G) {
       s_col[t] = c_idx[cs + t];
       s_acc[t] = 0.0;
     }
-    __syncthreads();
-    const int first = s_col[0], last = s_col[len - 1];
-    auto add = [&](int j, double prod) {
-      if (j < first || j > last) return;
-      int lo = 0, hi = len - 1;
-      while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (s_col[mid] < j)
-          lo = mid + 1;
-        else
-          hi = mid;
-      }
-      if (s_col[lo] == j) s_acc[lo] += prod;
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    int top = 1;  // largest power of two below len (1 at least)
+    while (2 * top < len) top *= 2;
+    auto add = [&](int j, double prod) {  // the last staged column <= j
+      int at = 0;
+      for (int step = top; step > 0; step >>= 1)
+        if (at + step < len && s_col[at + step] <= j) at += step;
+      if (s_col[at] == j) unsafeAtomicAdd(&s_acc[at], prod);
     };
-    for (int ps = a0; ps < a1; ps += kStage) {
-      const int na = min(kStage, a1 - ps);
-      for (int t = lane; t < na; t += kLanes) {
-        const int l = a_idx[ps + t];
-        s_a[t] = static_cast<double>(a_val[ps + t]);
-        s_b0[t] = b_ptr[l];
-        s_b1[t] = b_ptr[l + 1];
+    for (int ps = a0; ps < a1; ps += G) {
+      const int na = min(G, a1 - ps);
+      double av = 0.0;
+      int b0 = 0, b1 = 0;
+      if (lane < na) {
+        const int l = a_idx[ps + lane];
+        av = static_cast<double>(a_val[ps + lane]);
+        b0 = b_ptr[l];
+        b1 = b_ptr[l + 1];
       }
-      __syncthreads();
-      // the first 64 entries of the next B row are loaded while the current one is added
-      int jn = -1;
-      double bn = 0.0;
-      {
-        const int q = s_b0[0] + lane;
-        if (q < s_b1[0]) {
-          jn = b_idx[q];
-          bn = b_val[q];
-        }
-      }
-      for (int t = 0; t < na; ++t) {
-        const int jc = jn;
-        const double bc = bn;
-        const double a = s_a[t];
-        const int b0 = s_b0[t], b1 = s_b1[t];
-        if (t + 1 < na) {
-          const int q = s_b0[t + 1] + lane;
-          jn = -1;
-          if (q < s_b1[t + 1]) {
-            jn = b_idx[q];
-            bn = b_val[q];
+      for (int t0 = 0; t0 < na; t0 += kPf) {
+        int j[kPf * W], q0[kPf], q1[kPf];
+        double a[kPf], b[kPf * W];
+#pragma unroll
+        for (int i = 0; i < kPf; ++i) {  // beyond na: an empty row
+          const int t = min(t0 + i, G - 1);
+          a[i] = __shfl(av, t, G);
+          q0[i] = __shfl(b0, t, G) + lane;
+          q1[i] = t0 + i < na ? __shfl(b1, t, G) : 0;
+#pragma unroll
+          for (int w = 0; w < W; ++w) {
+            j[i * W + w] = -1;
+            b[i * W + w] = 0.0;
+            if (q0[i] + w * G < q1[i]) {
+              j[i * W + w] = b_idx[q0[i] + w * G];
+              b[i * W + w] = b_val[q0[i] + w * G];
+            }
           }
         }
-        if (jc >= 0) add(jc, a * bc);
-        for (int q = b0 + kLanes + lane; q < b1; q += kLanes) add(b_idx[q], a * b_val[q]);
-        __syncthreads();  // entry t's additions land before entry t+1's (fixed order)
+        int at[kPf * W];
+#pragma unroll
+        for (int i = 0; i < kPf * W; ++i) at[i] = 0;
+        for (int step = top; step > 0; step >>= 1) {
+#pragma unroll
+          for (int i = 0; i < kPf * W; ++i) {
+            const int to = min(at[i] + step, len - 1);
+            if (s_col[to] <= j[i]) at[i] = to;  // (from len - 1 itself: no move)
+          }
+        }
+        bool hit[kPf * W];
+#pragma unroll
+        for (int i = 0; i < kPf * W; ++i) hit[i] = j[i] >= 0 && s_col[at[i]] == j[i];
+#pragma unroll
+        for (int i = 0; i < kPf; ++i) {
+#pragma unroll
+          for (int w = 0; w < W; ++w)
+            if (hit[i * W + w]) unsafeAtomicAdd(&s_acc[at[i * W + w]], a[i] * b[i * W + w]);
+          for (int q = q0[i] + W * G; q < q1[i]; q += G) add(b_idx[q], a[i] * b_val[q]);
+          __builtin_amdgcn_wave_barrier();  // entry t's additions land before entry t+1's (fixed order)
+        }
       }
     }
-    for (int t = lane; t < len; t += kLanes) c_val[cs + t] = s_acc[t];
-    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    for (int t = lane; t < len; t += G) c_val[cs + t] = s_acc[t];
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+template <typename TA>
+void launch_spgemm(int n_rows, const int32_t* a_ptr, const int32_t* a_idx, const TA* a_val, const int32_t* b_ptr,
+                   const int32_t* b_idx, const double* b_val, const int32_t* c_ptr, const int32_t* c_idx,
+                   double* c_val, int lanes, hipStream_t s) {
+  auto go = [&](auto kern) {
+    const int rows = 256 / lanes;
+    hipLaunchKernelGGL(kern, dim3((n_rows + rows - 1) / rows), dim3(256), 0, s, n_rows, a_ptr, a_idx, a_val, b_ptr,
+                       b_idx, b_val, c_ptr, c_idx, c_val);
+  };
+  switch (lanes) {
+    case 8: go(spgemm_numeric_kernel<TA, 8>); break;
+    case 16: go(spgemm_numeric_kernel<TA, 16>); break;
+    case 32: go(spgemm_numeric_kernel<TA, 32>); break;
+    default: go(spgemm_numeric_kernel<TA, 64>);
   }
 }
 
@@ -463,14 +492,20 @@ extern "C" int fne_spgemm_numeric(int32_t n_rows, const int32_t* a_indptr, const
     fne_set_error("fne_spgemm_numeric: null pointer");
     return FNE_EINVAL;
   }
-  const dim3 grid(n_rows), block(kLanes);
+  int lanes = (a_precision >> 8) & 0xff;
+  if (lanes == 0) lanes = 64;
+  if (lanes != 8 && lanes != 16 && lanes != 32 && lanes != 64) {
+    fne_set_error("fne_spgemm_numeric: lanes per row must be 8, 16, 32 or 64");
+    return FNE_EINVAL;
+  }
   hipStream_t s = (hipStream_t)stream;
-  if (a_precision == FNE_FP64)
-    hipLaunchKernelGGL(spgemm_numeric_kernel<double>, grid, block, 0, s, n_rows, a_indptr, a_indices,
-                       (const double*)a_vals, b_indptr, b_indices, b_vals, c_indptr, c_indices, c_vals);
-  else if (a_precision == FNE_FP32)
-    hipLaunchKernelGGL(spgemm_numeric_kernel<float>, grid, block, 0, s, n_rows, a_indptr, a_indices,
-                       (const float*)a_vals, b_indptr, b_indices, b_vals, c_indptr, c_indices, c_vals);
+  const int prec = a_precision & 0xff;
+  if (prec == FNE_FP64 && (a_precision >> 16) == 0)
+    launch_spgemm(n_rows, a_indptr, a_indices, (const double*)a_vals, b_indptr, b_indices, b_vals, c_indptr,
+                  c_indices, c_vals, lanes, s);
+  else if (prec == FNE_FP32 && (a_precision >> 16) == 0)
+    launch_spgemm(n_rows, a_indptr, a_indices, (const float*)a_vals, b_indptr, b_indices, b_vals, c_indptr,
+                  c_indices, c_vals, lanes, s);
   else {
     fne_set_error("fne_spgemm_numeric: precision must be FNE_FP64 or FNE_FP32");
     return FNE_EINVAL;

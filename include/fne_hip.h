@@ -286,6 +286,11 @@ int fne_vcycle_cheb(int32_t n_rows, const int32_t* indptr, const int32_t* indice
                     int32_t precision, const double* x, const double* x_prev, const double* r, const double* w,
                     double c, double* y, fne_stream_t stream);
 
+/*
+ * c = A B on C's pattern (columns outside it are dropped).  a_precision: FNE_FP64 / FNE_FP32 |
+ * lanes_per_row << 8 (8, 16, 32 or 64; 0 = 64): lanes for about 1.5 of B's average rows do best; the
+ * sums are the same for all.
+ */
 int fne_spgemm_numeric(int32_t n_rows, const int32_t* a_indptr, const int32_t* a_indices, const void* a_vals,
                        int32_t a_precision, const int32_t* b_indptr, const int32_t* b_indices,
                        const double* b_vals, const int32_t* c_indptr, const int32_t* c_indices, double* c_vals,

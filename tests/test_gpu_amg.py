@@ -120,6 +120,51 @@ def test_spgemm_numeric_matches_scipy(require_gpu, a_prec):
     assert torch.equal(first, Cd.data)
 
 
+@pytest.mark.parametrize("a_prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("lanes", [0, 8, 16, 32, 64])
+def test_spgemm_lane_groups_match_scipy(require_gpu, lanes, a_prec):
+    """Every lane-group width on rows at its edges: empty rows of A, B and C, rows of A and B one
+    shorter, as long and one longer than the group, result rows longer than its 8 x lanes staged
+    columns; sums in the order of A's row, so all widths agree bitwise."""
+    import scipy.sparse as sp
+    import torch
+
+    from fenics_nonlinear_energies_amd import amg, native
+
+    rng = np.random.default_rng(11)
+
+    def rows_of(lengths, n_cols):
+        cols = [np.sort(rng.choice(n_cols, size=m, replace=False)) for m in lengths]
+        ptr = np.concatenate(([0], np.cumsum(lengths)))
+        return sp.csr_matrix((rng.standard_normal(ptr[-1]), np.concatenate(cols), ptr), shape=(len(lengths), n_cols))
+
+    edges = [m for g in (8, 16, 32, 64) for m in (g - 1, g, g + 1)]
+    A = rows_of([0, 1, 3, 4, 5, *edges, 0, 1], 97)
+    B = rows_of(([0, 1, 2, *edges] * 7)[:97], 1500)
+    if a_prec == "fp32":
+        A.data = A.data.astype(np.float32).astype(np.float64)
+    C_pat = amg._pattern_product(A, B)
+    assert np.diff(C_pat.indptr).max() > 8 * 64
+    dev = torch.device("cuda")
+    i32 = lambda a: torch.as_tensor(a.astype(np.int32)).to(dev)  # noqa: E731
+    a = [i32(A.indptr), i32(A.indices), torch.as_tensor(A.data).to(dev, torch.float32 if a_prec == "fp32" else torch.float64)]
+    b = [i32(B.indptr), i32(B.indices), torch.as_tensor(B.data).to(dev)]
+    c = [i32(C_pat.indptr), i32(C_pat.indices)]
+    prec = native.FNE_FP32 if a_prec == "fp32" else native.FNE_FP64
+    out = []
+    for g in (lanes, 64):
+        val = torch.full((C_pat.nnz,), float("nan"), dtype=torch.float64, device=dev)
+        native.check(native.lib().fne_spgemm_numeric(
+            A.shape[0], *(native.ptr(t) for t in a), prec | g << 8, *(native.ptr(t) for t in b),
+            *(native.ptr(t) for t in c), native.ptr(val), native.stream_ptr()), "fne_spgemm_numeric")
+        out.append(val.cpu().numpy())
+    assert np.array_equal(out[0], out[1])
+    # a sum of at most 65 products in another order
+    bound = 2 * 65 * 2.0**-53 * (abs(A) @ abs(B)).toarray()
+    got = sp.csr_matrix((out[0], C_pat.indices, C_pat.indptr), shape=C_pat.shape).toarray()
+    assert np.all(np.abs(got - (A @ B).toarray()) <= bound)
+
+
 def _host_levels(pc, A0):
     """Operators of every level read back from the device (FP64 masters)."""
     import scipy.sparse as sp
