@@ -137,6 +137,24 @@ def _spgemm(a_indptr, a_indices, a_data, b: _DevMat, b_data: torch.Tensor, c: _D
     )
 
 
+def _lanczos_work_len(n: int, code: int) -> int:
+    """Doubles of ``fne_lanczos_max``'s work array (``fne_lanczos_work_len``)."""
+    return 6 * n + 512 + 128 + 8 + (n * (((code >> 8) & 0xFF) or 8) + 255) // 256
+
+
+def _spgemm_smoothed(a_indptr, a_indices, a_data, b: _DevMat, c: _DevMat, w: torch.Tensor):
+    """C's values <- B - diag(w) A B on C's pattern (fne_spgemm_smoothed); A given by its CSR arrays."""
+    prec = native.FNE_FP32 if a_data.dtype == torch.float32 else native.FNE_FP64
+    prec |= _spgemm_lanes(b.nnz / max(1, b.n_rows)) << 8
+    native.check(
+        native.lib().fne_spgemm_smoothed(int(a_indptr.numel() - 1), native.ptr(a_indptr), native.ptr(a_indices),
+                                         native.ptr(a_data), prec, native.ptr(b.indptr), native.ptr(b.indices),
+                                         native.ptr(b.data), native.ptr(c.indptr), native.ptr(c.indices),
+                                         native.ptr(c.data), native.ptr(w), native.stream_ptr()),
+        "fne_spgemm_smoothed",
+    )
+
+
 def _pattern(M: sp.csr_matrix) -> sp.csr_matrix:
     """Structure of M with all-ones values (sorted columns)."""
     M = sp.csr_matrix(M)
@@ -352,7 +370,6 @@ class SmoothedAggregationPC:
             Ac_pat = _pattern_product(R_pat, AP_pat)
             if Ac_pat.shape != (nc, nc):
                 raise RuntimeError("coarse pattern has the wrong shape")
-            pt_rows = np.repeat(np.arange(nl), np.diff(Pt.indptr))
             diag = _positions(A_pat, np.arange(nl), np.arange(nl))
             levels.append({
                 "n": nl,
@@ -369,11 +386,10 @@ class SmoothedAggregationPC:
                 # transfers of the cycle, in the operator's precision
                 "P": _DevMat(P_pat.indptr, P_pat.indices, nc, device, prec),
                 "R": _DevMat(R_pat.indptr, R_pat.indices, nl, device, prec),
-                "ptpos": torch.as_tensor(_positions(P_pat, pt_rows, Pt.indices)).to(device),
-                "p_rows": torch.as_tensor(np.repeat(np.arange(nl), np.diff(P_pat.indptr))).to(device),
                 "tperm_p": torch.as_tensor(_transpose_perm(P_pat)).to(device),
                 "tperm_ac": torch.as_tensor(_transpose_perm(Ac_pat)).to(device),
                 "diag": torch.as_tensor(diag).to(device),
+                "dinv": torch.zeros(nl, dtype=torch.float64, device=device),
                 "wd": torch.zeros(nl, dtype=torch.float64, device=device),
                 "wcheb": torch.zeros((max(1, self.sweeps), nl), dtype=torch.float64, device=device),
                 "Bc": torch.zeros((nc, k), dtype=torch.float64, device=device),
@@ -390,6 +406,15 @@ class SmoothedAggregationPC:
             L["A"] = _DevMat.sharing_pattern(ip, ix, L["n"], prec)
         nc = A_pat.shape[0]
         self._coarse_pat = A_pat
+        # scratch of a numeric set-up, one stage at a time: the Lanczos vectors, an unsymmetrised
+        # coarse product, the two copies of the coarse matrix during its inversion
+        need = [L["Ac64"].nnz for L in levels]
+        code0 = _spmv_code(native.FNE_FP64, A0.nnz / max(1, n))
+        need += [_lanczos_work_len(L["n"], code0 if i == 0 else levels[i - 1]["Ac64"].code)
+                 for i, L in enumerate(levels)]
+        if self.coarse_factor == "device":
+            need.append((2 * ((nc + 31) // 32 * 32) ** 2))
+        self._work = torch.empty(max(need, default=0), dtype=torch.float64, device=device)
         cols = np.tile(np.arange(nc), nc)
         self.coarse_op = _DevMat(np.arange(0, nc * nc + 1, nc), cols, nc, device, "fp64")
         self._coarse_n = nc
@@ -489,52 +514,72 @@ class SmoothedAggregationPC:
         else:
             Bh = B.detach().cpu().numpy() if isinstance(B, torch.Tensor) else B
             pt_vals = self._tentative_values(Bh)
+        lib, stream = native.lib(), native.stream_ptr()
         a_ptr, a_idx, a_dat = A0.indptr, A0.indices, A0.data
+        a_code = _spmv_code(A0.fne_precision, A0.nnz / max(1, A0.n))
         if self.levels:
             self.levels[0]["A"].data.copy_(A0.data)
+        nl = len(self.levels)
+        # per level {largest eigenvalue of D^-1 A, 1 if its Lanczos coefficients are finite}, and
+        # after them the status of the coarse inverse
+        state = torch.empty(2 * nl + 1, dtype=torch.float64, device=device)
+        cheb = np.asarray(self._cheb_weights(1.0) if self.smoother == "chebyshev" else [], dtype=np.float64)
         for lvl, L in enumerate(self.levels):
-            d = A0.diagonal() if lvl == 0 else a_dat[L["diag"]]
-            d = torch.where(d == 0.0, torch.ones_like(d), d)
-            dinv = 1.0 / d
             # rho(D^-1 A): largest Ritz value of a Lanczos run on D^-1/2 A D^-1/2, times a safety
             # factor, so that the smoother's omega rho stays well below 2
-            lam = self._lanczos_lambda_max(lvl, A0, dinv, L["v0"])
-            omega = 4.0 / (3.0 * self.RHO_SAFETY * lam)
-            L["wd"].copy_(omega * dinv)
-            if self.smoother == "chebyshev":
-                for k, coef in enumerate(self._cheb_weights(lam)):
-                    L["wcheb"][k].copy_(coef * dinv)
+            n_l, lam = L["n"], state[2 * lvl:2 * lvl + 2]
+            native.check(lib.fne_lanczos_max(n_l, native.ptr(a_ptr), native.ptr(a_idx), native.ptr(a_dat), a_code,
+                                             native.ptr(L["diag"]), native.ptr(L["v0"]), self.LANCZOS_STEPS,
+                                             native.ptr(L["dinv"]), native.ptr(self._work), self._work.numel(),
+                                             native.ptr(lam), stream), "fne_lanczos_max")
+            for k0 in range(0, max(1, cheb.size), 8):  # omega = 4 / (3 safety lambda); Chebyshev steps by eights
+                f = np.ascontiguousarray(cheb[k0:k0 + 8])
+                native.check(lib.fne_smoother_weights(n_l, native.ptr(L["dinv"]), native.ptr(lam),
+                                                      4.0 / (3.0 * self.RHO_SAFETY), native.f64_ptr(f), f.size,
+                                                      native.ptr(L["wd"]), native.ptr(L["wcheb"][k0:]), stream),
+                             "fne_smoother_weights")
             Pt, P64 = L["Pt"], L["P64"]
             if L["fixed"]:  # a given transfer, used as it is
                 P64.data.copy_(L["Pfix"])
             else:  # P = P_tent - omega D^-1 (A P_tent)
                 if pt_vals is not None:
                     Pt.data.copy_(torch.as_tensor(pt_vals[lvl]))
-                _spgemm(a_ptr, a_idx, a_dat, Pt, Pt.data, P64, P64.data)
-                P64.data.mul_(-omega * dinv[L["p_rows"]])
-                P64.data.index_add_(0, L["ptpos"], Pt.data)
+                _spgemm_smoothed(a_ptr, a_idx, a_dat, Pt, P64, L["wd"])
             # A P, R = P^T, A_c = R (A P), symmetrised
             AP64, R64, Ac64 = L["AP64"], L["R64"], L["Ac64"]
             _spgemm(a_ptr, a_idx, a_dat, P64, P64.data, AP64, AP64.data)
-            torch.index_select(P64.data, 0, L["tperm_p"], out=R64.data)
-            _spgemm(R64.indptr, R64.indices, R64.data, AP64, AP64.data, Ac64, Ac64.data)
-            Ac64.data.copy_(0.5 * (Ac64.data + Ac64.data[L["tperm_ac"]]))
-            L["P"].data.copy_(P64.data)
-            L["R"].data.copy_(R64.data)
-            if lvl + 1 < len(self.levels):
-                self.levels[lvl + 1]["A"].data.copy_(Ac64.data)
-            a_ptr, a_idx, a_dat = Ac64.indptr, Ac64.indices, Ac64.data
+            native.check(lib.fne_amg_transfers(P64.nnz, native.ptr(P64.data), native.ptr(L["tperm_p"]),
+                                               native.ptr(R64.data), native.ptr(L["P"].data), native.ptr(L["R"].data),
+                                               L["P"].prec, stream), "fne_amg_transfers")
+            _spgemm(R64.indptr, R64.indices, R64.data, AP64, AP64.data, Ac64, self._work)
+            cycle = self.levels[lvl + 1]["A"] if lvl + 1 < nl else None
+            native.check(lib.fne_amg_symmetrise(Ac64.nnz, native.ptr(self._work), native.ptr(L["tperm_ac"]),
+                                                native.ptr(Ac64.data), None if cycle is None else native.ptr(cycle.data),
+                                                native.FNE_FP64 if cycle is None else cycle.prec, stream),
+                         "fne_amg_symmetrise")
+            a_ptr, a_idx, a_dat, a_code = Ac64.indptr, Ac64.indices, Ac64.data, Ac64.code
         # coarsest level: dense FP64 inverse (Cholesky; positive-part pseudo-inverse if the
         # operator is not positive definite), on the host or the device, applied on the device
         nc, cp = self._coarse_n, self._coarse_pat
+        fallback = False
         if getattr(self, "_coarse_flat", None) is not None:
-            Ad = torch.zeros(nc * nc, dtype=torch.float64, device=self.coarse_op.data.device)
-            Ad.index_copy_(0, self._coarse_flat, a_dat.double())
-            Ad = Ad.view(nc, nc)
-            Ainv, fallback = coarse_inverse_device(0.5 * (Ad + Ad.T))
-            self.coarse_op.data.copy_(Ainv.reshape(-1))
+            vals = a_dat.double()
+            native.check(lib.fne_spd_inverse(nc, native.ptr(a_ptr), native.ptr(a_idx), native.ptr(vals),
+                                             native.ptr(self._work), self._work.numel(),
+                                             native.ptr(self.coarse_op.data), native.ptr(state[2 * nl:]), stream),
+                         "fne_spd_inverse")
+            st = state.cpu().numpy()
+            self._check_lanczos(st)
+            fallback = nc > 0 and bool(st[2 * nl] != 0.0)
+            if fallback:
+                Ad = torch.zeros(nc * nc, dtype=torch.float64, device=self.coarse_op.data.device)
+                Ad.index_copy_(0, self._coarse_flat, vals)
+                Ad = Ad.view(nc, nc)
+                Ainv, fallback = coarse_inverse_device(0.5 * (Ad + Ad.T))
+                self.coarse_op.data.copy_(Ainv.reshape(-1))
         else:
             Ad = sp.csr_matrix((a_dat.double().cpu().numpy(), cp.indices, cp.indptr), shape=(nc, nc)).toarray()
+            self._check_lanczos(state.cpu().numpy())
             Ainv, fallback = coarse_inverse(0.5 * (Ad + Ad.T))
             self.coarse_op.data.copy_(torch.as_tensor(np.ascontiguousarray(Ainv).ravel()))
         self.coarse_eig_fallbacks += int(fallback)
@@ -542,6 +587,10 @@ class SmoothedAggregationPC:
         self.setup_time += time.perf_counter() - t_setup
         if self.use_graph and self._graph is None and torch.device(device).type == "cuda":
             self._capture(n, device)
+
+    def _check_lanczos(self, state: np.ndarray) -> None:
+        if not np.all(state[1:2 * len(self.levels):2] == 1.0):
+            raise FloatingPointError("non-finite Lanczos coefficients in the multigrid set-up")
 
     CHEB_BOUNDS = (0.1, 1.1)  # [a, b] = these times the estimate of rho(D^-1 A)
 
@@ -569,8 +618,9 @@ class SmoothedAggregationPC:
 
     def _lanczos_lambda_max(self, lvl: int, A0, dinv: torch.Tensor, v0: torch.Tensor) -> float:
         """Largest eigenvalue of D^-1 A (similar to S = D^-1/2 A D^-1/2) from LANCZOS_STEPS
-        Lanczos steps on S from the fixed start vector v0; the recurrence stays on the device and
-        one transfer brings the tridiagonal coefficients to the host.  A Krylov estimate: a
+        Lanczos steps on S from the fixed start vector v0: the set-up's ``fne_lanczos_max`` in vector
+        operations (kept for checking it, and for operators that are not on the GPU), with one
+        transfer of the tridiagonal coefficients to the host.  A Krylov estimate: a
         few warm-started power iterations, used before, under-estimated rho once plasticity
         changed the spectrum, and the smoother (and so the V-cycle) became indefinite."""
         s = torch.sqrt(torch.abs(dinv))  # |D|^-1/2: finite where an indefinite Hessian has a negative diagonal

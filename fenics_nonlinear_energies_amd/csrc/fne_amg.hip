@@ -22,11 +22,13 @@
 
 namespace {
 
-template <typename TA, int G>
+// SMOOTH: C = B - diag(w) A B, the smoothed prolongator of B = P_tent
+template <typename TA, int G, bool SMOOTH>
 __global__ __launch_bounds__(256) void spgemm_numeric_kernel(
     int n_rows, const int32_t* __restrict__ a_ptr, const int32_t* __restrict__ a_idx, const TA* __restrict__ a_val,
     const int32_t* __restrict__ b_ptr, const int32_t* __restrict__ b_idx, const double* __restrict__ b_val,
-    const int32_t* __restrict__ c_ptr, const int32_t* __restrict__ c_idx, double* __restrict__ c_val) {
+    const int32_t* __restrict__ c_ptr, const int32_t* __restrict__ c_idx, double* __restrict__ c_val,
+    const double* __restrict__ w) {
   constexpr int kRows = 256 / G, kChunk = 8 * G;
   constexpr int W = G == 64 ? 2 : 1, kPf = 8 / W;  // entries of a B row per lane, B rows in flight
   __shared__ int32_t s_cols[kRows][kChunk];
@@ -107,6 +109,15 @@ __global__ __launch_bounds__(256) void spgemm_numeric_kernel(
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    if (SMOOTH) {
+      const double scale = -w[row];
+      for (int t = lane; t < len; t += G) s_acc[t] *= scale;
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      for (int q = b_ptr[row] + lane; q < b_ptr[row + 1]; q += G) add(b_idx[q], b_val[q]);
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    }
     for (int t = lane; t < len; t += G) c_val[cs + t] = s_acc[t];
     __builtin_amdgcn_wave_barrier();
   }
@@ -115,18 +126,22 @@ __global__ __launch_bounds__(256) void spgemm_numeric_kernel(
 template <typename TA>
 void launch_spgemm(int n_rows, const int32_t* a_ptr, const int32_t* a_idx, const TA* a_val, const int32_t* b_ptr,
                    const int32_t* b_idx, const double* b_val, const int32_t* c_ptr, const int32_t* c_idx,
-                   double* c_val, int lanes, hipStream_t s) {
+                   double* c_val, const double* w, int lanes, hipStream_t s) {
   auto go = [&](auto kern) {
     const int rows = 256 / lanes;
     hipLaunchKernelGGL(kern, dim3((n_rows + rows - 1) / rows), dim3(256), 0, s, n_rows, a_ptr, a_idx, a_val, b_ptr,
-                       b_idx, b_val, c_ptr, c_idx, c_val);
+                       b_idx, b_val, c_ptr, c_idx, c_val, w);
   };
+#define SPGEMM_G(G)                                  \
+  if (w) go(spgemm_numeric_kernel<TA, G, true>);     \
+  else go(spgemm_numeric_kernel<TA, G, false>)
   switch (lanes) {
-    case 8: go(spgemm_numeric_kernel<TA, 8>); break;
-    case 16: go(spgemm_numeric_kernel<TA, 16>); break;
-    case 32: go(spgemm_numeric_kernel<TA, 32>); break;
-    default: go(spgemm_numeric_kernel<TA, 64>);
+    case 8: SPGEMM_G(8); break;
+    case 16: SPGEMM_G(16); break;
+    case 32: SPGEMM_G(32); break;
+    default: SPGEMM_G(64);
   }
+#undef SPGEMM_G
 }
 
 // Fused multigrid operators: one CSR pass per smoothing sweep, residual or prolongation.
@@ -478,6 +493,39 @@ extern "C" int fne_vcycle_cheb(int32_t n_rows, const int32_t* indptr, const int3
   return FNE_EINVAL;
 }
 
+namespace {
+int spgemm(const char* name, int32_t n_rows, const int32_t* a_indptr, const int32_t* a_indices, const void* a_vals,
+           int32_t a_precision, const int32_t* b_indptr, const int32_t* b_indices, const double* b_vals,
+           const int32_t* c_indptr, const int32_t* c_indices, double* c_vals, const double* w, fne_stream_t stream) {
+  if (n_rows == 0) return FNE_OK;
+  if (!a_indptr || !a_indices || !a_vals || !b_indptr || !b_indices || !b_vals || !c_indptr || !c_indices ||
+      !c_vals) {
+    fne_set_error(std::string(name) + ": null pointer");
+    return FNE_EINVAL;
+  }
+  int lanes = (a_precision >> 8) & 0xff;
+  if (lanes == 0) lanes = 64;
+  if (lanes != 8 && lanes != 16 && lanes != 32 && lanes != 64) {
+    fne_set_error(std::string(name) + ": lanes per row must be 8, 16, 32 or 64");
+    return FNE_EINVAL;
+  }
+  hipStream_t s = (hipStream_t)stream;
+  const int prec = a_precision & 0xff;
+  if (prec == FNE_FP64 && (a_precision >> 16) == 0)
+    launch_spgemm(n_rows, a_indptr, a_indices, (const double*)a_vals, b_indptr, b_indices, b_vals, c_indptr,
+                  c_indices, c_vals, w, lanes, s);
+  else if (prec == FNE_FP32 && (a_precision >> 16) == 0)
+    launch_spgemm(n_rows, a_indptr, a_indices, (const float*)a_vals, b_indptr, b_indices, b_vals, c_indptr,
+                  c_indices, c_vals, w, lanes, s);
+  else {
+    fne_set_error(std::string(name) + ": precision must be FNE_FP64 or FNE_FP32");
+    return FNE_EINVAL;
+  }
+  FNE_LAUNCH_CHECK();
+  return FNE_OK;
+}
+}  // namespace
+
 extern "C" int fne_spgemm_numeric(int32_t n_rows, const int32_t* a_indptr, const int32_t* a_indices,
                                   const void* a_vals, int32_t a_precision, const int32_t* b_indptr,
                                   const int32_t* b_indices, const double* b_vals, const int32_t* c_indptr,
@@ -486,30 +534,18 @@ extern "C" int fne_spgemm_numeric(int32_t n_rows, const int32_t* a_indptr, const
     fne_set_error("fne_spgemm_numeric: n_rows < 0");
     return FNE_EINVAL;
   }
-  if (n_rows == 0) return FNE_OK;
-  if (!a_indptr || !a_indices || !a_vals || !b_indptr || !b_indices || !b_vals || !c_indptr || !c_indices ||
-      !c_vals) {
-    fne_set_error("fne_spgemm_numeric: null pointer");
+  return spgemm("fne_spgemm_numeric", n_rows, a_indptr, a_indices, a_vals, a_precision, b_indptr, b_indices, b_vals,
+                c_indptr, c_indices, c_vals, nullptr, stream);
+}
+
+extern "C" int fne_spgemm_smoothed(int32_t n, const int32_t* a_indptr, const int32_t* a_indices, const void* a_vals,
+                                   int32_t a_precision, const int32_t* b_indptr, const int32_t* b_indices,
+                                   const double* b_vals, const int32_t* c_indptr, const int32_t* c_indices,
+                                   double* c_vals, const double* w, fne_stream_t stream) {
+  if (n < 0 || !w) {
+    fne_set_error("fne_spgemm_smoothed: n < 0 or null pointer");
     return FNE_EINVAL;
   }
-  int lanes = (a_precision >> 8) & 0xff;
-  if (lanes == 0) lanes = 64;
-  if (lanes != 8 && lanes != 16 && lanes != 32 && lanes != 64) {
-    fne_set_error("fne_spgemm_numeric: lanes per row must be 8, 16, 32 or 64");
-    return FNE_EINVAL;
-  }
-  hipStream_t s = (hipStream_t)stream;
-  const int prec = a_precision & 0xff;
-  if (prec == FNE_FP64 && (a_precision >> 16) == 0)
-    launch_spgemm(n_rows, a_indptr, a_indices, (const double*)a_vals, b_indptr, b_indices, b_vals, c_indptr,
-                  c_indices, c_vals, lanes, s);
-  else if (prec == FNE_FP32 && (a_precision >> 16) == 0)
-    launch_spgemm(n_rows, a_indptr, a_indices, (const float*)a_vals, b_indptr, b_indices, b_vals, c_indptr,
-                  c_indices, c_vals, lanes, s);
-  else {
-    fne_set_error("fne_spgemm_numeric: precision must be FNE_FP64 or FNE_FP32");
-    return FNE_EINVAL;
-  }
-  FNE_LAUNCH_CHECK();
-  return FNE_OK;
+  return spgemm("fne_spgemm_smoothed", n, a_indptr, a_indices, a_vals, a_precision, b_indptr, b_indices, b_vals,
+                c_indptr, c_indices, c_vals, w, stream);
 }

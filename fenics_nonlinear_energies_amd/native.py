@@ -135,6 +135,40 @@ _SIGNATURES = [
         [C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
          C.c_void_p, C.c_void_p, C.c_void_p],
     ),
+    (
+        "fne_spgemm_smoothed",
+        C.c_int,
+        [C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
+         C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p],
+    ),
+    ("fne_lanczos_work_len", C.c_int64, [C.c_int32, C.c_int32]),
+    (
+        "fne_lanczos_max",
+        C.c_int,
+        [C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p,
+         C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p],
+    ),
+    (
+        "fne_smoother_weights",
+        C.c_int,
+        [C.c_int32, C.c_void_p, C.c_void_p, C.c_double, _f64p, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p],
+    ),
+    (
+        "fne_amg_transfers",
+        C.c_int,
+        [C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p],
+    ),
+    (
+        "fne_amg_symmetrise",
+        C.c_int,
+        [C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p],
+    ),
+    ("fne_spd_inverse_work_len", C.c_int64, [C.c_int32]),
+    (
+        "fne_spd_inverse",
+        C.c_int,
+        [C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p],
+    ),
     ("fne_dot", C.c_int, [C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]),
     ("fne_dot_work_len", C.c_int32, []),
     (
@@ -253,6 +287,11 @@ def ptr(t) -> int | None:
     if t is None:
         return None
     return int(t.data_ptr())
+
+
+def f64_ptr(a):
+    """``double *`` of a contiguous host array (kept alive by the caller for the call)."""
+    return a.ctypes.data_as(_f64p)
 
 
 def stream_ptr(stream=None) -> int | None:

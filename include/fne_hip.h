@@ -297,6 +297,46 @@ int fne_spgemm_numeric(int32_t n_rows, const int32_t* a_indptr, const int32_t* a
                        fne_stream_t stream);
 
 /*
+ * C = B - diag(w) A B on C's pattern, which must hold B's: the smoothed prolongator of B = P_tent with
+ * w = omega D^-1 (n x n A, n-row B).  Otherwise as fne_spgemm_numeric.
+ */
+int fne_spgemm_smoothed(int32_t n, const int32_t* a_indptr, const int32_t* a_indices, const void* a_vals,
+                        int32_t a_precision, const int32_t* b_indptr, const int32_t* b_indices,
+                        const double* b_vals, const int32_t* c_indptr, const int32_t* c_indices, double* c_vals,
+                        const double* w, fne_stream_t stream);
+
+/*
+ * Largest eigenvalue of D^-1 A (as the Ritz value of `steps` <= 64 Lanczos steps on D^-1/2 A D^-1/2
+ * from v0), for the level smoothers' bounds; PETSc's GAMG estimates it with a Krylov method too
+ * (pc_type "gamg", hyperelasticity/jax_petsc/solver.py:138-143).  diag: index of each row's diagonal
+ * entry; dinv receives 1 / diagonal (1 where it is zero).  work: fne_lanczos_work_len(n, precision)
+ * doubles.  out (device): {eigenvalue (>= 1e-300), 1 if every coefficient was finite else 0}; nothing
+ * is read back.  precision as in fne_spmv.
+ */
+int64_t fne_lanczos_work_len(int32_t n, int32_t precision);
+int fne_lanczos_max(int32_t n, const int32_t* indptr, const int32_t* indices, const void* vals, int32_t precision,
+                    const int64_t* diag, const double* v0, int32_t steps, double* dinv, double* work,
+                    int64_t work_len, double* out, fne_stream_t stream);
+/* wd = wd_factor / lam[0] dinv and wcheb[k] = cheb_factors[k] / lam[0] dinv (k < n_cheb <= 8; HOST factors,
+ * device lam): the weights of the damped-Jacobi sweeps and of the Chebyshev steps. */
+int fne_smoother_weights(int32_t n, const double* dinv, const double* lam, double wd_factor,
+                         const double* cheb_factors, int32_t n_cheb, double* wd, double* wcheb, fne_stream_t stream);
+/* r[k] = p[perm[k]] (perm of the transpose), and p and r in the cycle's precision */
+int fne_amg_transfers(int32_t nnz, const double* p, const int64_t* perm, double* r, void* p_cycle, void* r_cycle,
+                      int32_t precision, fne_stream_t stream);
+/* a[k] = (c[k] + c[perm[k]]) / 2, and a in the cycle's precision unless a_cycle is NULL */
+int fne_amg_symmetrise(int32_t nnz, const double* c, const int64_t* perm, double* a, void* a_cycle,
+                       int32_t precision, fne_stream_t stream);
+/*
+ * Dense inverse (n x n, row-major, symmetric) of the symmetric part of a sparse FP64 matrix.  work:
+ * fne_spd_inverse_work_len(n) doubles.  status (device): 0, or 1 where a pivot was not positive and
+ * finite, i.e. the matrix is not positive definite and inv is not valid.
+ */
+int64_t fne_spd_inverse_work_len(int32_t n);
+int fne_spd_inverse(int32_t n, const int32_t* indptr, const int32_t* indices, const double* vals, double* work,
+                    int64_t work_len, double* inv, double* status, fne_stream_t stream);
+
+/*
  * Preconditioned CG on the device (KSPCG semantics: zero initial guess, point-Jacobi left
  * preconditioning via inv_diag (NULL = none), convergence when the preconditioned residual
  * norm <= max(rtol*initial, atol), divergence at dtol*initial, indefinite checks).  Replaces

@@ -165,6 +165,117 @@ def test_spgemm_lane_groups_match_scipy(require_gpu, lanes, a_prec):
     assert np.all(np.abs(got - (A @ B).toarray()) <= bound)
 
 
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("n,width", [(1, 1), (2, 2), (13, 3), (255, 7), (257, 30), (4097, 60), (150_000, 7)])
+def test_lanczos_and_smoothed_product_match_host(require_gpu, n, width, prec):
+    """fne_lanczos_max in both forms of its product against the host recurrence (the same Krylov
+    space in other roundings: 1e-9 of the eigenvalue), its inverse diagonal with a zero entry, and
+    fne_spgemm_smoothed; sizes around a block, above the partial sums one block adds up, and below
+    the number of steps."""
+    import scipy.sparse as sp
+    import torch
+
+    from fenics_nonlinear_energies_amd import amg, linalg, native
+
+    rng = np.random.default_rng(n)
+    off = [sp.diags(rng.uniform(-1.0, 0.0, n - k), k) for k in sorted({int(j) for j in np.linspace(1, n - 1, width)})
+           if 0 < k < n] if n > 1 else []
+    U = sum(off, sp.csr_matrix((n, n)))
+    A = (U + U.T + sp.diags(np.asarray(abs(U + U.T).sum(axis=1)).ravel() + rng.uniform(0.5, 1.0, n))).tocsr()
+    A.sort_indices()
+    if prec == "fp32":
+        A.data = A.data.astype(np.float32).astype(np.float64)
+    diag = amg._positions(A, np.arange(n), np.arange(n))
+    dev = torch.device("cuda")
+    ptr, idx = (torch.as_tensor(a.astype(np.int32)).to(dev) for a in (A.indptr, A.indices))
+    val = torch.as_tensor(A.data).to(dev, torch.float32 if prec == "fp32" else torch.float64)
+    dg, v0 = torch.as_tensor(diag).to(dev), torch.as_tensor(rng.standard_normal(n)).to(dev)
+    dinv, out = torch.empty(n, dtype=torch.float64, device=dev), torch.empty(2, dtype=torch.float64, device=dev)
+    base = native.FNE_FP32 if prec == "fp32" else native.FNE_FP64
+
+    class _Host:
+        @staticmethod
+        def mult_tensor(x, y):
+            y.copy_(torch.as_tensor(A @ x.numpy()))
+
+    ref = amg.SmoothedAggregationPC()._lanczos_lambda_max(0, _Host, torch.as_tensor(1.0 / A.diagonal()), v0.cpu())
+
+    def run(code, values):
+        m = int(native.lib().fne_lanczos_work_len(n, code))
+        assert m == amg._lanczos_work_len(n, code)
+        work = torch.full((m,), float("nan"), dtype=torch.float64, device=dev)
+        native.check(native.lib().fne_lanczos_max(n, native.ptr(ptr), native.ptr(idx), native.ptr(values), code,
+                                                  native.ptr(dg), native.ptr(v0), 12, native.ptr(dinv),
+                                                  native.ptr(work), m, native.ptr(out), native.stream_ptr()), "lanczos")
+        return out.cpu().numpy()
+
+    for code in (linalg.spmv_code(base, A.nnz / n), base, base | 64 << 8):
+        lam, ok = run(code, val)
+        assert ok == 1.0 and abs(lam - ref) <= 1e-9 * ref
+        np.testing.assert_array_equal(dinv.cpu().numpy(), 1.0 / A.diagonal())
+    holes = val.clone()
+    holes[diag[0]] = 0.0
+    assert np.isfinite(run(base, holes)).all() and dinv[0].item() == 1.0
+    holes[diag[n // 2]] = float("nan")
+    assert run(base, holes)[1] == 0.0
+
+    # P = P_tent - diag(w) A P_tent with aggregates of three
+    Pt, _ = amg.tentative_prolongator(rng.standard_normal((n, 1)), 3)
+    w = rng.uniform(0.1, 1.0, n)
+    C_pat = amg._pattern(amg._pattern_product(A, Pt) + amg._pattern(Pt))
+    B = amg._DevMat(Pt.indptr, Pt.indices, Pt.shape[1], dev, "fp64")
+    B.data.copy_(torch.as_tensor(Pt.data))
+    C = amg._DevMat(C_pat.indptr, C_pat.indices, C_pat.shape[1], dev, "fp64")
+    C.data.fill_(float("nan"))
+    amg._spgemm_smoothed(ptr, idx, val, B, C, torch.as_tensor(w).to(dev))
+    got = sp.csr_matrix((C.data.cpu().numpy(), C_pat.indices, C_pat.indptr), shape=C_pat.shape)
+    want = (Pt - sp.diags(w) @ (A @ Pt)).tocsr()
+    scale = abs(Pt) + sp.diags(w) @ (abs(A) @ abs(Pt))
+    # at most 61 products, the scaling and the addition
+    assert abs(got - want).max() <= 2 * 64 * 2.0**-53 * scale.max()
+
+
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 64, 97, 287])
+def test_spd_inverse_matches_numpy(require_gpu, n):
+    """fne_spd_inverse at the edges of its 32-column blocks: a matrix of condition 1e4 (n eps cond is
+    6e-10 at most of the inverse's largest entry), the symmetric part of an unsymmetric one, and the
+    status of an indefinite one and of a NaN."""
+    import scipy.sparse as sp
+    import torch
+
+    from fenics_nonlinear_energies_amd import native
+
+    rng = np.random.default_rng(n)
+    Q, _ = np.linalg.qr(rng.standard_normal((n, n)))
+    S = (Q * np.geomspace(1.0, 1e-4, n)) @ Q.T
+    S = 0.5 * (S + S.T)
+    K = rng.standard_normal((n, n)) * 1e-3
+    dev = torch.device("cuda")
+    m = int(native.lib().fne_spd_inverse_work_len(n))
+    work, inv = (torch.full((k,), float("nan"), dtype=torch.float64, device=dev) for k in (m, n * n))
+    status = torch.full((1,), 7.0, dtype=torch.float64, device=dev)
+
+    def run(M):
+        C = sp.csr_matrix(M)
+        ptr, idx = (torch.as_tensor(a.astype(np.int32)).to(dev) for a in (C.indptr, C.indices))
+        val = torch.as_tensor(C.data).to(dev)
+        native.check(native.lib().fne_spd_inverse(n, native.ptr(ptr), native.ptr(idx), native.ptr(val),
+                                                  native.ptr(work), m, native.ptr(inv), native.ptr(status),
+                                                  native.stream_ptr()), "fne_spd_inverse")
+        return inv.cpu().numpy().reshape(n, n), status.item()
+
+    X, st = run(S + (K - K.T))
+    ref = np.linalg.inv(S)
+    assert st == 0.0 and np.array_equal(X, X.T)
+    assert np.abs(X - ref).max() <= 1e-9 * np.abs(ref).max()
+    flip = np.geomspace(1.0, 1e-4, n)
+    flip[-1] = -0.5
+    assert run((Q * flip) @ Q.T)[1] == 1.0
+    bad = S.copy()
+    bad[n // 2, n // 2] = np.nan
+    assert run(bad)[1] == 1.0
+
+
 def _host_levels(pc, A0):
     """Operators of every level read back from the device (FP64 masters)."""
     import scipy.sparse as sp
