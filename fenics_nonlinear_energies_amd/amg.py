@@ -49,10 +49,18 @@ import torch
 from . import native
 
 
-def _spmv_code(prec: int, avg: float) -> int:
-    from .linalg import spmv_code
+# Operators with fewer entries than this take the row kernels' lanes-per-row form: the CSR-stream
+# form's 256 / lanes rows per workgroup leave most of the GPU idle there (smoothing step of 18,241
+# rows with 15 entries 6.6 against 4.1 us, of 2,281 with 55 8.2 against 3.9; 145,924 rows with 7
+# the other way, 5.2 against 7.8)
+_STREAM_MIN_NNZ = 600_000
 
-    return spmv_code(prec, avg)
+
+def _spmv_code(prec: int, avg: float, nnz: int) -> int:
+    """Precision argument (value type, form, lanes per row) of a level's row kernels."""
+    from .linalg import lanes_per_row, spmv_code
+
+    return prec | lanes_per_row(avg) << 8 if nnz < _STREAM_MIN_NNZ else spmv_code(prec, avg)
 
 
 # fne_vcycle_op operations
@@ -71,7 +79,7 @@ class _DevMat:
         dt = torch.float32 if precision == "fp32" else torch.float64
         self.data = torch.zeros(self.nnz, dtype=dt, device=device)
         self.prec = native.FNE_FP32 if precision == "fp32" else native.FNE_FP64
-        self.code = _spmv_code(self.prec, self.nnz / max(1, self.n_rows))
+        self.code = _spmv_code(self.prec, self.nnz / max(1, self.n_rows), self.nnz)
 
     @classmethod
     def sharing_pattern(cls, indptr: torch.Tensor, indices: torch.Tensor, n_cols: int, precision: str) -> "_DevMat":
@@ -82,7 +90,7 @@ class _DevMat:
         dt = torch.float32 if precision == "fp32" else torch.float64
         m.data = torch.zeros(m.nnz, dtype=dt, device=indices.device)
         m.prec = native.FNE_FP32 if precision == "fp32" else native.FNE_FP64
-        m.code = _spmv_code(m.prec, m.nnz / max(1, m.n_rows))
+        m.code = _spmv_code(m.prec, m.nnz / max(1, m.n_rows), m.nnz)
         return m
 
     def op(self, op: int, x, r, w, y_in, y: torch.Tensor) -> None:
@@ -103,6 +111,15 @@ class _DevMat:
                                          native.ptr(x_prev), native.ptr(r), native.ptr(w), float(c), native.ptr(y),
                                          native.stream_ptr()),
             "fne_vcycle_cheb",
+        )
+
+    def cheb_first(self, r, w0, w, c: float, y: torch.Tensor) -> None:
+        """The first two Chebyshev steps from zero (fne_vcycle_cheb_first)."""
+        native.check(
+            native.lib().fne_vcycle_cheb_first(self.n_rows, native.ptr(self.indptr), native.ptr(self.indices),
+                                               native.ptr(self.data), self.code, native.ptr(r), native.ptr(w0),
+                                               native.ptr(w), float(c), native.ptr(y), native.stream_ptr()),
+            "fne_vcycle_cheb_first",
         )
 
     def mult(self, x: torch.Tensor, y: torch.Tensor) -> None:
@@ -128,6 +145,8 @@ def _spgemm(a_indptr, a_indices, a_data, b: _DevMat, b_data: torch.Tensor, c: _D
     n_rows = int(a_indptr.numel() - 1)
     prec = native.FNE_FP32 if a_data.dtype == torch.float32 else native.FNE_FP64
     prec |= _spgemm_lanes(b.nnz / max(1, b.n_rows)) << 8
+    if prec >> 8 == 64 and n_rows <= 1024:  # a workgroup per row where there are few (4 per CU)
+        prec |= 1 << 16
     native.check(
         native.lib().fne_spgemm_numeric(n_rows, native.ptr(a_indptr), native.ptr(a_indices), native.ptr(a_data), prec,
                                         native.ptr(b.indptr), native.ptr(b.indices), native.ptr(b_data),
@@ -409,7 +428,7 @@ class SmoothedAggregationPC:
         # scratch of a numeric set-up, one stage at a time: the Lanczos vectors, an unsymmetrised
         # coarse product, the two copies of the coarse matrix during its inversion
         need = [L["Ac64"].nnz for L in levels]
-        code0 = _spmv_code(native.FNE_FP64, A0.nnz / max(1, n))
+        code0 = _spmv_code(native.FNE_FP64, A0.nnz / max(1, n), A0.nnz)
         need += [_lanczos_work_len(L["n"], code0 if i == 0 else levels[i - 1]["Ac64"].code)
                  for i, L in enumerate(levels)]
         if self.coarse_factor == "device":
@@ -516,7 +535,7 @@ class SmoothedAggregationPC:
             pt_vals = self._tentative_values(Bh)
         lib, stream = native.lib(), native.stream_ptr()
         a_ptr, a_idx, a_dat = A0.indptr, A0.indices, A0.data
-        a_code = _spmv_code(A0.fne_precision, A0.nnz / max(1, A0.n))
+        a_code = _spmv_code(A0.fne_precision, A0.nnz / max(1, A0.n), A0.nnz)
         if self.levels:
             self.levels[0]["A"].data.copy_(A0.data)
         nl = len(self.levels)
@@ -660,41 +679,54 @@ class SmoothedAggregationPC:
         side.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(side):
             for _ in range(2):
-                self._g_out.copy_(self._cycle(0, self._g_in))
+                self._cycle_to_out()
         torch.cuda.current_stream().wait_stream(side)
         g = torch.cuda.CUDAGraph()
         with torch.cuda.graph(g):
-            self._g_out.copy_(self._cycle(0, self._g_in))
+            self._cycle_to_out()
         self._graph = g
 
-    def _coarse_solve(self, r: torch.Tensor) -> torch.Tensor:
-        y = torch.empty(self.coarse_op.n_rows, dtype=r.dtype, device=r.device)
+    def _cycle_to_out(self) -> None:
+        x = self._cycle(0, self._g_in, self._g_out)
+        if x is not self._g_out:  # no smoothing step after the correction
+            self._g_out.copy_(x)
+
+    def _coarse_solve(self, r: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
+        y = torch.empty(self.coarse_op.n_rows, dtype=r.dtype, device=r.device) if out is None else out
         self.coarse_op.mult(r, y)
         return y
 
-    def _cheb_smooth(self, L: dict, r: torch.Tensor, x: torch.Tensor | None) -> torch.Tensor:
+    def _cheb_smooth(self, L: dict, r: torch.Tensor, x: torch.Tensor | None,
+                     out: torch.Tensor | None = None) -> torch.Tensor:
         """``sweeps`` Chebyshev steps on A x = r from x (from zero when x is None): step k is
         x_{k+1} = x_k + c_k (x_k - x_{k-1}) + w_k (r - A x_k), one CSR pass (fne_vcycle_cheb);
-        from zero the first step is x_1 = w_0 r."""
+        from zero the first step is x_1 = w_0 r, and two steps are one pass."""
         A, W, cs = L["A"], L["wcheb"], self._cheb_coefs()
         x_prev = None
         start = 0
+        if x is None and W.shape[0] == 2:
+            y = torch.empty_like(r) if out is None else out
+            A.cheb_first(r, W[0], W[1], cs[1], y)
+            return y
         if x is None:
             x = W[0] * r
             x_prev = torch.zeros_like(r)
             start = 1
         for k in range(start, W.shape[0]):
-            y = x_prev if (x_prev is not None and k > 1) else torch.empty_like(r)
+            if out is not None and k == W.shape[0] - 1:
+                y = out
+            else:
+                y = x_prev if (x_prev is not None and k > 1) else torch.empty_like(r)
             A.cheb(x, x_prev if cs[k] != 0.0 else None, r, W[k], cs[k], y)
             x_prev, x = x, y
         return x
 
-    def _cycle(self, lvl: int, r: torch.Tensor) -> torch.Tensor:
-        """One V-cycle from level ``lvl``: a fused CSR pass per smoothing step, residual and
-        prolongation.  Jacobi: x_{k+1} = x_k + w (r - A x_k), w = omega D^-1, from x = 0;
-        Chebyshev: ``_cheb_smooth``."""
+    def _cycle(self, lvl: int, r: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
+        """One V-cycle from level ``lvl`` (into ``out`` if given): a fused CSR pass per smoothing
+        step, residual and prolongation.  Jacobi: x_{k+1} = x_k + w (r - A x_k), w = omega D^-1,
+        from x = 0; Chebyshev: ``_cheb_smooth``."""
         if lvl == len(self.levels):
-            return self._coarse_solve(r)
+            return self._coarse_solve(r, out)
         L = self.levels[lvl]
         A, wd = L["A"], L["wd"]
         t = torch.empty_like(r)
@@ -714,8 +746,10 @@ class SmoothedAggregationPC:
         xc = self._cycle(lvl + 1, rc)
         L["P"].op(_ADD_PRODUCT, xc, None, None, x, x)
         if self.smoother == "chebyshev":
-            return self._cheb_smooth(L, r, x)
-        for _ in range(self.sweeps):
+            return self._cheb_smooth(L, r, x, out)
+        for k in range(self.sweeps):
+            if out is not None and k == self.sweeps - 1:
+                t = out
             A.op(_SWEEP, x, r, wd, None, t)
             x, t = t, x
         return x

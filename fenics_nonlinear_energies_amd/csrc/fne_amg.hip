@@ -23,23 +23,31 @@
 namespace {
 
 // SMOOTH: C = B - diag(w) A B, the smoothed prolongator of B = P_tent
-template <typename TA, int G, bool SMOOTH>
+// SPLIT (G = 64): the workgroup's four wavefronts share one row, each a contiguous quarter of A's row with
+// accumulators of its own, joined in order: for the few long rows of coarse levels (286 rows of 117
+// entries, 62-entry rows of B: 131 -> 40 us).
+template <typename TA, int G, bool SMOOTH, bool SPLIT>
 __global__ __launch_bounds__(256) void spgemm_numeric_kernel(
     int n_rows, const int32_t* __restrict__ a_ptr, const int32_t* __restrict__ a_idx, const TA* __restrict__ a_val,
     const int32_t* __restrict__ b_ptr, const int32_t* __restrict__ b_idx, const double* __restrict__ b_val,
     const int32_t* __restrict__ c_ptr, const int32_t* __restrict__ c_idx, double* __restrict__ c_val,
     const double* __restrict__ w) {
-  constexpr int kRows = 256 / G, kChunk = 8 * G;
+  constexpr int kGroups = 256 / G, kRows = SPLIT ? 1 : kGroups, kChunk = 8 * G;
   constexpr int W = G == 64 ? 2 : 1, kPf = 8 / W;  // entries of a B row per lane, B rows in flight
-  __shared__ int32_t s_cols[kRows][kChunk];
-  __shared__ double s_accs[kRows][kChunk];
+  __shared__ int32_t s_cols[kGroups][kChunk];
+  __shared__ double s_accs[kGroups][kChunk];
   const int lane = threadIdx.x & (G - 1), grp = threadIdx.x / G;
   int32_t* s_col = s_cols[grp];
   double* s_acc = s_accs[grp];
-  const int row = xcd_remap(blockIdx.x, gridDim.x) * kRows + grp;
-  if (row >= n_rows) return;  // the whole lane group; no block-level barrier below
+  const int row = xcd_remap(blockIdx.x, gridDim.x) * kRows + (SPLIT ? 0 : grp);
+  if (row >= n_rows) return;  // the whole lane group (SPLIT: workgroup); no block-level barrier unless SPLIT
   const int c0 = c_ptr[row], c1 = c_ptr[row + 1];
-  const int a0 = a_ptr[row], a1 = a_ptr[row + 1];
+  int a0 = a_ptr[row], a1 = a_ptr[row + 1];
+  if (SPLIT) {
+    const int per = (a1 - a0 + kGroups - 1) / kGroups;
+    a0 = min(a0 + grp * per, a1);
+    a1 = min(a0 + per, a1);
+  }
   for (int cs = c0; cs < c1; cs += kChunk) {
     const int len = min(kChunk, c1 - cs);
     for (int t = lane; t < len; t += G) {
@@ -109,6 +117,15 @@ __global__ __launch_bounds__(256) void spgemm_numeric_kernel(
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    if (SPLIT) {
+      __syncthreads();
+      if (grp == 0) {
+        for (int t = lane; t < len; t += G) {
+#pragma unroll
+          for (int i = 1; i < kGroups; ++i) s_acc[t] += s_accs[i][t];
+        }
+      }
+    }
     if (SMOOTH) {
       const double scale = -w[row];
       for (int t = lane; t < len; t += G) s_acc[t] *= scale;
@@ -118,7 +135,9 @@ __global__ __launch_bounds__(256) void spgemm_numeric_kernel(
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     }
-    for (int t = lane; t < len; t += G) c_val[cs + t] = s_acc[t];
+    if (!SPLIT || grp == 0)
+      for (int t = lane; t < len; t += G) c_val[cs + t] = s_acc[t];
+    if (SPLIT) __syncthreads();  // before the next chunk's columns
     __builtin_amdgcn_wave_barrier();
   }
 }
@@ -126,15 +145,19 @@ __global__ __launch_bounds__(256) void spgemm_numeric_kernel(
 template <typename TA>
 void launch_spgemm(int n_rows, const int32_t* a_ptr, const int32_t* a_idx, const TA* a_val, const int32_t* b_ptr,
                    const int32_t* b_idx, const double* b_val, const int32_t* c_ptr, const int32_t* c_idx,
-                   double* c_val, const double* w, int lanes, hipStream_t s) {
+                   double* c_val, const double* w, int lanes, bool split, hipStream_t s) {
   auto go = [&](auto kern) {
-    const int rows = 256 / lanes;
+    const int rows = split ? 1 : 256 / lanes;
     hipLaunchKernelGGL(kern, dim3((n_rows + rows - 1) / rows), dim3(256), 0, s, n_rows, a_ptr, a_idx, a_val, b_ptr,
                        b_idx, b_val, c_ptr, c_idx, c_val, w);
   };
-#define SPGEMM_G(G)                                  \
-  if (w) go(spgemm_numeric_kernel<TA, G, true>);     \
-  else go(spgemm_numeric_kernel<TA, G, false>)
+#define SPGEMM_G(G)                                         \
+  if (w) go(spgemm_numeric_kernel<TA, G, true, false>);     \
+  else go(spgemm_numeric_kernel<TA, G, false, false>)
+  if (split) {
+    go(spgemm_numeric_kernel<TA, 64, false, true>);
+    return;
+  }
   switch (lanes) {
     case 8: SPGEMM_G(8); break;
     case 16: SPGEMM_G(16); break;
@@ -405,8 +428,10 @@ extern "C" int fne_vcycle_op(int32_t op, int32_t n_rows, const int32_t* indptr, 
 // pass.  With w = (2 rho_k / delta) D^-1 and c = rho_k rho_{k-1} it is step k of the Chebyshev
 // iteration for D^-1 A on [a, b] (theta = (a + b) / 2, delta = (b - a) / 2); x_prev may be null
 // when c = 0.  y may alias x_prev (each row reads its own x_prev entry before writing it).
+// FIRST: the first two steps from x = 0 in the one pass, with x = w0.r read as the product it is
+// (x_prev = w0, and the x_prev of the second step is zero).
 namespace {
-template <typename VT, int LPR, int FORM>
+template <typename VT, int LPR, int FORM, bool FIRST>
 __global__ __launch_bounds__(256) void vcycle_cheb_kernel(int n, const int32_t* __restrict__ indptr,
                                                           const int32_t* __restrict__ indices,
                                                           const VT* __restrict__ vals, const double* __restrict__ x,
@@ -416,16 +441,20 @@ __global__ __launch_bounds__(256) void vcycle_cheb_kernel(int n, const int32_t* 
   int row;
   bool leader;
   const double acc =
-      csr_form_dot<VT, LPR, FORM>(n, indptr, indices, vals, [&](int col) { return x[col]; }, prod, row, leader);
+      csr_form_dot<VT, LPR, FORM>(n, indptr, indices, vals, [&](int col) { return FIRST ? x_prev[col] * r[col] : x[col]; }, prod,
+                                  row, leader);
   if (leader) {
-    const double xr = x[row];
+    const double xr = FIRST ? x_prev[row] * r[row] : x[row];
     double out = xr + w[row] * (r[row] - acc);
-    if (x_prev) out += c * (xr - x_prev[row]);
+    if (FIRST)
+      out += c * xr;
+    else if (x_prev)
+      out += c * (xr - x_prev[row]);
     y[row] = out;
   }
 }
 
-template <typename VT>
+template <typename VT, bool FIRST>
 int launch_vcycle_cheb(int n, const int32_t* indptr, const int32_t* indices, const VT* vals, const double* x,
                        const double* x_prev, const double* r, const double* w, double c, double* y, int lpr,
                        int form, hipStream_t s) {
@@ -436,9 +465,9 @@ int launch_vcycle_cheb(int n, const int32_t* indptr, const int32_t* indices, con
   };
 #define CHEB_L(L)                                                   \
   case L:                                                           \
-    if (form == 2) go(vcycle_cheb_kernel<VT, L, 2>, L);              \
-    else if (form == 1) go(vcycle_cheb_kernel<VT, L, 1>, L);         \
-    else go(vcycle_cheb_kernel<VT, L, 0>, L);                        \
+    if (form == 2) go(vcycle_cheb_kernel<VT, L, 2, FIRST>, L);              \
+    else if (form == 1) go(vcycle_cheb_kernel<VT, L, 1, FIRST>, L);         \
+    else go(vcycle_cheb_kernel<VT, L, 0, FIRST>, L);                        \
     break;
   switch (lpr) {
     CHEB_L(1)
@@ -448,13 +477,37 @@ int launch_vcycle_cheb(int n, const int32_t* indptr, const int32_t* indices, con
     CHEB_L(16)
     CHEB_L(32)
     default:
-      if (form == 2) go(vcycle_cheb_kernel<VT, 64, 2>, 64);
-      else if (form == 1) go(vcycle_cheb_kernel<VT, 64, 1>, 64);
-      else go(vcycle_cheb_kernel<VT, 64, 0>, 64);
+      if (form == 2) go(vcycle_cheb_kernel<VT, 64, 2, FIRST>, 64);
+      else if (form == 1) go(vcycle_cheb_kernel<VT, 64, 1, FIRST>, 64);
+      else go(vcycle_cheb_kernel<VT, 64, 0, FIRST>, 64);
   }
 #undef CHEB_L
   FNE_LAUNCH_CHECK();
   return FNE_OK;
+}
+}  // namespace
+
+namespace {
+template <bool FIRST>
+int vcycle_cheb(const char* name, int32_t n_rows, const int32_t* indptr, const int32_t* indices, const void* vals,
+                int32_t precision, const double* x, const double* x_prev, const double* r, const double* w, double c,
+                double* y, hipStream_t s) {
+  int lpr = (precision >> 8) & 0xff;
+  if (lpr == 0) lpr = 8;
+  if (lpr != 1 && lpr != 2 && lpr != 4 && lpr != 8 && lpr != 16 && lpr != 32 && lpr != 64) {
+    fne_set_error(std::string(name) + ": lanes per row must be a power of two <= 64");
+    return FNE_EINVAL;
+  }
+  const int prec = precision & 0xff;
+  const int form = csr_kernel_form(precision, indices, vals, lpr);
+  if (prec == FNE_FP64)
+    return launch_vcycle_cheb<double, FIRST>(n_rows, indptr, indices, (const double*)vals, x, x_prev, r, w, c, y, lpr,
+                                             form, s);
+  if (prec == FNE_FP32)
+    return launch_vcycle_cheb<float, FIRST>(n_rows, indptr, indices, (const float*)vals, x, x_prev, r, w, c, y, lpr,
+                                            form, s);
+  fne_set_error(std::string(name) + ": precision must be FNE_FP64 or FNE_FP32");
+  return FNE_EINVAL;
 }
 }  // namespace
 
@@ -474,23 +527,28 @@ extern "C" int fne_vcycle_cheb(int32_t n_rows, const int32_t* indptr, const int3
     fne_set_error("fne_vcycle_cheb: the output aliases an input read across rows");
     return FNE_EINVAL;
   }
-  int lpr = (precision >> 8) & 0xff;
-  if (lpr == 0) lpr = 8;
-  if (lpr != 1 && lpr != 2 && lpr != 4 && lpr != 8 && lpr != 16 && lpr != 32 && lpr != 64) {
-    fne_set_error("fne_vcycle_cheb: lanes per row must be a power of two <= 64");
+  return vcycle_cheb<false>("fne_vcycle_cheb", n_rows, indptr, indices, vals, precision, x, x_prev, r, w, c, y,
+                            (hipStream_t)stream);
+}
+
+extern "C" int fne_vcycle_cheb_first(int32_t n_rows, const int32_t* indptr, const int32_t* indices, const void* vals,
+                                     int32_t precision, const double* r, const double* w0, const double* w, double c,
+                                     double* y, fne_stream_t stream) {
+  if (n_rows < 0) {
+    fne_set_error("fne_vcycle_cheb_first: n_rows < 0");
     return FNE_EINVAL;
   }
-  const int prec = precision & 0xff;
-  const int form = csr_kernel_form(precision, indices, vals, lpr);
-  hipStream_t s = (hipStream_t)stream;
-  if (prec == FNE_FP64)
-    return launch_vcycle_cheb<double>(n_rows, indptr, indices, (const double*)vals, x, x_prev, r, w, c, y, lpr, form,
-                                      s);
-  if (prec == FNE_FP32)
-    return launch_vcycle_cheb<float>(n_rows, indptr, indices, (const float*)vals, x, x_prev, r, w, c, y, lpr, form,
-                                     s);
-  fne_set_error("fne_vcycle_cheb: precision must be FNE_FP64 or FNE_FP32");
-  return FNE_EINVAL;
+  if (n_rows == 0) return FNE_OK;
+  if (!indptr || !indices || !vals || !r || !w0 || !w || !y) {
+    fne_set_error("fne_vcycle_cheb_first: null pointer");
+    return FNE_EINVAL;
+  }
+  if (y == r || y == w0 || y == w) {
+    fne_set_error("fne_vcycle_cheb_first: the output aliases an input read across rows");
+    return FNE_EINVAL;
+  }
+  return vcycle_cheb<true>("fne_vcycle_cheb_first", n_rows, indptr, indices, vals, precision, nullptr, w0, r, w, c, y,
+                           (hipStream_t)stream);
 }
 
 namespace {
@@ -510,13 +568,18 @@ int spgemm(const char* name, int32_t n_rows, const int32_t* a_indptr, const int3
     return FNE_EINVAL;
   }
   hipStream_t s = (hipStream_t)stream;
-  const int prec = a_precision & 0xff;
-  if (prec == FNE_FP64 && (a_precision >> 16) == 0)
+  const int prec = a_precision & 0xff, flags = a_precision >> 16;
+  const bool split = flags == 1;
+  if ((flags & ~1) != 0 || (split && (lanes != 64 || w))) {
+    fne_set_error(std::string(name) + ": rows are split over 64-lane groups of a plain product only");
+    return FNE_EINVAL;
+  }
+  if (prec == FNE_FP64)
     launch_spgemm(n_rows, a_indptr, a_indices, (const double*)a_vals, b_indptr, b_indices, b_vals, c_indptr,
-                  c_indices, c_vals, w, lanes, s);
-  else if (prec == FNE_FP32 && (a_precision >> 16) == 0)
+                  c_indices, c_vals, w, lanes, split, s);
+  else if (prec == FNE_FP32)
     launch_spgemm(n_rows, a_indptr, a_indices, (const float*)a_vals, b_indptr, b_indices, b_vals, c_indptr,
-                  c_indices, c_vals, w, lanes, s);
+                  c_indices, c_vals, w, lanes, split, s);
   else {
     fne_set_error(std::string(name) + ": precision must be FNE_FP64 or FNE_FP32");
     return FNE_EINVAL;

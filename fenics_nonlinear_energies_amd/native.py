@@ -141,6 +141,12 @@ _SIGNATURES = [
         [C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
          C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p],
     ),
+    (
+        "fne_vcycle_cheb_first",
+        C.c_int,
+        [C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_double,
+         C.c_void_p, C.c_void_p],
+    ),
     ("fne_lanczos_work_len", C.c_int64, [C.c_int32, C.c_int32]),
     (
         "fne_lanczos_max",

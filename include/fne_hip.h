@@ -286,10 +286,17 @@ int fne_vcycle_cheb(int32_t n_rows, const int32_t* indptr, const int32_t* indice
                     int32_t precision, const double* x, const double* x_prev, const double* r, const double* w,
                     double c, double* y, fne_stream_t stream);
 
+/* The first two Chebyshev steps from x = 0 in one pass: with x_1 = w0.r,
+ *   y = x_1 + c x_1 + w.(r - A x_1)            (y must not alias r, w0 or w) */
+int fne_vcycle_cheb_first(int32_t n_rows, const int32_t* indptr, const int32_t* indices, const void* vals,
+                          int32_t precision, const double* r, const double* w0, const double* w, double c, double* y,
+                          fne_stream_t stream);
+
 /*
  * c = A B on C's pattern (columns outside it are dropped).  a_precision: FNE_FP64 / FNE_FP32 |
  * lanes_per_row << 8 (8, 16, 32 or 64; 0 = 64): lanes for about 1.5 of B's average rows do best; the
- * sums are the same for all.
+ * sums are the same for all.  1 << 16 with 64 lanes: four groups share a row, for few long rows (A's row
+ * in four parts, joined in order).
  */
 int fne_spgemm_numeric(int32_t n_rows, const int32_t* a_indptr, const int32_t* a_indices, const void* a_vals,
                        int32_t a_precision, const int32_t* b_indptr, const int32_t* b_indices,

@@ -165,6 +165,73 @@ def test_spgemm_lane_groups_match_scipy(require_gpu, lanes, a_prec):
     assert np.all(np.abs(got - (A @ B).toarray()) <= bound)
 
 
+@pytest.mark.parametrize("a_prec", ["fp64", "fp32"])
+def test_spgemm_split_rows_match_scipy(require_gpu, a_prec):
+    """Four lane groups per row: rows of A shorter than four, with and without a remainder, result rows
+    longer than the staged columns; a sum of at most 300 products in another order."""
+    import scipy.sparse as sp
+    import torch
+
+    from fenics_nonlinear_energies_amd import amg, native
+
+    rng = np.random.default_rng(5)
+    lengths = [0, 1, 2, 3, 4, 5, 63, 64, 65, 255, 256, 257, 300]
+    ptr = np.concatenate(([0], np.cumsum(lengths)))
+    cols = np.concatenate([np.sort(rng.choice(301, size=m, replace=False)) for m in lengths]).astype(int)
+    A = sp.csr_matrix((rng.standard_normal(ptr[-1]), cols, ptr), shape=(len(lengths), 301))
+    B = sp.random(301, 900, density=0.08, random_state=9, format="csr")
+    if a_prec == "fp32":
+        A.data = A.data.astype(np.float32).astype(np.float64)
+    C_pat = amg._pattern_product(A, B)
+    assert np.diff(C_pat.indptr).max() > 512 and np.diff(B.indptr).max() > 64
+    dev = torch.device("cuda")
+    i32 = lambda a: torch.as_tensor(a.astype(np.int32)).to(dev)  # noqa: E731
+    prec = native.FNE_FP32 if a_prec == "fp32" else native.FNE_FP64
+    args = [i32(A.indptr), i32(A.indices), torch.as_tensor(A.data).to(dev, torch.float32 if prec == native.FNE_FP32
+                                                                      else torch.float64)]
+    rest = [i32(B.indptr), i32(B.indices), torch.as_tensor(B.data).to(dev), i32(C_pat.indptr), i32(C_pat.indices)]
+    val = torch.full((C_pat.nnz,), float("nan"), dtype=torch.float64, device=dev)
+
+    def run(code):
+        return native.lib().fne_spgemm_numeric(A.shape[0], *(native.ptr(t) for t in args), code,
+                                               *(native.ptr(t) for t in rest), native.ptr(val), native.stream_ptr())
+
+    assert run(prec | 32 << 8 | 1 << 16) != 0 and run(prec | 64 << 8 | 2 << 16) != 0
+    native.check(run(prec | 64 << 8 | 1 << 16), "fne_spgemm_numeric")
+    got = sp.csr_matrix((val.cpu().numpy(), C_pat.indices, C_pat.indptr), shape=C_pat.shape).toarray()
+    bound = 2 * 304 * 2.0**-53 * (abs(A) @ abs(B)).toarray()
+    assert np.all(np.abs(got - (A @ B).toarray()) <= bound)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("n,width", [(1, 1), (255, 7), (257, 60), (4097, 20)])
+def test_first_two_chebyshev_steps_equal_the_steps_one_by_one(require_gpu, n, width, prec):
+    """fne_vcycle_cheb_first against w_0 r and fne_vcycle_cheb with a zero vector before it, in the forms of the row
+    kernels: the same sums, and one more or one less fused multiply-add per entry."""
+    import scipy.sparse as sp
+    import torch
+
+    from fenics_nonlinear_energies_amd import amg, linalg, native
+
+    rng = np.random.default_rng(n)
+    A = (sp.random(n, n, density=min(1.0, width / n), random_state=2) + sp.identity(n)).tocsr()
+    A.sort_indices()
+    dev = torch.device("cuda")
+    M = amg._DevMat(A.indptr, A.indices, n, dev, prec)
+    M.data.copy_(torch.as_tensor(A.data))
+    r, w0, w1 = (torch.as_tensor(rng.uniform(0.5, 1.5, n)).to(dev) for _ in range(3))
+    for code in (linalg.spmv_code(M.prec, A.nnz / n), M.prec, M.prec | 64 << 8, M.prec | 1 << 8):
+        M.code = code
+        y, ref = torch.full_like(r, float("nan")), torch.empty_like(r)
+        M.cheb_first(r, w0, w1, 0.3, y)
+        M.cheb(w0 * r, torch.zeros_like(r), r, w1, 0.3, ref)
+        # |A| x_1 is at most 2.25 (nnz of the row); a few roundings of each product
+        assert (y - ref).abs().max().item() <= 8 * 2.0**-53 * 1.5 * 2.25 * (2 + np.diff(A.indptr).max())
+    assert native.lib().fne_vcycle_cheb_first(n, native.ptr(M.indptr), native.ptr(M.indices), native.ptr(M.data),
+                                              M.code, native.ptr(r), native.ptr(w0), native.ptr(w1), 0.3,
+                                              native.ptr(r), native.stream_ptr()) != 0
+
+
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
 @pytest.mark.parametrize("n,width", [(1, 1), (2, 2), (13, 3), (255, 7), (257, 30), (4097, 60), (150_000, 7)])
 def test_lanczos_and_smoothed_product_match_host(require_gpu, n, width, prec):
