@@ -77,6 +77,7 @@ struct FneRowUnits {
 struct fne_plan {
   fne_plan_desc d;
   double2* partials = nullptr;  // per-block (sum, compensation) pairs for energy reductions
+  int energy_blocks = 0;  // set by fne_energy_partials
   int n_partials = 0;
   int device = 0;
   int mode = 0;  // constitutive mode (Mohr-Coulomb: 0 full, 1 elastic)
@@ -370,6 +371,9 @@ int fne_launch_p1(fne_plan* plan, FneOp op, const FneCall& c);
 int fne_launch_tet(fne_plan* plan, FneOp op, const FneCall& c);
 int fne_launch_mc(fne_plan* plan, FneOp op, const FneCall& c);
 int fne_finalize_energy(fne_plan* plan, int nblocks, double* out, hipStream_t stream);
+// the energy's per-block (sum, compensation) pairs in plan->partials, without their sum
+int fne_energy_partials(fne_plan* plan, const double* x, const double* dvals, const double* f, int* nblocks,
+                        hipStream_t stream);
 // bytes of the element-matrix scratch (and, via gbytes, of the gradient scratch) used by the
 // row-gather assembly (Mohr-Coulomb always, tetrahedra with FNE_FLAG_ROW_GATHER)
 size_t fne_mc_scratch_bytes(const fne_plan_desc& d, size_t* gbytes);

@@ -251,9 +251,26 @@ FneCall make_call(const double* x, const double* dvals, const double* f, hipStre
 void fne_set_error(const std::string& msg) { g_last_error = msg; }
 
 int fne_finalize_energy(fne_plan* plan, int nblocks, double* out, hipStream_t stream) {
+  if (!out) {  // fne_energy_partials: the caller adds the blocks up
+    plan->energy_blocks = nblocks;
+    return FNE_OK;
+  }
   hipLaunchKernelGGL(finalize_pairs_kernel, dim3(1), dim3(kFinalizeThreads), 0, stream, plan->partials, nblocks,
                      out);
   FNE_LAUNCH_CHECK();
+  return FNE_OK;
+}
+
+int fne_energy_partials(fne_plan* plan, const double* x, const double* dvals, const double* f, int* nblocks,
+                        hipStream_t stream) {
+  plan->energy_blocks = -1;
+  const int rc = dispatch(plan, kOpEnergy, make_call(x, dvals, f, stream));
+  if (rc) return rc;
+  if (plan->energy_blocks < 0) {
+    fne_set_error("the energy left no partial sums");
+    return FNE_EUNSUPPORTED;
+  }
+  *nblocks = plan->energy_blocks;
   return FNE_OK;
 }
 

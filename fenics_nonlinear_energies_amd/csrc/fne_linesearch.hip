@@ -2,12 +2,14 @@
 //
 // The Newton driver's line search minimises J(x + alpha p) over [lo, hi] by golden-section
 // search; each step needs one energy, and the host's only work between energies is comparing
-// two numbers.  Here that comparison runs in a one-thread kernel after each energy: the state
-// holds the bracket, the two interior points and their values, the best point so far and the
-// next alpha to evaluate, so the host enqueues trial-point / energy / step triples back to back
-// and synchronises once at the end.  The arithmetic and the order of every comparison are the
-// reference's (same points, same tie-breaking), so the chosen alpha is the one the host
-// search would choose from the same energies.
+// two numbers.  Here the comparison runs on the device: the state holds the bracket, the two interior
+// points and their values, the best point so far and the next alpha to evaluate, so the host enqueues
+// the whole search and synchronises once at the end.  A point is two launches, the energy's partial
+// sums and golden_point_kernel (fne_golden_search); both are bound by latency (4.7 and 3.8 us on the
+// 160x8x8 beam, 24 points 251 us; four launches per point enqueued one by one took 404 to 438).
+// fne_golden_trial and fne_golden_step are the same steps for energies that the caller evaluates.
+// The arithmetic and the order of every comparison are the reference's (same points, same
+// tie-breaking), so the chosen alpha is the one the host search would choose from the same energies.
 #include "fne_common.h"
 
 #include <algorithm>
@@ -72,11 +74,9 @@ __device__ __forceinline__ void golden_probe(double* st, double a, double f) {
   }
 }
 
-__global__ void golden_step_kernel(double* __restrict__ st, const double* __restrict__ f_new) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+__device__ void golden_step(double* st, double v) {
   const int phase = int(st[kPhase]);
   if (phase >= 7) return;
-  double v = f_new[0];
   if (!isfinite(v)) v = INFINITY;  // the host search maps non-finite energies to +inf
   switch (phase) {
     case 0:
@@ -135,6 +135,11 @@ __global__ void golden_step_kernel(double* __restrict__ st, const double* __rest
   }
 }
 
+__global__ void golden_step_kernel(double* __restrict__ st, const double* __restrict__ f_new) {
+  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+  golden_step(st, f_new[0]);
+}
+
 // trial = x + alpha p with alpha from the state (skipped once the search is done)
 __global__ __launch_bounds__(256) void golden_trial_kernel(int n, const double* __restrict__ x,
                                                            const double* __restrict__ p,
@@ -146,7 +151,73 @@ __global__ __launch_bounds__(256) void golden_trial_kernel(int n, const double* 
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) trial[i] = x[i] + a * p[i];
 }
 
+// One point's bookkeeping in one launch: the sum of the energy's per-block partials, the step of the
+// state machine and the next trial point.  Every workgroup sums the partials and steps a copy of the
+// state itself (16 B x 240 to 3,062 of them from the cache); the state goes from one copy to the other,
+// so that no workgroup reads what another writes.  nb < 0: start a search instead.
+struct GoldenStart {
+  double lo, hi, tol;
+};
+__global__ __launch_bounds__(256) void golden_point_kernel(int n, const double* __restrict__ x,
+                                                           const double* __restrict__ p,
+                                                           const double* __restrict__ st_in,
+                                                           double* __restrict__ st_out,
+                                                           const double2* __restrict__ partial, int nb,
+                                                           GoldenStart start, double* __restrict__ trial) {
+  __shared__ double st[kGoldenLen];
+  const int tid = threadIdx.x;
+  if (nb < 0) {
+    if (tid < kGoldenLen)
+      st[tid] = tid == kLo || tid == kAlpha ? start.lo : (tid == kHi ? start.hi : (tid == kTol ? start.tol : 0.0));
+  } else {
+    if (tid < kGoldenLen) st[tid] = st_in[tid];
+    double s = 0.0, c = 0.0;
+    for (int i = tid; i < nb; i += 256) acc_merge(s, c, partial[i].x, partial[i].y);
+    block_reduce_pair<256>(s, c);  // (a barrier: the state is in LDS)
+    if (tid == 0) golden_step(st, s + c);
+  }
+  __syncthreads();
+  if (blockIdx.x == 0 && tid < kGoldenLen) st_out[tid] = st[tid];
+  if (st[kPhase] >= 7.0) return;
+  const double a = st[kAlpha];
+  for (int i = blockIdx.x * 256 + tid; i < n; i += gridDim.x * 256) trial[i] = x[i] + a * p[i];
+}
+
 }  // namespace
+
+extern "C" int fne_golden_search(fne_plan* plan, int32_t n, const double* x, const double* p, const double* dvals,
+                                 const double* f, double lo, double hi, double tol, int32_t points, int32_t resume,
+                                 double* state, double* trial, fne_stream_t stream) {
+  if (!plan || !x || !p || !state || !trial || points < 1 || n != plan->d.n_free || trial == x || trial == p) {
+    fne_set_error("fne_golden_search: invalid arguments");
+    return FNE_EINVAL;
+  }
+  if (resume && (points & 1)) {
+    fne_set_error("fne_golden_search: a search is resumed for an even number of points");
+    return FNE_EINVAL;
+  }
+  if (plan->d.n_total > 0 && !dvals) {
+    fne_set_error("Dirichlet values missing");
+    return FNE_EINVAL;
+  }
+  hipStream_t s = (hipStream_t)stream;
+  const dim3 grid(unsigned(std::max<int64_t>(1, std::min<int64_t>(512, (int64_t(n) + 255) / 256))));
+  const GoldenStart start{lo, hi, tol};
+  // the state moves between its two copies and ends in the first
+  int at = resume ? 0 : points & 1;
+  if (!resume)
+    hipLaunchKernelGGL(golden_point_kernel, grid, dim3(256), 0, s, n, x, p, state, state + at * kGoldenLen,
+                       plan->partials, -1, start, trial);
+  for (int k = 0; k < points; ++k, at ^= 1) {
+    int nb = 0;
+    const int rc = fne_energy_partials(plan, trial, dvals, f, &nb, s);
+    if (rc) return rc;
+    hipLaunchKernelGGL(golden_point_kernel, grid, dim3(256), 0, s, n, x, p, state + at * kGoldenLen,
+                       state + (at ^ 1) * kGoldenLen, plan->partials, nb, start, trial);
+  }
+  FNE_LAUNCH_CHECK();
+  return FNE_OK;
+}
 
 extern "C" int fne_golden_state_len(void) { return kGoldenLen; }
 

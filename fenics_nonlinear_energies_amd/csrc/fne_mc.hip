@@ -251,7 +251,7 @@ constexpr int kMcMatrix = NN * kMcNodeRow<NN>;
 // elements, Hessian alone 65 -> 39 us, gradient alone 11.8 -> 10.8; product with a direction, P4,
 // 32,000 elements 46 -> 22 us.
 template <int NN, int NS, typename HT, bool WE, bool WG, bool WH, bool HV>
-__global__ __launch_bounds__(kBlock, 4) void mc_elem_kernel(
+__global__ __launch_bounds__(kBlock, WH && sizeof(HT) == 8 && (WG || (NN == 15 && NS == 11)) ? 3 : 4) void mc_elem_kernel(
     fne_plan_desc d, McConst k, const double* __restrict__ x, const double* __restrict__ dvals,
     const double* __restrict__ f, const double* __restrict__ vin, double2* __restrict__ partial,
     double* __restrict__ eelem, double* __restrict__ gbuf, HT* __restrict__ hbuf, McBlocks B) {

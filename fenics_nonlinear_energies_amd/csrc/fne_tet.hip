@@ -12,6 +12,8 @@
 //                     alpha = 2 C1 - 2 D1 J (J-1),  beta = 2 D1 J (2J-1)
 #include "fne_common.h"
 
+#include <algorithm>
+
 namespace {
 
 struct TetElem {
@@ -709,7 +711,8 @@ int launch_tet_node_patches(fne_plan* plan, bool want_e, bool want_g, bool want_
 int fne_launch_tet(fne_plan* plan, FneOp op, const FneCall& c) {
   const fne_plan_desc& d = plan->d;
   if (op == kOpEnergy) {
-    const int nb = plan->n_partials;
+    // one element per thread, so that a small mesh is one pass of few blocks and few partial sums
+    const int nb = std::max(1, std::min(plan->n_partials, (d.n_elem + kBlock - 1) / kBlock));
     hipLaunchKernelGGL(tet_energy_kernel, dim3(nb), dim3(kBlock), 0, c.stream, d, c.x, c.dvals, c.f,
                        plan->partials);
     FNE_LAUNCH_CHECK();

@@ -15,6 +15,7 @@ import numpy as np
 import torch
 
 from . import native
+from .assembler import ReorderedElementAssemblerBase
 from .minimizers import newton
 from .repair import as_policy, primary_rung, solve_with_repair
 
@@ -33,19 +34,20 @@ NEWTON_DEFAULTS = {
 
 
 class DeviceGoldenSearch:
-    """Golden-section line search on the device (``fne_golden_trial`` / ``fne_energy`` /
-    ``fne_golden_step`` per point): the same points and comparisons as
-    ``minimizers.golden_section_search`` (``core/petsc/minimizers.py:14-64``), with one host
-    synchronisation per search instead of one per energy."""
+    """Golden-section line search on the device (``fne_golden_search``): the same points and
+    comparisons as ``minimizers.golden_section_search`` (``core/petsc/minimizers.py:14-64``), with
+    one host synchronisation per search instead of one per energy."""
 
     def __init__(self, assembler):
         self.asm = assembler
         dev = assembler.device
         n_state = int(native.lib().fne_golden_state_len())
-        self.state = torch.zeros(n_state, dtype=torch.float64, device=dev)
+        self.state = torch.zeros(2 * n_state, dtype=torch.float64, device=dev)
         self.trial = torch.empty(assembler.layout.n_free, dtype=torch.float64, device=dev)
         self.energy = torch.zeros(1, dtype=torch.float64, device=dev)
         self._init = torch.zeros(n_state, dtype=torch.float64)
+        # an assembler with an energy of its own evaluates it point by point
+        self._native = type(assembler).energy_device is ReorderedElementAssemblerBase.energy_device
         self.searches = 0
 
     def _point(self, xt: torch.Tensor, pt: torch.Tensor) -> None:
@@ -56,26 +58,38 @@ class DeviceGoldenSearch:
         self.asm.energy_device(self.trial, out=self.energy)
         native.check(lib.fne_golden_step(native.ptr(self.state), native.ptr(self.energy), sp), "fne_golden_step")
 
+    def _points(self, xt: torch.Tensor, pt: torch.Tensor, bracket: tuple, points: int, resume: bool) -> None:
+        lo, hi, tol = bracket
+        if self._native:
+            asm = self.asm
+            native.check(native.lib().fne_golden_search(
+                asm._plan, int(xt.numel()), native.ptr(xt), native.ptr(pt), native.ptr(asm.dvals),
+                native.ptr(asm._f_dev), lo, hi, tol, points, int(resume), native.ptr(self.state),
+                native.ptr(self.trial), native.stream_ptr()), "fne_golden_search")
+            return
+        if not resume:
+            init = self._init
+            init.zero_()
+            init[0], init[1], init[10], init[13] = lo, hi, lo, tol  # lo, hi, first point, tol
+            self.state[:init.numel()].copy_(init)
+        for _ in range(points):
+            self._point(xt, pt)
+
     def __call__(self, x_prev, p, lo: float, hi: float, tol: float):
         lo, hi, tol = float(lo), float(hi), float(tol)
         gamma = 0.5 + math.sqrt(5.0) / 2.0
-        init = self._init
-        init.zero_()
-        init[0], init[1], init[10], init[13] = lo, hi, lo, tol  # lo, hi, first point, tol
-        self.state.copy_(init)
         # 4 initial points, the shrink steps until hi - lo <= tol (+2 for rounding), the midpoint;
         # steps after the search has finished are no-ops
         n_loop = int(math.ceil(math.log(tol / (hi - lo)) / math.log(1.0 / gamma))) + 2 if hi - lo > tol else 0
         xt, pt = x_prev.t, p.t
-        for _ in range(4 + max(n_loop, 0) + 1):
-            self._point(xt, pt)
+        self._points(xt, pt, (lo, hi, tol), 4 + max(n_loop, 0) + 1, False)
         st = self.state.cpu().numpy()
         extra = 0
         while st[11] < 7.0:  # not finished (rounding made the bracket shrink more slowly)
             if extra >= 200:
                 raise RuntimeError("device golden-section search did not finish")
-            self._point(xt, pt)
-            extra += 1
+            self._points(xt, pt, (lo, hi, tol), 2, True)
+            extra += 2
             st = self.state.cpu().numpy()
         self.searches += 1
         return float(st[8]), float(st[9]), int(st[12])

@@ -119,6 +119,12 @@ _SIGNATURES = [
     ("fne_golden_trial", C.c_int, [C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]),
     ("fne_golden_step", C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p]),
     (
+        "fne_golden_search",
+        C.c_int,
+        [C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_double, C.c_double, C.c_double,
+         C.c_int32, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p],
+    ),
+    (
         "fne_aggregate_qr",
         C.c_int,
         [C.c_int32, C.c_int32, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p],

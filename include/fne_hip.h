@@ -246,6 +246,15 @@ int fne_golden_state_len(void);
 int fne_golden_trial(int32_t n, const double* x, const double* p, const double* state, double* trial,
                      fne_stream_t stream);
 int fne_golden_step(double* state, const double* f_new, fne_stream_t stream);
+/*
+ * `points` points of that search with the plan's energy, two launches each.  state: device array of
+ * 2 fne_golden_state_len() slots (two copies; the first holds the result as above), trial: n_free
+ * slots.  resume = 0 starts a search (state need not be initialised), resume = 1 goes on with one that
+ * is not finished, for an even number of points.  n must be n_free.
+ */
+int fne_golden_search(fne_plan* plan, int32_t n, const double* x, const double* p, const double* dvals,
+                      const double* f, double lo, double hi, double tol, int32_t points, int32_t resume,
+                      double* state, double* trial, fne_stream_t stream);
 
 /*
  * Tentative prolongator of the multigrid set-up: thin QR of every aggregate's rows of the

@@ -54,3 +54,47 @@ def test_newton_same_path_with_device_linesearch(require_gpu):
         asm.cleanup()
     assert res[True][0] == res[False][0]
     assert res[True][1] == pytest.approx(res[False][1], rel=1e-13)
+
+
+def _he_asm():
+    from fenics_nonlinear_energies_amd.problems.hyperelasticity import HEReorderedElementAssembler, build_beam_problem
+
+    p, adj, u0 = build_beam_problem(6, 2, 2)
+    asm = HEReorderedElementAssembler(p, None, adj)
+    return asm, np.asarray(u0)[asm.layout.perm], 1e-4
+
+
+def _mc_asm():
+    from fenics_nonlinear_energies_amd.problems.slope_stability import SlopeStabilityReorderedElementAssembler
+    from tests.test_oracle_mc import mc_params
+
+    p, adj = mc_params(h=4.0, degree=2, lam=1.2)
+    asm = SlopeStabilityReorderedElementAssembler(p, None, adj)
+    return asm, np.zeros(asm.layout.n_free), 1e-2
+
+
+def _p1_asm():
+    asm = _asm()
+    return asm, np.random.default_rng(1).random(asm.layout.n_free), 0.5
+
+
+@pytest.mark.parametrize("make", [_p1_asm, _he_asm, _mc_asm])
+def test_search_in_one_call_equals_point_by_point(require_gpu, make):
+    """fne_golden_search against fne_golden_trial / fne_energy / fne_golden_step per point, and resumed two points at a
+    time: the same energies up to the order of their sums, so the same points."""
+    asm, x0, amp = make()
+    x = asm.create_vec(x0)
+    d = asm.create_vec(amp * np.random.default_rng(3).standard_normal(x0.size))
+    one, each = DeviceGoldenSearch(asm), DeviceGoldenSearch(asm)
+    assert one._native
+    each._native = False
+    got, ref = one(x, d, -0.5, 2.0, 1e-4), each(x, d, -0.5, 2.0, 1e-4)
+    assert got[2] == ref[2]
+    assert abs(got[0] - ref[0]) <= 1e-12 and got[1] == pytest.approx(ref[1], rel=1e-13)
+    steps = DeviceGoldenSearch(asm)
+    steps._points(x.t, d.t, (-0.5, 2.0, 1e-4), 2, False)
+    for _ in range(40):
+        steps._points(x.t, d.t, (-0.5, 2.0, 1e-4), 2, True)
+    st = steps.state.cpu().numpy()
+    assert st[11] == 7.0 and (float(st[8]), float(st[9]), int(st[12])) == got
+    asm.cleanup()
