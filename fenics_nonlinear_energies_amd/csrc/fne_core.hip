@@ -7,12 +7,11 @@ namespace {
 thread_local std::string g_last_error;
 
 // Final deterministic reduction of the per-block (sum, compensation) partials.
-// One 1024-thread block; four independent loads in flight per thread, merged in index order.
-constexpr int kFinalizeThreads = 1024;
-__global__ __launch_bounds__(kFinalizeThreads) void finalize_pairs_kernel(const double2* __restrict__ partial,
-                                                                          int n, double* __restrict__ out) {
+// One block of T threads; four independent loads in flight per thread, merged in index order.
+template <int T>
+__global__ __launch_bounds__(T) void finalize_pairs_kernel(const double2* __restrict__ partial, int n,
+                                                           double* __restrict__ out) {
   double s = 0.0, c = 0.0;
-  constexpr int T = kFinalizeThreads;
   int i = threadIdx.x;
   for (; i + 3 * T < n; i += 4 * T) {
     const double2 a = partial[i], b = partial[i + T], e = partial[i + 2 * T], f = partial[i + 3 * T];
@@ -24,6 +23,14 @@ __global__ __launch_bounds__(kFinalizeThreads) void finalize_pairs_kernel(const 
   for (; i < n; i += T) acc_merge(s, c, partial[i].x, partial[i].y);
   block_reduce_pair<T>(s, c);
   if (threadIdx.x == 0) out[0] = s + c;
+}
+
+// 256 threads take up to 1,024 pairs in one pass of loads, and join in half the steps of 1,024 threads
+void launch_finalize(const double2* partial, int n, double* out, hipStream_t s) {
+  if (n <= 1024)
+    hipLaunchKernelGGL(finalize_pairs_kernel<256>, dim3(1), dim3(256), 0, s, partial, n, out);
+  else
+    hipLaunchKernelGGL(finalize_pairs_kernel<1024>, dim3(1), dim3(1024), 0, s, partial, n, out);
 }
 
 // y = A x with LPR lanes per row (LPR | 64), each lane taking groups of four entries
@@ -250,13 +257,26 @@ FneCall make_call(const double* x, const double* dvals, const double* f, hipStre
 
 void fne_set_error(const std::string& msg) { g_last_error = msg; }
 
+// Workgroups up to which an energy's launch adds its own partial sums up (EnergySum): the release of
+// each arrival writes its XCD's L2 back, some 70 ns one after the other, against 3 to 5 us for a
+// launch of finalize_pairs_kernel (10 workgroups of the 32x32 Ginzburg-Landau grid 10.6 -> 9.1 us,
+// energy alone 7.5 -> 4.6; 128 workgroups 7.6 -> 9.5).
+static bool energy_in_launch(int nblocks) {
+  constexpr int kEnergyInLaunch = 32;
+  return nblocks <= kEnergyInLaunch;
+}
+
+EnergySum fne_energy_sum(fne_plan* plan, int nblocks, double* out) {
+  return EnergySum{plan->partials, out && energy_in_launch(nblocks) ? out : nullptr, plan->done};
+}
+
 int fne_finalize_energy(fne_plan* plan, int nblocks, double* out, hipStream_t stream) {
+  if (out && energy_in_launch(nblocks)) return FNE_OK;
   if (!out) {  // fne_energy_partials: the caller adds the blocks up
     plan->energy_blocks = nblocks;
     return FNE_OK;
   }
-  hipLaunchKernelGGL(finalize_pairs_kernel, dim3(1), dim3(kFinalizeThreads), 0, stream, plan->partials, nblocks,
-                     out);
+  launch_finalize(plan->partials, nblocks, out, stream);
   FNE_LAUNCH_CHECK();
   return FNE_OK;
 }
@@ -300,7 +320,10 @@ int fne_plan_create(const fne_plan_desc* desc, fne_plan** out) {
     if (kEnergyBlocks > need) need = kEnergyBlocks;
     p->n_partials = int(need);
   }
-  if (hipMalloc(&p->partials, sizeof(double2) * p->n_partials) != hipSuccess) {
+  if (hipMalloc(&p->partials, sizeof(double2) * p->n_partials) != hipSuccess ||
+      hipMalloc(&p->done, sizeof(unsigned)) != hipSuccess || hipMemset(p->done, 0, sizeof(unsigned)) != hipSuccess) {
+    if (p->partials) (void)hipFree(p->partials);
+    if (p->done) (void)hipFree(p->done);
     delete p;
     fne_set_error("hipMalloc of reduction scratch failed");
     return FNE_ENOMEM;
@@ -313,6 +336,7 @@ int fne_plan_create(const fne_plan_desc* desc, fne_plan** out) {
     if (hipMalloc(&p->mc_h, hbytes) != hipSuccess || hipMalloc(&p->mc_g, gbytes) != hipSuccess) {
       if (p->mc_h) (void)hipFree(p->mc_h);
       (void)hipFree(p->partials);
+      (void)hipFree(p->done);
       delete p;
       fne_set_error("hipMalloc of the element scratch failed");
       return FNE_ENOMEM;
@@ -325,6 +349,7 @@ int fne_plan_create(const fne_plan_desc* desc, fne_plan** out) {
 int fne_plan_destroy(fne_plan* plan) {
   if (!plan) return FNE_OK;
   if (plan->partials) (void)hipFree(plan->partials);
+  if (plan->done) (void)hipFree(plan->done);
   if (plan->mc_h) (void)hipFree(plan->mc_h);
   if (plan->mc_g) (void)hipFree(plan->mc_g);
   if (plan->np.storage) (void)hipFree(plan->np.storage);
@@ -466,8 +491,7 @@ int fne_dot(int64_t n, const double* a, const double* b, double* out, void* work
   if (nb < 1) nb = 1;
   hipLaunchKernelGGL(dot_kernel, dim3(nb), dim3(kBlock), 0, (hipStream_t)stream, n, a, b, work);
   FNE_LAUNCH_CHECK();
-  hipLaunchKernelGGL(finalize_pairs_kernel, dim3(1), dim3(kFinalizeThreads), 0, (hipStream_t)stream, work, nb,
-                     out);
+  launch_finalize(work, nb, out, (hipStream_t)stream);
   FNE_LAUNCH_CHECK();
   return FNE_OK;
 }

@@ -253,7 +253,7 @@ constexpr int kMcMatrix = NN * kMcNodeRow<NN>;
 template <int NN, int NS, typename HT, bool WE, bool WG, bool WH, bool HV>
 __global__ __launch_bounds__(kBlock, WH && sizeof(HT) == 8 && (WG || (NN == 15 && NS == 11)) ? 3 : 4) void mc_elem_kernel(
     fne_plan_desc d, McConst k, const double* __restrict__ x, const double* __restrict__ dvals,
-    const double* __restrict__ f, const double* __restrict__ vin, double2* __restrict__ partial,
+    const double* __restrict__ f, const double* __restrict__ vin, EnergySum energy,
     double* __restrict__ eelem, double* __restrict__ gbuf, HT* __restrict__ hbuf, McBlocks B) {
   constexpr int NL = 2 * NN;
   constexpr bool kOneTile = NL <= 16;
@@ -494,8 +494,7 @@ __global__ __launch_bounds__(kBlock, WH && sizeof(HT) == 8 && (WG || (NN == 15 &
       const int all = B.all * kBlock;
       for (int i = block * kBlock + threadIdx.x; i < d.n_free; i += all) acc_add(es, ec, -(f[i] * x[i]));
     }
-    block_reduce_pair(es, ec);
-    if (threadIdx.x == 0) partial[block] = make_double2(es, ec);
+    block_energy(energy, block, es, ec);
   }
 }
 
@@ -799,11 +798,12 @@ int launch_mc(fne_plan* plan, FneOp op, const FneCall& c) {
   const bool want_e = op == kOpEnergy || (op == kOpFused && c.out);
   const bool want_g = op == kOpGradient || ((op == kOpHessian || op == kOpFused) && c.g);
   const bool want_h = op == kOpHessian || op == kOpFused;
+  const EnergySum energy = fne_energy_sum(plan, nb, c.out);
   double* gb = plan->mc_g;
   void* hb = plan->mc_h;
 #define MC_ELEM_NS(NS, HT, E, G, H, FV, EV)                                                                      \
   hipLaunchKernelGGL((mc_elem_kernel<NN, NS, HT, E, G, H, false>), dim3(nb), dim3(kBlock), 0, c.stream, d, k, c.x, \
-                     c.dvals, FV, (const double*)nullptr, plan->partials, EV, gb, (HT*)hb, B)
+                     c.dvals, FV, (const double*)nullptr, energy, EV, gb, (HT*)hb, B)
   // NS: products of four K rows that cover 2 n_q
 #define MC_ELEM(HT, E, G, H, FV, EV)            \
   do {                                          \
@@ -971,7 +971,7 @@ int launch_mc_aux(fne_plan* plan, const double* x, const double* dvals, const do
     const double* none = nullptr;
 #define MC_HVP(NS)                                                                                                 \
   hipLaunchKernelGGL((mc_elem_kernel<NN, NS, double, false, true, false, true>), grid, dim3(kBlock), 0, stream, d, k, \
-                     x, dvals, none, v, plan->partials, (double*)nullptr, plan->mc_g, (double*)nullptr, B)
+                     x, dvals, none, v, EnergySum{}, (double*)nullptr, plan->mc_g, (double*)nullptr, B)
     if (d.nq <= 20)
       MC_HVP(10);
     else

@@ -17,6 +17,8 @@
 //               H_ab = vol [ eps K_ab + sum_q w_q (3 u_q^2 - 1) ip[a][q] ip[b][q] ]
 #include "fne_common.h"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int kMaxQ = 16;
@@ -294,7 +296,7 @@ template <int FAM>
 __global__ __launch_bounds__(kBlock) void p1_energy_kernel(fne_plan_desc d, const double* __restrict__ x,
                                                            const double* __restrict__ dvals,
                                                            const double* __restrict__ f,
-                                                           double2* __restrict__ partial) {
+                                                           EnergySum energy) {
   // block b covers elements [b*2B, (b+1)*2B) and free DOFs [b*2B, (b+1)*2B) of the load term
   double s = 0.0, c = 0.0;
   const double* prm = d.param;
@@ -317,8 +319,7 @@ __global__ __launch_bounds__(kBlock) void p1_energy_kernel(fne_plan_desc d, cons
     if (e1 < d.n_free) acc_add(s, c, -(f[e1] * x[e1]));
     if (e2 < d.n_free) acc_add(s, c, -(f[e2] * x[e2]));
   }
-  block_reduce_pair(s, c);
-  if (threadIdx.x == 0) partial[blockIdx.x] = make_double2(s, c);
+  block_energy(energy, blockIdx.x, s, c);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -335,7 +336,7 @@ __global__ __launch_bounds__(kBlock) void p1_color_kernel(fne_plan_desc d, const
                                                           const double* __restrict__ dvals,
                                                           const double* __restrict__ f,
                                                           double* __restrict__ g, HT* __restrict__ vals,
-                                                          double2* __restrict__ partial) {
+                                                          EnergySum energy) {
   extern __shared__ double smem[];
   const int p = xcd_remap(blockIdx.x, gridDim.x);
   const int tid = threadIdx.x;
@@ -433,8 +434,7 @@ __global__ __launch_bounds__(kBlock) void p1_color_kernel(fne_plan_desc d, const
   if (WANT_G)
     for (int i = tid; i < nrows; i += B) g[r0 + i] = f ? sG[i] - f[r0 + i] : sG[i];
   if (WANT_E) {
-    block_reduce_pair(es, ec);
-    if (tid == 0) partial[p] = make_double2(es, ec);
+    block_energy<kBlock>(energy, p, es, ec);
   }
 }
 
@@ -451,12 +451,15 @@ __global__ __launch_bounds__(kBlock) void p1_color_kernel(fne_plan_desc d, const
 // ---------------------------------------------------------------------------------------------
 constexpr int kStagedPrefetch = 8;
 
-template <int FAM, typename HT, bool WANT_E, bool WANT_G, bool WANT_H, bool NG>
+// ES: EnergySum on grids so small that the launch adds its partial sums up itself, else double2*: the
+// code for it costs the 1024x1024 Ginzburg-Landau assembly a wavefront per SIMD (80 -> 81 registers,
+// 52 -> 55 us)
+template <int FAM, typename HT, bool WANT_E, bool WANT_G, bool WANT_H, bool NG, typename ES>
 __global__ __launch_bounds__(kBlock) void p1_staged_kernel(fne_plan_desc d, const double* __restrict__ x,
                                                            const double* __restrict__ dvals,
                                                            const double* __restrict__ f,
                                                            double* __restrict__ g, HT* __restrict__ vals,
-                                                           double2* __restrict__ partial) {
+                                                           ES energy) {
   extern __shared__ double smem[];
   const int p = xcd_remap(blockIdx.x, gridDim.x);
   const int tid = threadIdx.x;
@@ -551,8 +554,12 @@ __global__ __launch_bounds__(kBlock) void p1_staged_kernel(fne_plan_desc d, cons
     }
   }
   if (WANT_E) {
-    block_reduce_pair(es, ec);
-    if (tid == 0) partial[p] = make_double2(es, ec);
+    if constexpr (std::is_same<ES, EnergySum>::value) {
+      block_energy(energy, p, es, ec);
+    } else {
+      block_reduce_pair(es, ec);
+      if (tid == 0) energy[p] = make_double2(es, ec);
+    }
   }
 }
 
@@ -693,7 +700,7 @@ int launch_p1(fne_plan* plan, FneOp op, const FneCall& c) {
       return FNE_EINVAL;
     }
     hipLaunchKernelGGL(p1_energy_kernel<FAM>, dim3(nb), dim3(kBlock), 0, c.stream, d, c.x, c.dvals, c.f,
-                       plan->partials);
+                       fne_energy_sum(plan, nb, c.out));
     FNE_LAUNCH_CHECK();
     return fne_finalize_energy(plan, nb, c.out, c.stream);
   }
@@ -774,10 +781,21 @@ int launch_p1(fne_plan* plan, FneOp op, const FneCall& c) {
       return FNE_EINVAL;
     }
     const dim3 grid(d.n_patch), block(kBlock);
-    double2* part = plan->partials;
-#define ST_GO(HT, E, G, H, NG)                                                                          \
-  hipLaunchKernelGGL((p1_staged_kernel<FAM, HT, E, G, H, NG>), grid, block, shm, c.stream, d, c.x, c.dvals, c.f, \
-                     c.g, (HT*)c.vals, part)
+    const EnergySum part = fne_energy_sum(plan, d.n_patch, c.out);
+#define ST_KERNEL(HT, E, G, H, NG, ES, PART)                                                             \
+  hipLaunchKernelGGL((p1_staged_kernel<FAM, HT, E, G, H, NG, ES>), grid, block, shm, c.stream, d, c.x, c.dvals, c.f, \
+                     c.g, (HT*)c.vals, PART)
+#define ST_GO(HT, E, G, H, NG)                              \
+  do {                                                      \
+    if constexpr (E) {                                      \
+      if (part.out)                                         \
+        ST_KERNEL(HT, E, G, H, NG, EnergySum, part);        \
+      else                                                  \
+        ST_KERNEL(HT, E, G, H, NG, double2*, part.partial); \
+    } else {                                                \
+      ST_KERNEL(HT, E, G, H, NG, double2*, part.partial);   \
+    }                                                       \
+  } while (0)
 #define ST_MR(HT, E, G, H) \
   do {                     \
     if (ng)                \
@@ -800,6 +818,7 @@ int launch_p1(fne_plan* plan, FneOp op, const FneCall& c) {
     }
 #undef ST_MR
 #undef ST_GO
+#undef ST_KERNEL
     FNE_LAUNCH_CHECK();
     if (want_e) return fne_finalize_energy(plan, d.n_patch, c.out, c.stream);
     return FNE_OK;
@@ -831,7 +850,7 @@ int launch_p1(fne_plan* plan, FneOp op, const FneCall& c) {
     return FNE_EINVAL;
   }
   const dim3 grid(d.n_patch), block(kBlock);
-  double2* part = plan->partials;
+  const EnergySum part = fne_energy_sum(plan, d.n_patch, c.out);
 #define P1_GO(HT, E, G, H, EP)                                                                          \
   hipLaunchKernelGGL((p1_color_kernel<FAM, HT, E, G, H, EP>), grid, block, shm, c.stream, d, c.x, c.dvals, c.f, \
                      c.g, (HT*)c.vals, part)

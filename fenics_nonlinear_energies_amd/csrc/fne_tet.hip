@@ -113,7 +113,7 @@ constexpr int kTetStage = 39;
 __global__ __launch_bounds__(kBlock) void tet_energy_kernel(fne_plan_desc d, const double* __restrict__ x,
                                                             const double* __restrict__ dvals,
                                                             const double* __restrict__ f,
-                                                            double2* __restrict__ partial) {
+                                                            EnergySum energy) {
   double s = 0.0, c = 0.0;
   const bool absdet = (d.flags & FNE_FLAG_ABS_DET) != 0;
   const int stride = gridDim.x * blockDim.x;
@@ -127,8 +127,7 @@ __global__ __launch_bounds__(kBlock) void tet_energy_kernel(fne_plan_desc d, con
   if (f) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < d.n_free; i += stride) acc_add(s, c, -(f[i] * x[i]));
   }
-  block_reduce_pair(s, c);
-  if (threadIdx.x == 0) partial[blockIdx.x] = make_double2(s, c);
+  block_energy(energy, blockIdx.x, s, c);
 }
 
 // Patch kernel.  Rows come in node triples; thread t of the workgroup owns scalar row r0+t.
@@ -442,7 +441,7 @@ __device__ __forceinline__ void np_store3(HT* dst, double a, double b, double c)
 template <typename HT, bool WANT_E, bool WANT_G, bool WANT_H>
 __global__ __launch_bounds__(kNodePatchThreads, 2) void tet_node_patch_kernel(
     fne_plan_desc d, FneNodePatches P, const double* __restrict__ x, const double* __restrict__ dvals,
-    const double* __restrict__ f, double* __restrict__ g, HT* __restrict__ vals, double2* __restrict__ partial) {
+    const double* __restrict__ f, double* __restrict__ g, HT* __restrict__ vals, EnergySum energy) {
   constexpr int kThreads = kNodePatchThreads;
   __shared__ double sS[(kNodePatchElems + 1) * (WANT_H ? kNpStride : kNpGStride)];
   __shared__ uint2 sDiag[kNodePatchNodes * 8];
@@ -676,8 +675,7 @@ __global__ __launch_bounds__(kNodePatchThreads, 2) void tet_node_patch_kernel(
     }
   }
   if (WANT_E) {
-    block_reduce_pair<kNodePatchThreads>(es, ec);
-    if (tid == 0) partial[p] = make_double2(es, ec);
+    block_energy<kNodePatchThreads>(energy, p, es, ec);
   }
 }
 
@@ -686,7 +684,7 @@ int launch_tet_node_patches(fne_plan* plan, bool want_e, bool want_g, bool want_
   const dim3 grid(P.n_patch), block(kNodePatchThreads);
 #define NP_GO(HT, E, G, H)                                                                                    \
   hipLaunchKernelGGL((tet_node_patch_kernel<HT, E, G, H>), grid, block, 0, c.stream, plan->d, P, c.x, c.dvals, c.f, \
-                     c.g, (HT*)c.vals, plan->partials)
+                     c.g, (HT*)c.vals, fne_energy_sum(plan, P.n_patch, c.out))
   if (!want_h) {
     NP_GO(double, false, true, false);
   } else if (c.precision == FNE_FP32) {
@@ -714,7 +712,7 @@ int fne_launch_tet(fne_plan* plan, FneOp op, const FneCall& c) {
     // one element per thread, so that a small mesh is one pass of few blocks and few partial sums
     const int nb = std::max(1, std::min(plan->n_partials, (d.n_elem + kBlock - 1) / kBlock));
     hipLaunchKernelGGL(tet_energy_kernel, dim3(nb), dim3(kBlock), 0, c.stream, d, c.x, c.dvals, c.f,
-                       plan->partials);
+                       fne_energy_sum(plan, nb, c.out));
     FNE_LAUNCH_CHECK();
     return fne_finalize_energy(plan, nb, c.out, c.stream);
   }

@@ -219,3 +219,25 @@ def test_fused_energy_reduction_is_exact_and_reproducible_over_many_calls(requir
     assert abs(e[0] - e_sep) <= 1e-14 * abs(e_sep)
     assert torch.equal(h0, asm.A.data) and torch.equal(g0, g.t)
     asm.cleanup()
+
+
+@pytest.mark.parametrize("amode", ["patch", "staged"])
+@pytest.mark.parametrize("n", [3, 16, 56, 60, 64, 96, 128])
+def test_energy_summed_by_its_own_launch(require_gpu, n, amode):
+    """Small grids add their partial sums up in the energy's launch, larger ones in one of their own (the line
+    lies at 32 workgroups: 16 to 128 cells around it for both energies): the oracle's energy from
+    the energy and the fused call in turn, the same bits every time."""
+    p, adj = build_gl_problem(n)[:2]
+    asm = GLReorderedElementAssembler(p, None, adj, assembly_mode=amode)
+    u = np.random.default_rng(n).uniform(-1, 1, p["freedofs"].size)
+    ref = assembly.assemble("gl", p, u)["e"]
+    x = asm.create_vec(u[asm.layout.perm])
+    g = x.duplicate()
+    seen = set()
+    for _ in range(20):
+        e = float(asm.energy_device(x.t).item())
+        f = float(asm.energy_grad_hessian_device(x.t, g.t).item())
+        assert abs(e - ref) <= 1e-13 * max(1.0, abs(ref)) and abs(f - ref) <= 1e-13 * max(1.0, abs(ref))
+        seen.add((e, f))
+    assert len(seen) == 1
+    asm.cleanup()
