@@ -21,7 +21,30 @@ __global__ __launch_bounds__(T) void finalize_pairs_kernel(const double2* __rest
     acc_merge(s, c, f.x, f.y);
   }
   for (; i < n; i += T) acc_merge(s, c, partial[i].x, partial[i].y);
-  block_reduce_pair<T>(s, c);
+  if constexpr (T == 256) {
+    block_reduce_pair<T>(s, c);
+  } else {  // sixteen wavefronts: a second tree instead of fifteen additions in a row
+    __shared__ double sh_s[T / 64], sh_c[T / 64];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      const double s2 = __shfl_xor(s, off, 64), c2 = __shfl_xor(c, off, 64);
+      acc_merge(s, c, s2, c2);
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (lane == 0) {
+      sh_s[wave] = s;
+      sh_c[wave] = c;
+    }
+    __syncthreads();
+    if (wave > 0) return;
+    s = sh_s[lane & (T / 64 - 1)];
+    c = sh_c[lane & (T / 64 - 1)];
+#pragma unroll
+    for (int off = T / 128; off > 0; off >>= 1) {
+      const double s2 = __shfl_xor(s, off, 64), c2 = __shfl_xor(c, off, 64);
+      acc_merge(s, c, s2, c2);
+    }
+  }
   if (threadIdx.x == 0) out[0] = s + c;
 }
 
