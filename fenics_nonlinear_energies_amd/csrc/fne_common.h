@@ -77,7 +77,7 @@ struct FneRowUnits {
 struct fne_plan {
   fne_plan_desc d;
   double2* partials = nullptr;  // per-block (sum, compensation) pairs for energy reductions
-  unsigned* done = nullptr;  // arrival counter of EnergySum
+  unsigned* done = nullptr;  // arrival counters of EnergySum: energies alone, energies of fused calls
   int energy_blocks = 0;  // set by fne_energy_partials
   int n_partials = 0;
   int device = 0;
@@ -151,7 +151,8 @@ __device__ __forceinline__ void block_reduce_pair(double& s, double& c) {
 // the last workgroup to arrive also adds the pairs up, in their order and so the same whichever it
 // is, instead of a launch of its own (kEnergyInLaunch).  The pairs travel through
 // agent-scope atomics: the release and acquire of the arrival counter order them between the XCDs.
-// done is zero between launches; the last workgroup leaves it so.
+// done counts up to the launch's workgroups and wraps to zero, so that it is zero whenever as many
+// launches have ended as begun, whatever else ran beside them; a plan has one per launch size.
 struct EnergySum {
   double2* partial;
   double* out;
@@ -171,7 +172,7 @@ __device__ __forceinline__ void block_energy(const EnergySum& E, int slot, doubl
   if (threadIdx.x == 0) {
     __hip_atomic_store(pairs + 2 * slot, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(pairs + 2 * slot + 1, c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    last = __hip_atomic_fetch_add(E.done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+    last = __builtin_amdgcn_atomic_inc32(E.done, gridDim.x - 1, __ATOMIC_ACQ_REL, "agent") == gridDim.x - 1;
   }
   __syncthreads();
   if (!last) return;
@@ -180,10 +181,7 @@ __device__ __forceinline__ void block_energy(const EnergySum& E, int slot, doubl
     acc_merge(s, c, __hip_atomic_load(pairs + 2 * i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
               __hip_atomic_load(pairs + 2 * i + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
   block_reduce_pair<NT>(s, c);
-  if (threadIdx.x == 0) {
-    E.out[0] = s + c;
-    __hip_atomic_store(E.done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
+  if (threadIdx.x == 0) E.out[0] = s + c;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -412,7 +410,7 @@ int fne_launch_tet(fne_plan* plan, FneOp op, const FneCall& c);
 int fne_launch_mc(fne_plan* plan, FneOp op, const FneCall& c);
 // (nothing to do where fne_energy_sum had the energy's own launch do it)
 int fne_finalize_energy(fne_plan* plan, int nblocks, double* out, hipStream_t stream);
-EnergySum fne_energy_sum(fne_plan* plan, int nblocks, double* out);
+EnergySum fne_energy_sum(fne_plan* plan, FneOp op, int nblocks, double* out);
 // the energy's per-block (sum, compensation) pairs in plan->partials, without their sum
 int fne_energy_partials(fne_plan* plan, const double* x, const double* dvals, const double* f, int* nblocks,
                         hipStream_t stream);

@@ -289,8 +289,9 @@ static bool energy_in_launch(int nblocks) {
   return nblocks <= kEnergyInLaunch;
 }
 
-EnergySum fne_energy_sum(fne_plan* plan, int nblocks, double* out) {
-  return EnergySum{plan->partials, out && energy_in_launch(nblocks) ? out : nullptr, plan->done};
+EnergySum fne_energy_sum(fne_plan* plan, FneOp op, int nblocks, double* out) {
+  return EnergySum{plan->partials, out && energy_in_launch(nblocks) ? out : nullptr,
+                   plan->done + (op == kOpEnergy ? 0 : 1)};
 }
 
 int fne_finalize_energy(fne_plan* plan, int nblocks, double* out, hipStream_t stream) {
@@ -344,7 +345,8 @@ int fne_plan_create(const fne_plan_desc* desc, fne_plan** out) {
     p->n_partials = int(need);
   }
   if (hipMalloc(&p->partials, sizeof(double2) * p->n_partials) != hipSuccess ||
-      hipMalloc(&p->done, sizeof(unsigned)) != hipSuccess || hipMemset(p->done, 0, sizeof(unsigned)) != hipSuccess) {
+      hipMalloc(&p->done, 2 * sizeof(unsigned)) != hipSuccess ||
+      hipMemset(p->done, 0, 2 * sizeof(unsigned)) != hipSuccess) {
     if (p->partials) (void)hipFree(p->partials);
     if (p->done) (void)hipFree(p->done);
     delete p;

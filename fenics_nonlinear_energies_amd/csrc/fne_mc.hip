@@ -798,7 +798,7 @@ int launch_mc(fne_plan* plan, FneOp op, const FneCall& c) {
   const bool want_e = op == kOpEnergy || (op == kOpFused && c.out);
   const bool want_g = op == kOpGradient || ((op == kOpHessian || op == kOpFused) && c.g);
   const bool want_h = op == kOpHessian || op == kOpFused;
-  const EnergySum energy = fne_energy_sum(plan, nb, c.out);
+  const EnergySum energy = fne_energy_sum(plan, op, nb, c.out);
   double* gb = plan->mc_g;
   void* hb = plan->mc_h;
 #define MC_ELEM_NS(NS, HT, E, G, H, FV, EV)                                                                      \

@@ -700,7 +700,7 @@ int launch_p1(fne_plan* plan, FneOp op, const FneCall& c) {
       return FNE_EINVAL;
     }
     hipLaunchKernelGGL(p1_energy_kernel<FAM>, dim3(nb), dim3(kBlock), 0, c.stream, d, c.x, c.dvals, c.f,
-                       fne_energy_sum(plan, nb, c.out));
+                       fne_energy_sum(plan, op, nb, c.out));
     FNE_LAUNCH_CHECK();
     return fne_finalize_energy(plan, nb, c.out, c.stream);
   }
@@ -781,7 +781,7 @@ int launch_p1(fne_plan* plan, FneOp op, const FneCall& c) {
       return FNE_EINVAL;
     }
     const dim3 grid(d.n_patch), block(kBlock);
-    const EnergySum part = fne_energy_sum(plan, d.n_patch, c.out);
+    const EnergySum part = fne_energy_sum(plan, op, d.n_patch, c.out);
 #define ST_KERNEL(HT, E, G, H, NG, ES, PART)                                                             \
   hipLaunchKernelGGL((p1_staged_kernel<FAM, HT, E, G, H, NG, ES>), grid, block, shm, c.stream, d, c.x, c.dvals, c.f, \
                      c.g, (HT*)c.vals, PART)
@@ -850,7 +850,7 @@ int launch_p1(fne_plan* plan, FneOp op, const FneCall& c) {
     return FNE_EINVAL;
   }
   const dim3 grid(d.n_patch), block(kBlock);
-  const EnergySum part = fne_energy_sum(plan, d.n_patch, c.out);
+  const EnergySum part = fne_energy_sum(plan, op, d.n_patch, c.out);
 #define P1_GO(HT, E, G, H, EP)                                                                          \
   hipLaunchKernelGGL((p1_color_kernel<FAM, HT, E, G, H, EP>), grid, block, shm, c.stream, d, c.x, c.dvals, c.f, \
                      c.g, (HT*)c.vals, part)

@@ -684,7 +684,7 @@ int launch_tet_node_patches(fne_plan* plan, bool want_e, bool want_g, bool want_
   const dim3 grid(P.n_patch), block(kNodePatchThreads);
 #define NP_GO(HT, E, G, H)                                                                                    \
   hipLaunchKernelGGL((tet_node_patch_kernel<HT, E, G, H>), grid, block, 0, c.stream, plan->d, P, c.x, c.dvals, c.f, \
-                     c.g, (HT*)c.vals, fne_energy_sum(plan, P.n_patch, c.out))
+                     c.g, (HT*)c.vals, fne_energy_sum(plan, kOpFused, P.n_patch, c.out))
   if (!want_h) {
     NP_GO(double, false, true, false);
   } else if (c.precision == FNE_FP32) {
@@ -712,7 +712,7 @@ int fne_launch_tet(fne_plan* plan, FneOp op, const FneCall& c) {
     // one element per thread, so that a small mesh is one pass of few blocks and few partial sums
     const int nb = std::max(1, std::min(plan->n_partials, (d.n_elem + kBlock - 1) / kBlock));
     hipLaunchKernelGGL(tet_energy_kernel, dim3(nb), dim3(kBlock), 0, c.stream, d, c.x, c.dvals, c.f,
-                       fne_energy_sum(plan, nb, c.out));
+                       fne_energy_sum(plan, kOpEnergy, nb, c.out));
     FNE_LAUNCH_CHECK();
     return fne_finalize_energy(plan, nb, c.out, c.stream);
   }
