@@ -227,14 +227,21 @@ __global__ __launch_bounds__(256) void symmetrise_kernel(int nnz, const double* 
 }
 
 // ---------------------------------------------------------------------------------------------
-// Dense inverse of a symmetric positive definite matrix by block Gauss-Jordan without pivoting: for
-// every block column K, with D = A_KK^-1, A_KK <- D, A_KJ <- D A_KJ, A_IK <- -A_IK D and
-// A_IJ <- A_IJ - A_IK D A_KJ.  One launch per block column from one copy of the matrix to the other, a
-// workgroup per 32x32 tile; each inverts A_KK for itself in LDS (32 pivots, the pivots of an LDL^T
-// factorisation, so the matrix is positive definite exactly when all are positive), which is
-// cheaper than a launch of its own.  Products by v_mfma 16x16x4 in FP64, a quadrant per wavefront.
-// 286 unknowns: nine launches, 137 us (bound by the 32 pivots, one after the other); the library's
-// factorisation and inverse took 870 us.
+// Dense inverse of a symmetric positive definite matrix by its Cholesky factor: A = L L^T,
+// F = L^-1, A^-1 = F^T F, in 32x32 tiles.  One launch per block column K, a workgroup per tile of the
+// lower triangle from row K down.  Each factors A_KK for itself in LDS (32 pivots, one after the other,
+// which is cheaper than a launch of its own) and keeps T = L_KK^-1; then, with L_IK = A_IK T^T,
+//   row K:     F_KJ = T M_KJ (J < K), F_KK = T
+//   rows I>K:  M_IJ -= L_IK (T M_KJ) (J < K), M_IK = -L_IK T, A_IJ -= L_IK L_JK^T (J > K)
+// where M is the part of L^-1 that is still being eliminated.  A_IJ lies in the lower tiles and M_IJ in
+// the tiles above the diagonal, so nothing that a workgroup reads is written in the same launch.
+// Only L_KK is inverted explicitly, whose condition is the square root of A_KK's: the inverse is as
+// accurate as LAPACK's potrf and potri (block Gauss-Jordan with explicit inverses of the A_KK themselves
+// loses 1e5 of that at condition 1e8 and 33 unknowns).  The pivots are those of an LDL^T factorisation,
+// all positive exactly when the matrix is positive definite.  Products by v_mfma 16x16x4 in FP64, a
+// quadrant per wavefront.  Bound by the 32 pivots of each launch, one after the other.  Call after call,
+// 286 unknowns 152 us, 1,200 unknowns 853 (Gauss-Jordan on the whole square 146 and 1,417, the library's
+// factorisation and inverse 993 and 4,230).
 // ---------------------------------------------------------------------------------------------
 constexpr int kTile = 32, kTs = kTile + 1;  // LDS row stride
 typedef double d4 __attribute__((ext_vector_type(4)));
@@ -252,55 +259,61 @@ __global__ __launch_bounds__(256) void spd_rows_kernel(int n, int npad, const in
   if (row == 0 && threadIdx.x == 0) status[0] = 0.0;
 }
 
-// out = (a + a^T) / 2; out has ld_out columns and n rows
-__global__ __launch_bounds__(256) void spd_symmetrise_kernel(int n, int npad, const double* __restrict__ a,
-                                                             int ld_out, double* __restrict__ out) {
+// out = (a + a^T) / 2
+__global__ __launch_bounds__(256) void spd_symmetrise_kernel(int npad, const double* __restrict__ a,
+                                                             double* __restrict__ out) {
   __shared__ double t[kTile][kTs];
   const int bi = blockIdx.y * kTile, bj = blockIdx.x * kTile, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   for (int i = ty; i < kTile; i += 8) t[i][tx] = a[size_t(bj + i) * npad + bi + tx];
   __syncthreads();
   for (int i = ty; i < kTile; i += 8)
-    if (bi + i < n && bj + tx < n)
-      out[size_t(bi + i) * ld_out + bj + tx] = 0.5 * (a[size_t(bi + i) * npad + bj + tx] + t[tx][i]);
+    out[size_t(bi + i) * npad + bj + tx] = 0.5 * (a[size_t(bi + i) * npad + bj + tx] + t[tx][i]);
 }
 
-// the wavefront's 16x16 quadrant of X Y (32x32 in LDS, row stride kTs)
+// the wavefront's 16x16 quadrant of c + X Y (32x32 in LDS, row stride kTs), TX, TY: with X^T, Y^T
+template <bool TX, bool TY>
 __device__ __forceinline__ d4 tile_product(const double* X, const double* Y, int qi, int qj, int lane, d4 c) {
   const int r = lane & 15, k = lane >> 4;
 #pragma unroll
-  for (int s = 0; s < kTile / 4; ++s)
-    c = __builtin_amdgcn_mfma_f64_16x16x4f64(X[(qi + r) * kTs + 4 * s + k], Y[(4 * s + k) * kTs + qj + r], c, 0, 0, 0);
+  for (int s = 0; s < kTile / 4; ++s) {
+    const int m = 4 * s + k;
+    c = __builtin_amdgcn_mfma_f64_16x16x4f64(TX ? X[m * kTs + qi + r] : X[(qi + r) * kTs + m],
+                                             TY ? Y[(qj + r) * kTs + m] : Y[m * kTs + qj + r], c, 0, 0, 0);
+  }
   return c;
 }
 
-__global__ __launch_bounds__(256) void spd_step_kernel(int npad, int K, const double* __restrict__ a,
-                                                       double* __restrict__ b, double* __restrict__ status) {
-  __shared__ double sD[kTile * kTs], sL[kTile * kTs], sR[kTile * kTs];
+__global__ __launch_bounds__(256) void spd_step_kernel(int npad, int K, double* __restrict__ a,
+                                                       double* __restrict__ f, double* __restrict__ status) {
+  __shared__ double sT[kTile * kTs], sL[kTile * kTs], sR[kTile * kTs];
   __shared__ double s_col[2][kTile], s_row[2][kTile];
   const int tid = threadIdx.x, tx = tid & 31, ty = tid >> 5;
-  const int I = blockIdx.y, J = blockIdx.x;
-  const double* akk = a + (size_t(K) * npad + K) * kTile;
-  const double* aik = a + (size_t(I) * npad + K) * kTile;
-  const double* akj = a + (size_t(K) * npad + J) * kTile;
-  const double* aij = a + (size_t(I) * npad + J) * kTile;
-  double* bij = b + (size_t(I) * npad + J) * kTile;
+  const int I = K + blockIdx.y, J = blockIdx.x;
+  if (J > I) return;  // the whole workgroup
+  auto tile = [&](double* m, int i, int j) { return m + (size_t(i) * npad + j) * kTile; };
+  const double* akk = tile(a, K, K);
+  const double* left = tile(a, I, K);
+  const double* right = tile(a, J, K);  // M_KJ above the diagonal, A_JK below
+  double* out = I == K ? tile(f, K, J) : (J > K ? tile(a, I, J) : tile(a, J, I));  // F_KJ, A_IJ, M_IJ
   // A_KK in registers, four rows per thread: rows ty + 8 i, column tx
-  double m[4];
+  double m[4], d[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const size_t at = size_t(ty + 8 * i) * npad + tx;
     m[i] = akk[at];
-    if (I != K) sL[(ty + 8 * i) * kTs + tx] = aik[at];
-    if (J != K) sR[(ty + 8 * i) * kTs + tx] = akj[at];
+    d[i] = 1.0;
+    if (I != K) sL[(ty + 8 * i) * kTs + tx] = left[at];
+    if (J != K) sR[(ty + 8 * i) * kTs + tx] = right[at];
   }
   const int lane = tid & 63, wave = tid >> 6, qi = (wave >> 1) * 16, qj = (wave & 1) * 16;
   d4 c = {0, 0, 0, 0};
   if (I != K && J != K) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) c[r] = aij[size_t(qi + (lane >> 4) + 4 * r) * npad + qj + (lane & 15)];
+    for (int r = 0; r < 4; ++r) c[r] = out[size_t(qi + (lane >> 4) + 4 * r) * npad + qj + (lane & 15)];
   }
   bool bad = false;
-  // Gauss-Jordan on the block: pivot p, then a_ij -= a_ip a_pj / a_pp; row p scaled, column p negated
+  // elimination of the rows below each pivot; the columns behind it take up the inverse of the unit
+  // lower factor
 #pragma unroll
   for (int p = 0; p < kTile; ++p) {
     const int buf = p & 1;
@@ -315,43 +328,95 @@ __global__ __launch_bounds__(256) void spd_step_kernel(int npad, int K, const do
     double ip = __builtin_amdgcn_rcp(piv);  // two Newton steps: within an ulp, a third of a division's chain
     ip = fma(ip, fma(-piv, ip, 1.0), ip);
     ip = fma(ip, fma(-piv, ip, 1.0), ip);
-    const double rj = tx == p ? ip : s_row[buf][tx] * ip;  // new row p
+    const double rj = tx == p ? ip : s_row[buf][tx] * ip;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int row = ty + 8 * i;
-      if (row == p)
-        m[i] = rj;
-      else
-        m[i] = (tx == p ? 0.0 : m[i]) - s_col[buf][row] * rj;
+      if (row > p) m[i] = (tx == p ? 0.0 : m[i]) - s_col[buf][row] * rj;
+      if (row == p) d[i] = piv;
     }
+  }
+  // T = D^-1/2 times the inverse of the unit factor
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = ty + 8 * i;
+    m[i] = (tx < row ? m[i] : (tx == row ? 1.0 : 0.0)) / sqrt(d[i]);
   }
   if (I == K && J == K) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) bij[size_t(ty + 8 * i) * npad + tx] = m[i];
+    for (int i = 0; i < 4; ++i) out[size_t(ty + 8 * i) * npad + tx] = m[i];
     if (bad && tid == 0) status[0] = 1.0;
     return;
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) sD[(ty + 8 * i) * kTs + tx] = m[i];
+  for (int i = 0; i < 4; ++i) sT[(ty + 8 * i) * kTs + tx] = m[i];
   __syncthreads();
   if (I == K) {
-    c = tile_product(sD, sR, qi, qj, lane, c);
+    c = tile_product<false, false>(sT, sR, qi, qj, lane, c);
   } else {
-    d4 z = {0, 0, 0, 0};
-    const d4 t = tile_product(sL, sD, qi, qj, lane, z);  // A_IK D
-    if (J == K) {
+    const d4 z = {0, 0, 0, 0};
+    const d4 l = tile_product<false, true>(sL, sT, qi, qj, lane, z);  // L_IK
+    d4 g = z;                                                         // T M_KJ, or L_JK
+    if (J < K) g = tile_product<false, false>(sT, sR, qi, qj, lane, z);
+    if (J > K) g = tile_product<false, true>(sR, sT, qi, qj, lane, z);
+    __syncthreads();  // sL and sR are read
 #pragma unroll
-      for (int r = 0; r < 4; ++r) c[r] = -t[r];
-    } else {
-      __syncthreads();  // sL is read
-#pragma unroll
-      for (int r = 0; r < 4; ++r) sL[(qi + (lane >> 4) + 4 * r) * kTs + qj + (lane & 15)] = -t[r];
-      __syncthreads();
-      c = tile_product(sL, sR, qi, qj, lane, c);
+    for (int r = 0; r < 4; ++r) {
+      const int at = (qi + (lane >> 4) + 4 * r) * kTs + qj + (lane & 15);
+      sL[at] = -l[r];
+      sR[at] = g[r];
     }
+    __syncthreads();
+    if (J == K)
+      c = tile_product<false, false>(sL, sT, qi, qj, lane, c);
+    else if (J < K)
+      c = tile_product<false, false>(sL, sR, qi, qj, lane, c);
+    else
+      c = tile_product<false, true>(sL, sR, qi, qj, lane, c);
   }
 #pragma unroll
-  for (int r = 0; r < 4; ++r) bij[size_t(qi + (lane >> 4) + 4 * r) * npad + qj + (lane & 15)] = c[r];
+  for (int r = 0; r < 4; ++r) out[size_t(qi + (lane >> 4) + 4 * r) * npad + qj + (lane & 15)] = c[r];
+}
+
+// inv = F^T F, tile (I, J) of the lower triangle and its transpose; the next tiles of F are loaded under
+// the products
+__global__ __launch_bounds__(256) void spd_product_kernel(int n, int npad, const double* __restrict__ f,
+                                                          double* __restrict__ inv) {
+  __shared__ double sX[kTile * kTs], sY[kTile * kTs];
+  const int I = blockIdx.y, J = blockIdx.x, nt = npad / kTile;
+  if (J > I) return;
+  const int tid = threadIdx.x, tx = tid & 31, ty = tid >> 5;
+  const int lane = tid & 63, wave = tid >> 6, qi = (wave >> 1) * 16, qj = (wave & 1) * 16;
+  double x[4], y[4];
+  auto load = [&](int K) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const size_t row = size_t(K * kTile + ty + 8 * i) * npad + tx;
+      x[i] = f[row + I * kTile];
+      y[i] = f[row + J * kTile];
+    }
+  };
+  d4 c = {0, 0, 0, 0};
+  load(I);
+  for (int K = I; K < nt; ++K) {
+    __syncthreads();  // the last tiles are read
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      sX[(ty + 8 * i) * kTs + tx] = x[i];
+      sY[(ty + 8 * i) * kTs + tx] = y[i];
+    }
+    if (K + 1 < nt) load(K + 1);
+    __syncthreads();
+    c = tile_product<true, false>(sX, sY, qi, qj, lane, c);
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int i = I * kTile + qi + (lane >> 4) + 4 * r, j = J * kTile + qj + (lane & 15);
+    if (i < n && j <= i) {
+      inv[size_t(i) * n + j] = c[r];
+      inv[size_t(j) * n + i] = c[r];
+    }
+  }
 }
 
 // lanes per row and form of the precision argument, as in fne_spmv; false: not valid
@@ -555,12 +620,10 @@ extern "C" int fne_spd_inverse(int32_t n, const int32_t* indptr, const int32_t* 
   double* a = work;
   double* b = work + size_t(npad) * npad;
   hipLaunchKernelGGL(spd_rows_kernel, dim3(npad), dim3(256), 0, s, n, npad, indptr, indices, vals, b, status);
-  hipLaunchKernelGGL(spd_symmetrise_kernel, dim3(nt, nt), dim3(256), 0, s, npad, npad, b, npad, a);
-  for (int k = 0; k < nt; ++k) {
-    hipLaunchKernelGGL(spd_step_kernel, dim3(nt, nt), dim3(256), 0, s, npad, k, a, b, status);
-    std::swap(a, b);
-  }
-  hipLaunchKernelGGL(spd_symmetrise_kernel, dim3(nt, nt), dim3(256), 0, s, n, npad, a, n, inv);
+  hipLaunchKernelGGL(spd_symmetrise_kernel, dim3(nt, nt), dim3(256), 0, s, npad, b, a);
+  for (int k = 0; k < nt; ++k)
+    hipLaunchKernelGGL(spd_step_kernel, dim3(nt, nt - k), dim3(256), 0, s, npad, k, a, b, status);
+  hipLaunchKernelGGL(spd_product_kernel, dim3(nt, nt), dim3(256), 0, s, n, npad, b, inv);
   FNE_LAUNCH_CHECK();
   return FNE_OK;
 }

@@ -344,7 +344,8 @@ int fne_amg_transfers(int32_t nnz, const double* p, const int64_t* perm, double*
 int fne_amg_symmetrise(int32_t nnz, const double* c, const int64_t* perm, double* a, void* a_cycle,
                        int32_t precision, fne_stream_t stream);
 /*
- * Dense inverse (n x n, row-major, symmetric) of the symmetric part of a sparse FP64 matrix.  work:
+ * Dense inverse (n x n, row-major, symmetric) of the symmetric part of a sparse FP64 matrix, by its
+ * Cholesky factor: error of order n eps cond(A) of the inverse's largest entry, as LAPACK's.  work:
  * fne_spd_inverse_work_len(n) doubles.  status (device): 0, or 1 where a pivot was not positive and
  * finite, i.e. the matrix is not positive definite and inv is not valid.
  */

@@ -343,6 +343,37 @@ def test_spd_inverse_matches_numpy(require_gpu, n):
     assert run(bad)[1] == 1.0
 
 
+@pytest.mark.parametrize("n,cond", [(32, 1e8), (33, 1e8), (33, 1e11), (65, 1e10), (97, 1e12), (287, 1e11), (1200, 1e8)])
+def test_spd_inverse_is_as_accurate_as_lapack(require_gpu, n, cond):
+    """fne_spd_inverse of ill-conditioned operators, up to the default coarse size, against coarse_inverse
+    (potrf, potri).  The factor's inverse is within n eps cond of the inverse's largest entry in either."""
+    import scipy.sparse as sp
+    import torch
+
+    from fenics_nonlinear_energies_amd import native
+    from fenics_nonlinear_energies_amd.amg import coarse_inverse
+
+    rng = np.random.default_rng(n)
+    Q, _ = np.linalg.qr(rng.standard_normal((n, n)))
+    S = (Q * np.geomspace(1.0, 1.0 / cond, n)) @ Q.T
+    S = 0.5 * (S + S.T)
+    dev = torch.device("cuda")
+    C = sp.csr_matrix(S)
+    ptr, idx = (torch.as_tensor(a.astype(np.int32)).to(dev) for a in (C.indptr, C.indices))
+    val = torch.as_tensor(C.data).to(dev)
+    m = int(native.lib().fne_spd_inverse_work_len(n))
+    work, inv, status = (torch.full((k,), float("nan"), dtype=torch.float64, device=dev) for k in (m, n * n, 1))
+    native.check(native.lib().fne_spd_inverse(n, native.ptr(ptr), native.ptr(idx), native.ptr(val), native.ptr(work), m,
+                                              native.ptr(inv), native.ptr(status), native.stream_ptr()),
+                 "fne_spd_inverse")
+    ref, fallback = coarse_inverse(S)
+    assert not fallback and status.item() == 0.0
+    X = inv.cpu().numpy().reshape(n, n)
+    err = np.abs(X - ref).max() / np.abs(ref).max()
+    print("spd inverse", n, cond, err, flush=True)
+    assert err <= 2.0 * n * np.finfo(float).eps * cond
+
+
 def _host_levels(pc, A0):
     """Operators of every level read back from the device (FP64 masters)."""
     import scipy.sparse as sp
