@@ -344,9 +344,10 @@ int fne_plan_create(const fne_plan_desc* desc, fne_plan** out) {
     if (kEnergyBlocks > need) need = kEnergyBlocks;
     p->n_partials = int(need);
   }
+  // the fill is on the null stream, which a caller's stream need not wait for: done when this returns
   if (hipMalloc(&p->partials, sizeof(double2) * p->n_partials) != hipSuccess ||
       hipMalloc(&p->done, 2 * sizeof(unsigned)) != hipSuccess ||
-      hipMemset(p->done, 0, 2 * sizeof(unsigned)) != hipSuccess) {
+      hipMemset(p->done, 0, 2 * sizeof(unsigned)) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
     if (p->partials) (void)hipFree(p->partials);
     if (p->done) (void)hipFree(p->done);
     delete p;

@@ -134,6 +134,12 @@ struct HostParts {
         fne_set_error(std::string(name) + ": upload of the schedule failed");
         return FNE_EHIP;
       }
+    // on the null stream, which a caller's stream need not wait for: done when this returns
+    if (hipStreamSynchronize(nullptr) != hipSuccess) {
+      (void)hipFree(base);
+      fne_set_error(std::string(name) + ": upload of the schedule failed");
+      return FNE_EHIP;
+    }
     *out = base;
     return FNE_OK;
   }
