@@ -562,6 +562,7 @@ long max_width(const fne_mlp_desc* net) {
 }
 
 constexpr int kWgradSplits = 64;
+constexpr int kWgradRows = 128;  // rows of a chunk at least (narrow networks)
 
 bool narrow(const fne_mlp_desc* net) { return max_width(net) <= kNarrow; }
 
@@ -578,11 +579,11 @@ NarrowSizes narrow_sizes(const fne_mlp_desc* net, int64_t n) {
   }
   z.hidden = z.widths - net->dims[net->n_layers];
   z.blocks = (n + kNarrowRows - 1) / kNarrowRows;
-  // whole 32-row steps, at most kWgradSplits chunks of at least 128 rows: 64 chunks x 5 layers give
+  // whole 32-row steps, at most kWgradSplits chunks of at least kWgradRows rows: 64 chunks x 5 layers give
   // every CU a workgroup (39.9 us with the reduction at 16,384 rows; 128 chunks 41.6: more partial
   // sums to reduce)
   z.chunk = ((n + kWgradSplits - 1) / kWgradSplits + 31) / 32 * 32;
-  if (z.chunk < 128) z.chunk = 128;
+  if (z.chunk < kWgradRows) z.chunk = kWgradRows;
   z.splits = (n + z.chunk - 1) / z.chunk;
   return z;
 }
@@ -627,9 +628,12 @@ extern "C" {
 int64_t fne_mlp_workspace_bytes(const fne_mlp_desc* net, int64_t n) {
   if (!net_ok(net) || n < 0) return FNE_EINVAL;
   if (narrow(net)) {
-    // every hidden gradient, the weight gradients' partials, the column sums' partials
+    // every hidden gradient, the weight gradients' partials, the column sums' partials.  Chunks grow in
+    // steps of 32 rows, so their number falls again above 64 chunks of 128 rows: the most that any
+    // smaller n has, so that a workspace serves every smaller batch too
     const NarrowSizes z = narrow_sizes(net, n);
-    return int64_t(sizeof(float)) * (n * z.hidden + z.splits * z.weights + z.blocks * z.widths);
+    const long splits = n < kWgradSplits * kWgradRows ? (n + kWgradRows - 1) / kWgradRows : kWgradSplits;
+    return int64_t(sizeof(float)) * (n * z.hidden + splits * z.weights + z.blocks * z.widths);
   }
   const long w = max_width(net);
   const long chunks = (n + kColsumRows - 1) / kColsumRows;

@@ -141,3 +141,24 @@ def test_first_step_prediction_and_start_sample():
     ext = _predictor("extrapolate")[0]
     ext.first_step = True
     assert ext(history[:1], 0.5) is None  # extrapolation needs two states
+
+
+@pytest.mark.parametrize("dims", [[10, 128, 128, 128, 128, 3], [7, 64, 2], [3, 5], [10, 256, 256, 3]])
+def test_workspace_of_a_batch_serves_smaller_ones(dims):
+    """fne_mlp_workspace_bytes never falls with n, so the workspace of the largest batch is accepted for the
+    last, smaller one of an epoch."""
+    import ctypes as C
+
+    from fenics_nonlinear_energies_amd import native
+    from fenics_nonlinear_energies_amd.warmstart import _MlpDesc
+
+    d = _MlpDesc()
+    d.n_layers = len(dims) - 1
+    buf = C.create_string_buffer(8)
+    for i, v in enumerate(dims):
+        d.dims[i] = v
+    for l in range(len(dims) - 1):
+        d.w[l] = d.b[l] = C.addressof(buf)
+    n = list(range(1, 2100)) + list(range(8000, 9000)) + [16384, 16385, 20000, 65535, 65536, 65537, 100000]
+    need = [int(native.lib().fne_mlp_workspace_bytes(C.byref(d), k)) for k in n]
+    assert need[0] > 0 and all(a <= b for a, b in zip(need, need[1:]))
