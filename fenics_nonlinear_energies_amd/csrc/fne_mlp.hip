@@ -198,6 +198,7 @@ __global__ __launch_bounds__(256) void mlp_to_bf16_kernel(long n, const float* _
 // ---------------------------------------------------------------------------------------------
 constexpr int kNarrow = 128;
 constexpr int kNarrowStride = kNarrow + 8;  // LDS row of BF16: 272 B, so 16 rows start in 16 bank groups
+static_assert(kNarrowStride * sizeof(unsigned short) % 8 == 0, "rows are read in vectors of 8 bytes");
 
 typedef __bf16 mlp_b8 __attribute__((ext_vector_type(8)));
 typedef unsigned short mlp_u8 __attribute__((ext_vector_type(8)));
@@ -245,7 +246,7 @@ __device__ __forceinline__ void narrow_load_rows(const float* __restrict__ X, lo
 template <int R>
 __global__ __launch_bounds__(256) void mlp_narrow_forward_kernel(fne_mlp_desc net, long n, const float* __restrict__ x,
                                                                  float* __restrict__ y, float* __restrict__ acts) {
-  __shared__ unsigned short sA[R][kNarrowStride];
+  __shared__ __align__(16) unsigned short sA[R][kNarrowStride];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c15 = lane & 15, kq = 4 * (lane >> 4);
   const long row0 = long(blockIdx.x) * R;
@@ -315,8 +316,8 @@ __global__ __launch_bounds__(256) void mlp_narrow_chain_kernel(fne_mlp_desc net,
                                                                const float* __restrict__ acts,
                                                                const float* __restrict__ dy, float* __restrict__ dz,
                                                                float* __restrict__ cpart, int widths) {
-  __shared__ unsigned short sA[R][kNarrowStride];
-  __shared__ unsigned short sW[kNarrow][kNarrowStride];  // W_l transposed: [input][output]
+  __shared__ __align__(16) unsigned short sA[R][kNarrowStride];
+  __shared__ __align__(16) unsigned short sW[kNarrow][kNarrowStride];  // W_l transposed: [input][output]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c15 = lane & 15, kq = 4 * (lane >> 4);
   const long row0 = long(blockIdx.x) * R;
@@ -419,6 +420,7 @@ __global__ __launch_bounds__(256) void mlp_narrow_chain_kernel(fne_mlp_desc net,
 // dout x din product (four wavefronts of 64x64).  Rows are transposed into LDS as BF16, 32 at a
 // time (one K step of the 16x16x32 MFMA), the next 32 being loaded meanwhile.
 constexpr int kWgStride = 40;  // LDS row of 32 BF16: 80 B, 16-byte aligned fragments in 16 bank groups
+static_assert(kWgStride * sizeof(unsigned short) % 16 == 0, "rows are written and read in vectors of 16 bytes");
 
 struct MlpWgradArgs {
   const float* dz[FNE_MLP_MAX_LAYERS];  // [n][dims[l+1]]
@@ -430,8 +432,8 @@ struct MlpWgradArgs {
 
 __global__ __launch_bounds__(256) void mlp_narrow_wgrad_kernel(MlpWgradArgs g, long n, long chunk,
                                                                float* __restrict__ part) {
-  __shared__ unsigned short sD[kNarrow][kWgStride];
-  __shared__ unsigned short sH[kNarrow][kWgStride];
+  __shared__ __align__(16) unsigned short sD[kNarrow][kWgStride];
+  __shared__ __align__(16) unsigned short sH[kNarrow][kWgStride];
   const int l = blockIdx.y;
   const int M = g.dims[l + 1], N = g.dims[l];
   const float* D = g.dz[l];
