@@ -33,6 +33,9 @@ NEWTON_DEFAULTS = {
 }
 
 
+_PLAN_ENERGY = ReorderedElementAssemblerBase.energy_device
+
+
 class DeviceGoldenSearch:
     """Golden-section line search on the device (``fne_golden_search``): the same points and
     comparisons as ``minimizers.golden_section_search`` (``core/petsc/minimizers.py:14-64``), with
@@ -46,9 +49,13 @@ class DeviceGoldenSearch:
         self.trial = torch.empty(assembler.layout.n_free, dtype=torch.float64, device=dev)
         self.energy = torch.zeros(1, dtype=torch.float64, device=dev)
         self._init = torch.zeros(n_state, dtype=torch.float64)
-        # an assembler with an energy of its own evaluates it point by point
-        self._native = type(assembler).energy_device is ReorderedElementAssemblerBase.energy_device
+        self._native = True  # False: point by point, whatever the assembler's energy is
         self.searches = 0
+
+    def _plan_energy(self) -> bool:
+        """Whether the assembler's energy is the plan's and nothing else: an override in the class, or a
+        counter or hook set on the instance, is called point by point."""
+        return self._native and getattr(self.asm.energy_device, "__func__", None) is _PLAN_ENERGY
 
     def _point(self, xt: torch.Tensor, pt: torch.Tensor) -> None:
         lib = native.lib()
@@ -60,7 +67,7 @@ class DeviceGoldenSearch:
 
     def _points(self, xt: torch.Tensor, pt: torch.Tensor, bracket: tuple, points: int, resume: bool) -> None:
         lo, hi, tol = bracket
-        if self._native:
+        if self._plan_energy():
             asm = self.asm
             native.check(native.lib().fne_golden_search(
                 asm._plan, int(xt.numel()), native.ptr(xt), native.ptr(pt), native.ptr(asm.dvals),

@@ -98,3 +98,29 @@ def test_search_in_one_call_equals_point_by_point(require_gpu, make):
     st = steps.state.cpu().numpy()
     assert st[11] == 7.0 and (float(st[8]), float(st[9]), int(st[12])) == got
     asm.cleanup()
+
+
+def test_search_calls_an_energy_set_on_the_instance(require_gpu):
+    """A counter put over one assembler's energy_device sees every point, also when it is put there after
+    the search was made, and the search is the same."""
+    asm, x0, amp = _p1_asm()
+    x = asm.create_vec(x0)
+    d = asm.create_vec(amp * np.random.default_rng(3).standard_normal(x0.size))
+    search = DeviceGoldenSearch(asm)
+    ref = search(x, d, -0.5, 2.0, 1e-3)
+    plain, calls = asm.energy_device, []
+
+    def counted(*args, **kw):
+        calls.append(1)
+        return plain(*args, **kw)
+
+    asm.energy_device = counted
+    for s in (search, DeviceGoldenSearch(asm)):
+        calls.clear()
+        got = s(x, d, -0.5, 2.0, 1e-3)
+        assert len(calls) >= got[2] == ref[2]
+        assert abs(got[0] - ref[0]) <= 1e-12 and got[1] == pytest.approx(ref[1], rel=1e-13)
+    del asm.energy_device
+    calls.clear()
+    assert search(x, d, -0.5, 2.0, 1e-3) == ref and not calls
+    asm.cleanup()
