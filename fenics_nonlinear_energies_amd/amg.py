@@ -63,6 +63,8 @@ def _spmv_code(prec: int, avg: float, nnz: int) -> int:
     return prec | lanes_per_row(avg) << 8 if nnz < _STREAM_MIN_NNZ else spmv_code(prec, avg)
 
 
+_LANCZOS_MAX = 64  # steps that fne_lanczos_max takes
+
 # fne_vcycle_op operations
 _SWEEP_FIRST, _SWEEP, _RESIDUAL, _ADD_PRODUCT = 0, 1, 2, 3
 
@@ -547,10 +549,16 @@ class SmoothedAggregationPC:
             # rho(D^-1 A): largest Ritz value of a Lanczos run on D^-1/2 A D^-1/2, times a safety
             # factor, so that the smoother's omega rho stays well below 2
             n_l, lam = L["n"], state[2 * lvl:2 * lvl + 2]
-            native.check(lib.fne_lanczos_max(n_l, native.ptr(a_ptr), native.ptr(a_idx), native.ptr(a_dat), a_code,
-                                             native.ptr(L["diag"]), native.ptr(L["v0"]), self.LANCZOS_STEPS,
-                                             native.ptr(L["dinv"]), native.ptr(self._work), self._work.numel(),
-                                             native.ptr(lam), stream), "fne_lanczos_max")
+            if self.LANCZOS_STEPS <= _LANCZOS_MAX:
+                native.check(lib.fne_lanczos_max(n_l, native.ptr(a_ptr), native.ptr(a_idx), native.ptr(a_dat), a_code,
+                                                 native.ptr(L["diag"]), native.ptr(L["v0"]), self.LANCZOS_STEPS,
+                                                 native.ptr(L["dinv"]), native.ptr(self._work), self._work.numel(),
+                                                 native.ptr(lam), stream), "fne_lanczos_max")
+            else:
+                d = a_dat[L["diag"]].double()
+                torch.reciprocal(torch.where(d == 0.0, torch.ones_like(d), d), out=L["dinv"])
+                top = self._lanczos_lambda_max(lvl, A0, L["dinv"], L["v0"])
+                lam.copy_(torch.tensor([top, 1.0], dtype=torch.float64))
             for k0 in range(0, max(1, cheb.size), 8):  # omega = 4 / (3 safety lambda); Chebyshev steps by eights
                 f = np.ascontiguousarray(cheb[k0:k0 + 8])
                 native.check(lib.fne_smoother_weights(n_l, native.ptr(L["dinv"]), native.ptr(lam),
@@ -637,9 +645,9 @@ class SmoothedAggregationPC:
 
     def _lanczos_lambda_max(self, lvl: int, A0, dinv: torch.Tensor, v0: torch.Tensor) -> float:
         """Largest eigenvalue of D^-1 A (similar to S = D^-1/2 A D^-1/2) from LANCZOS_STEPS
-        Lanczos steps on S from the fixed start vector v0: the set-up's ``fne_lanczos_max`` in vector
-        operations (kept for checking it, and for operators that are not on the GPU), with one
-        transfer of the tridiagonal coefficients to the host.  A Krylov estimate: a
+        Lanczos steps on S from the fixed start vector v0, in vector operations with one transfer of
+        the tridiagonal coefficients to the host: for more steps than ``fne_lanczos_max`` takes, and
+        what that one is tested against.  A Krylov estimate: a
         few warm-started power iterations, used before, under-estimated rho once plasticity
         changed the spectrum, and the smoother (and so the V-cycle) became indefinite."""
         s = torch.sqrt(torch.abs(dinv))  # |D|^-1/2: finite where an indefinite Hessian has a negative diagonal

@@ -302,6 +302,35 @@ def test_lanczos_and_smoothed_product_match_host(require_gpu, n, width, prec):
     assert abs(got - want).max() <= 2 * 64 * 2.0**-53 * scale.max()
 
 
+@pytest.mark.parametrize("steps", [12, 64, 65, 90])
+def test_setup_takes_any_number_of_lanczos_steps(require_gpu, steps):
+    """LANCZOS_STEPS beyond the 64 that fne_lanczos_max takes: the Jacobi weights of the finest level hold a
+    Ritz value, between 0.9 (12 steps; 0.99 from 64 on) and all of the largest eigenvalue of D^-1 A."""
+    import torch
+
+    from fenics_nonlinear_energies_amd import amg
+    from fenics_nonlinear_energies_amd.linalg import DeviceCSR
+
+    p, adj, _ = build_plaplace_problem(16)
+    asm = PLaplaceReorderedElementAssembler(p, None, adj)
+    asm.assemble_hessian(asm.create_vec(np.random.default_rng(2).random(asm.layout.n_free)))
+    pc = amg.SmoothedAggregationPC(max_coarse=20)
+    pc.LANCZOS_STEPS = steps
+    pc.setup(asm.A)
+    H = asm.A.to_scipy().toarray()
+    s = 1.0 / np.sqrt(H.diagonal())
+    top = np.linalg.eigvalsh(s[:, None] * H * s).max()
+    L = pc.levels[0]
+    lam = 4.0 / (3.0 * pc.RHO_SAFETY) * (L["dinv"] / L["wd"]).cpu().numpy()
+    assert np.ptp(lam) <= 1e-13 * lam.max()
+    assert (0.9 if steps < 64 else 0.99) * top <= lam[0] <= (1 + 1e-12) * top
+    r = torch.ones(asm.layout.n_free, dtype=torch.float64, device="cuda")
+    z = torch.empty_like(r)
+    pc.apply(r, z)
+    assert torch.isfinite(z).all()
+    asm.cleanup()
+
+
 @pytest.mark.parametrize("n", [1, 31, 32, 33, 64, 97, 287])
 def test_spd_inverse_matches_numpy(require_gpu, n):
     """fne_spd_inverse at the edges of its 32-column blocks: a matrix of condition 1e4 (n eps cond is
