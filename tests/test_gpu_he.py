@@ -158,3 +158,22 @@ def test_node_patches_leave_mixed_orders_to_the_row_gather(require_gpu):
         out.append(asm.A.data.clone())
         asm.cleanup()
     assert torch.equal(*out)
+
+
+@pytest.mark.parametrize("dims,amp", [((6, 2, 2), 1e-4), ((6, 2, 2), 1e-7), ((40, 9, 7), 1e-6)])
+def test_fused_energy_is_the_separate_one_near_rest(require_gpu, dims, amp):
+    """Near rest an element's energy is the difference of terms of size C1, so its rounding is relative
+    to those and not to the energy.  The fused call and fne_energy round every element alike and add
+    up with compensation: equal to the last two bits each, 4 eps."""
+    p, adj, u0 = build_beam_problem(*dims)
+    asm = HEReorderedElementAssembler(p, None, adj)
+    rest = np.asarray(p["nodes2coord"]).reshape(-1)[np.asarray(p["freedofs"])]
+    u = rest + amp * np.random.default_rng(1).standard_normal(rest.size) / max(dims[1:])
+    x = asm.create_vec(u[asm.layout.perm])
+    asm.dvals.copy_(torch.as_tensor(np.asarray(p["nodes2coord"]).reshape(-1)))
+    e = float(asm.energy_device(x.t).item())
+    g = x.duplicate()
+    fused = float(asm.energy_grad_hessian_device(x.t, g.t).item())
+    print("near rest", dims, amp, e, fused - e, flush=True)
+    assert np.isfinite(e) and abs(fused - e) <= 4 * np.finfo(float).eps * abs(e)
+    asm.cleanup()
