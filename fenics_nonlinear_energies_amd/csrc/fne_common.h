@@ -87,7 +87,7 @@ struct fne_plan {
   // [n_elem][n_loc][n_loc] (FP64 or FP32), written by the element kernel, read by the row gather
   double* mc_g = nullptr;
   void* mc_h = nullptr;
-  FneRowUnits units;  // Mohr-Coulomb: n_unit = 0 (every row by itself) until fne_plan_build_row_units
+  FneRowUnits units;  // Mohr-Coulomb: n_unit = 0 (row gather) until fne_plan_build_row_units
   FneNodePatches np;  // tetrahedra: n_patch = 0 until fne_plan_build_node_patches
 };
 

@@ -18,6 +18,7 @@
 //                          element (fixed ascending order) lane c adds the entries of node c into
 //                          an LDS copy of the CSR rows at the precomputed byte positions; the rows
 //                          are then written once.  No atomics: results are bitwise reproducible.
+//                          Plans without row units: row_gather_kernel, the same row by row.
 #include "fne_common.h"
 
 #include <algorithm>
@@ -209,9 +210,11 @@ template <> struct Pair<double> {
 __device__ __forceinline__ float mc_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double mc_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
-// blocks of the element kernel, each with `rounds` rounds of consecutive elements
+// blocks of the element kernel, each with `rounds` rounds of consecutive elements; by_rows: element
+// matrices row by row, for plans without row units
 struct McBlocks {
   int rounds = 1, all = 1;
+  bool by_rows = false;
 };
 
 // LDS of one wavefront
@@ -227,7 +230,8 @@ struct McWaveLds {
 
 // Values of an element matrix in the scratch, [n][m][j][i]: rows (n, i), columns (m, j).  The node rows
 // of P4 have 16 columns: 256 B (FP32) or 512 B at multiples of that, so that the row gather reads two
-// lines of 128 B for each instead of 2.75 (32,000 elements, assembly 140 -> 127 us).
+// lines of 128 B for each instead of 2.75 (32,000 elements, assembly 140 -> 127 us).  With by_rows a row
+// (n, i) is kMcNodeRow / 2 values in the order of its columns.
 template <int NN>
 constexpr int kMcNodeRow = 4 * (NN == 15 ? 16 : NN);
 template <int NN>
@@ -456,7 +460,8 @@ __global__ __launch_bounds__(kBlock, WH && sizeof(HT) == 8 && (WG || (NN == 15 &
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               const int row = Vec4<HT>::row(kk, r);  // 2 n + i
-              if (row < NL) H[(row >> 1) * kMcNodeRow<NN> + c15 * 2 + (row & 1)] = acc[r];
+              const int to = B.by_rows ? (row & 1) * (kMcNodeRow<NN> / 2) + c15 : c15 * 2 + (row & 1);
+              if (row < NL) H[(row >> 1) * kMcNodeRow<NN> + to] = acc[r];
             }
           }
         } else {
@@ -478,9 +483,13 @@ __global__ __launch_bounds__(kBlock, WH && sizeof(HT) == 8 && (WG || (NN == 15 &
 #pragma unroll
           for (int r = 0; r < 4; ++r) {  // column 15 is zero
             const int n = Vec4<HT>::row(kk, r);
-            if (n < NN) {
+            if (n < NN && !B.by_rows) {
               V4 v = {axx[r], ayx[r], axy[r], ayy[r]};
               *reinterpret_cast<V4*>(H + n * kMcNodeRow<NN> + c15 * 4) = v;
+            } else if (n < NN) {
+              HT2* to = reinterpret_cast<HT2*>(H + n * kMcNodeRow<NN>) + c15;
+              to[0] = HT2{axx[r], axy[r]};
+              to[kMcNodeRow<NN> / 4] = HT2{ayx[r], ayy[r]};
             }
           }
         }
@@ -498,79 +507,139 @@ __global__ __launch_bounds__(kBlock, WH && sizeof(HT) == 8 && (WG || (NN == 15 &
   }
 }
 
-// Row gather of tetrahedral plans without node patches (element matrices row-major [12][12]).  Eight
-// lanes own a CSR row; lane c < 6 handles the element columns 2c and 2c+1 (paired loads).
-// inc[it] = element * 32 + local row lists the incidences of every row (elements ascending);
-// pos[it*32 + c] is the position of the element's local column c inside the row (255 = constrained).
-// Up to 8 items' element rows and positions are fetched together and then added in item order into
-// an LDS copy of the row, which is written once.  Every CSR entry therefore sums its contributions
-// in a fixed order.  One row per group (320x16x16 beam: 0.335 ms; 0.37 with 2 rows, 0.40 with 4).
-template <typename HT, bool WG, bool WH>
-__global__ __launch_bounds__(kBlock) void tet_row_gather_kernel(fne_plan_desc d, const HT* __restrict__ hbuf,
-                                                                const double* __restrict__ gbuf,
-                                                                const double* __restrict__ f,
-                                                                double* __restrict__ g, HT* __restrict__ vals) {
-  extern __shared__ unsigned char mc_smem[];
-  constexpr int NL = 12, kL = mc_row_lanes(NL), kPf = 8;
+// Row gather of element matrices stored row by row: tetrahedral plans without node patches and
+// Mohr-Coulomb plans without row units.  A group of mc_row_lanes(NL) lanes owns kRB consecutive CSR rows;
+// lane c < NL/2 handles the element columns 2c and 2c+1 (paired loads).  inc[it] = element * 32 + local row
+// lists the incidences of every row (rows consecutive, elements ascending); pos[it*32 + c] is the
+// position of the element's local column c inside the row (255 = constrained).  The incidences of the
+// batch are read in one load (lane j holds item j), up to 8 items' element rows and positions are
+// fetched together and then added in item order into LDS copies of the rows, which are written once.
+// Every CSR entry therefore sums its contributions in a fixed order.  One row per group for 12 columns
+// (320x16x16 beam: 0.335 ms; 0.37 with 2 rows, 0.40 with 4), two for the 30 of P4 (98,000 elements: 0.50 ms;
+// 0.55 with 1, 0.52 with 4).
+template <int NL>
+constexpr int kRowStride = NL == 30 ? kMcNodeRow<15> / 2 : NL;  // of an element matrix
+template <int NL>
+constexpr int kRowBatch = NL == 30 ? 2 : 1;
+
+template <int NL, typename HT, bool WG, bool WH>
+__global__ __launch_bounds__(kBlock) void row_gather_kernel(fne_plan_desc d, const HT* __restrict__ hbuf,
+                                                            const double* __restrict__ gbuf,
+                                                            const double* __restrict__ f,
+                                                            double* __restrict__ g, HT* __restrict__ vals) {
+  extern __shared__ __align__(16) unsigned char mc_smem[];
+  constexpr int kL = mc_row_lanes(NL), kRB = kRowBatch<NL>, kRowsBlk = (kBlock / kL) * kRB, kPf = 8;
   typedef typename Pair<HT>::type HT2;
   const int cap = (d.max_row_len + 1) & ~1;
   const int grp = threadIdx.x / kL;
   const int c = threadIdx.x & (kL - 1);
-  HT* sRow = reinterpret_cast<HT*>(mc_smem) + size_t(grp) * cap;
-  const int row = xcd_remap(blockIdx.x, gridDim.x) * (kBlock / kL) + grp;
-  if (row >= d.n_free) return;  // uniform over the lane group; no block-level barrier below
+  HT* sRows = reinterpret_cast<HT*>(mc_smem) + size_t(grp) * kRB * cap;
+  const int r0 = xcd_remap(blockIdx.x, gridDim.x) * kRowsBlk + grp * kRB;
+  if (r0 >= d.n_free) return;  // uniform over the lane group; no block-level barrier below
+  const int nr = min(kRB, d.n_free - r0);
   const unsigned char* pos = reinterpret_cast<const unsigned char*>(d.pitem);
   const unsigned int* inc = reinterpret_cast<const unsigned int*>(d.inc);
-  const int ip_l = c <= 1 && WH ? d.indptr[row + c] : 0;
-  const int ic_l = c <= 1 ? d.inc_ptr[row + c] : 0;
-  const int k0 = __shfl(ip_l, 0, kL), k1 = __shfl(ip_l, 1, kL);
-  const int i0 = __shfl(ic_l, 0, kL), i1 = __shfl(ic_l, 1, kL);
+  const int ip_l = c <= nr && WH ? d.indptr[r0 + c] : 0;
+  const int ic_l = c <= nr ? d.inc_ptr[r0 + c] : 0;
+  int kb[kRB + 1], ib[kRB + 1];
+#pragma unroll
+  for (int t = 0; t <= kRB; ++t) {
+    kb[t] = __shfl(ip_l, t < nr ? t : nr, kL);
+    ib[t] = __shfl(ic_l, t < nr ? t : nr, kL);
+  }
   if (WH) {
-    for (int j = c; j < k1 - k0; j += kL) sRow[j] = HT(0);
+#pragma unroll
+    for (int t = 0; t < kRB; ++t)
+      if (t < nr)
+        for (int j = c; j < kb[t + 1] - kb[t]; j += kL) sRows[t * cap + j] = HT(0);
   }
   __builtin_amdgcn_wave_barrier();
-  double gacc = 0.0;
-  for (int base = i0; base < i1; base += kL) {
-    const int nb = min(kL, i1 - base);
+  double gacc = 0.0;  // lane t < nr: gradient of row r0 + t
+  for (int base = ib[0]; base < ib[nr]; base += kL) {
+    const int nb = min(kL, ib[nr] - base);
     const unsigned int mine = c < nb ? inc[base + c] : 0u;
+    int myslot = 0;
+#pragma unroll
+    for (int t = 1; t < kRB; ++t)
+      if (t < nr && base + c >= ib[t]) myslot = t;
     if (WG) {
       const double gv = c < nb ? gbuf[size_t(mine >> 5) * 32 + (mine & 31u)] : 0.0;
-      for (int j = 0; j < nb; ++j) gacc += __shfl(gv, j, kL);
+      for (int j = 0; j < nb; ++j) {
+        const double v = __shfl(gv, j, kL);
+        const int t = __shfl(myslot, j, kL);
+        if (c == t) gacc += v;
+      }
     }
     if (WH) {
-      HT2 v[kPf];
-      unsigned int pp[kPf];
+      for (int j0 = 0; j0 < nb; j0 += kPf) {
+        HT2 v[kPf];
+        unsigned int pp[kPf];
+        int sl[kPf];
 #pragma unroll
-      for (int j = 0; j < kPf; ++j) {
-        const unsigned int item = __shfl(mine, j < nb ? j : 0, kL);
-        v[j] = Pair<HT>::zero();
-        pp[j] = 0xFFFFu;
-        if (j < nb && c < NL / 2) {
-          pp[j] = *reinterpret_cast<const unsigned short*>(pos + size_t(base + j) * 32 + 2 * c);
-          v[j] = *reinterpret_cast<const HT2*>(hbuf + size_t(item >> 5) * (NL * NL) + (item & 31u) * NL + 2 * c);
+        for (int jj = 0; jj < kPf; ++jj) {
+          const int j = j0 + jj;
+          const unsigned int item = __shfl(mine, j < nb ? j : 0, kL);
+          sl[jj] = __shfl(myslot, j < nb ? j : 0, kL);
+          v[jj] = Pair<HT>::zero();
+          pp[jj] = 0xFFFFu;
+          if (j < nb && c < NL / 2) {
+            pp[jj] = *reinterpret_cast<const unsigned short*>(pos + size_t(base + j) * 32 + 2 * c);
+            v[jj] = *reinterpret_cast<const HT2*>(hbuf + size_t(item >> 5) * (NL * kRowStride<NL>) +
+                                                  (item & 31u) * kRowStride<NL> + 2 * c);
+          }
         }
-      }
 #pragma unroll
-      for (int j = 0; j < kPf; ++j) {
-        const unsigned int p0 = pp[j] & 0xFFu, p1 = pp[j] >> 8;
-        if (p0 != kPosNone) sRow[p0] += v[j].x;
-        if (p1 != kPosNone) sRow[p1] += v[j].y;
-        __builtin_amdgcn_wave_barrier();
+        for (int jj = 0; jj < kPf; ++jj) {
+          const unsigned int p0 = pp[jj] & 0xFFu, p1 = pp[jj] >> 8;
+          if (p0 != kPosNone) sRows[sl[jj] * cap + p0] += v[jj].x;
+          if (p1 != kPosNone) sRows[sl[jj] * cap + p1] += v[jj].y;
+          __builtin_amdgcn_wave_barrier();
+        }
       }
     }
   }
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   if (WH) {
-    for (int j = c; j < k1 - k0; j += kL) vals[k0 + j] = sRow[j];
+#pragma unroll
+    for (int t = 0; t < kRB; ++t)
+      if (t < nr)
+        for (int j = c; j < kb[t + 1] - kb[t]; j += kL) vals[kb[t] + j] = sRows[t * cap + j];
   }
-  if (WG && c == 0) g[row] = f ? gacc - f[row] : gacc;
+  if (WG && c < nr) g[r0 + c] = f ? gacc - f[r0 + c] : gacc;
+}
+
+template <int NL>
+int launch_row_gather(fne_plan* plan, bool want_g, bool want_h, const FneCall& c) {
+  const fne_plan_desc& d = plan->d;
+  const bool fp32 = c.precision == FNE_FP32;
+  const int rows_per_block = kBlock / mc_row_lanes(NL) * kRowBatch<NL>;
+  const dim3 grid((d.n_free + rows_per_block - 1) / rows_per_block);
+  const int cap = (d.max_row_len + 1) & ~1;
+  const size_t shm = want_h ? size_t(rows_per_block) * cap * (fp32 ? 4 : 8) : 0;
+  if (shm > plan->max_lds || d.max_row_len > 254) {
+    fne_set_error("row gather: CSR rows too long for the LDS row copies");
+    return FNE_EINVAL;
+  }
+  if (d.n_free == 0 || (!want_g && !want_h)) return FNE_OK;
+#define RG(HT, G, H)                                                                                \
+  hipLaunchKernelGGL((row_gather_kernel<NL, HT, G, H>), grid, dim3(kBlock), shm, c.stream, d,       \
+                     (const HT*)plan->mc_h, plan->mc_g, c.f, c.g, (HT*)c.vals)
+  if (!want_h) RG(double, true, false);
+  else if (fp32) { if (want_g) RG(float, true, true); else RG(float, false, true); }
+  else { if (want_g) RG(double, true, true); else RG(double, false, true); }
+#undef RG
+  FNE_LAUNCH_CHECK();
+  return FNE_OK;
 }
 
 // ---------------------------------------------------------------------------------------------
 // Mohr-Coulomb rows from element matrices stored as [n][m][j][i].  A unit is a CSR row, or the x and
-// y rows of a node with the same columns and elements (FneRowUnits; without them every row is one):
-// positions and incidences are then read once for two rows, and a lane reads its node pair as one
-// vector.  mc_row_lanes lanes per unit; the contributions are added in item order into LDS copies of
+// y rows of a node with the same columns and elements (FneRowUnits): positions and incidences are then
+// read once for two rows, and a lane reads its node pair as one vector.  Plans without units take
+// row_gather_kernel, whose rows lie together in memory: a unit of one row reads twice the bytes that it
+// needs (32,000 P4 elements, Hessian with every row a unit of its own: FP64 272 us, FP32 125 to 146; row
+// gather 195 and 109; pairs 198 and 101).
+// mc_row_lanes lanes per unit; the contributions are added in item order into LDS copies of
 // the rows, which are written once (storing rows of a single element straight from the registers
 // measured the same).  Bound by memory traffic: P4 FP32, 98,000 elements: 376 MB of element matrices,
 // 60 MB of positions and incidences, 314 MB of values, 231 us = 3.2 TB/s (before: rows one by one,
@@ -608,10 +677,8 @@ __global__ __launch_bounds__(kBlock) void mc_unit_gather_kernel(fne_plan_desc d,
   const int u = xcd_remap(blockIdx.x, gridDim.x) * kGroups + grp;
   if (u >= n_unit) return;  // uniform over the lane group; no block-level barrier below
   const McUnit w = mc_unit(d, U, u);
-  const unsigned char* pos = U.unit ? U.pos + size_t(w.item0) * (2 * kL) + 2 * c
-                                    : reinterpret_cast<const unsigned char*>(d.pitem) + size_t(w.item0) * 32 + 2 * c;
-  const int pos_stride = U.unit ? 2 * kL : 32;
-  const unsigned int* inc = (U.unit ? U.inc : reinterpret_cast<const unsigned int*>(d.inc)) + w.item0;
+  const unsigned char* pos = U.pos + size_t(w.item0) * (2 * kL) + 2 * c;
+  const unsigned int* inc = U.inc + w.item0;
   // both rows side by side; entry `none` takes what falls on constrained columns and idle lanes
   const unsigned none = d.max_row_len;
   HT2* buf = reinterpret_cast<HT2*>(mc_unit_smem) + size_t(grp) * (none + 1);
@@ -630,7 +697,7 @@ __global__ __launch_bounds__(kBlock) void mc_unit_gather_kernel(fne_plan_desc d,
       for (int jj = 0; jj < kPf; ++jj) {
         pp[jj] = 0xFFFFu;
         if (j0 + jj < nb && c < NN)
-          pp[jj] = *reinterpret_cast<const unsigned short*>(pos + size_t(base + j0 + jj) * pos_stride);
+          pp[jj] = *reinterpret_cast<const unsigned short*>(pos + size_t(base + j0 + jj) * (2 * kL));
       }
 #pragma unroll
       for (int jj = 0; jj < kPf; ++jj) {
@@ -761,6 +828,7 @@ int launch_mc_rows(fne_plan* plan, bool want_g, bool want_h, const FneCall& c) {
     FNE_LAUNCH_CHECK();
     return FNE_OK;
   }
+  if (plan->units.n_unit == 0) return launch_row_gather<2 * NN>(plan, want_g, true, c);
   constexpr int kGroups = kBlock / mc_row_lanes(2 * NN);
   const bool fp32 = c.precision == FNE_FP32;
   const size_t shm = size_t(kGroups) * 2 * (d.max_row_len + 1) * (fp32 ? 4 : 8);
@@ -788,7 +856,8 @@ template <int NN>
 int launch_mc(fne_plan* plan, FneOp op, const FneCall& c) {
   const fne_plan_desc& d = plan->d;
   const int ne = d.n_elem;
-  const McBlocks B = mc_blocks(ne);
+  McBlocks B = mc_blocks(ne);
+  B.by_rows = plan->units.n_unit == 0 && op != kOpElementEval;
   const int nb = B.all;
   if (nb > plan->n_partials) {
     fne_set_error("energy reduction scratch too small");
@@ -1042,30 +1111,11 @@ extern "C" int fne_hessian_diag(fne_plan* plan, const double* x, const double* d
 }
 
 int fne_launch_row_gather(fne_plan* plan, bool want_g, bool want_h, const FneCall& c) {
-  const fne_plan_desc& d = plan->d;
-  const bool fp32 = c.precision == FNE_FP32;
-  const int rows_per_block = kBlock / mc_row_lanes(12);
-  const dim3 grid((d.n_free + rows_per_block - 1) / rows_per_block);
-  const int cap = (d.max_row_len + 1) & ~1;
-  const size_t shm = want_h ? size_t(rows_per_block) * cap * (fp32 ? 4 : 8) : 0;
-  if (shm > plan->max_lds || d.max_row_len > 254) {
-    fne_set_error("row gather: CSR rows too long for the LDS row copies");
-    return FNE_EINVAL;
-  }
-  if (d.n_loc != 12) {
+  if (plan->d.n_loc != 12) {
     fne_set_error("row gather supports elements with 12 DOFs");
     return FNE_EINVAL;
   }
-  if (d.n_free == 0 || (!want_g && !want_h)) return FNE_OK;
-#define RG(HT, G, H)                                                                              \
-  hipLaunchKernelGGL((tet_row_gather_kernel<HT, G, H>), grid, dim3(kBlock), shm, c.stream, d,     \
-                     (const HT*)plan->mc_h, plan->mc_g, c.f, c.g, (HT*)c.vals)
-  if (!want_h) RG(double, true, false);
-  else if (fp32) { if (want_g) RG(float, true, true); else RG(float, false, true); }
-  else { if (want_g) RG(double, true, true); else RG(double, false, true); }
-#undef RG
-  FNE_LAUNCH_CHECK();
-  return FNE_OK;
+  return launch_row_gather<12>(plan, want_g, want_h, c);
 }
 
 size_t fne_mc_scratch_bytes(const fne_plan_desc& d, size_t* gbytes) {

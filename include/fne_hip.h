@@ -139,9 +139,10 @@ int fne_plan_build_node_patches(fne_plan* plan, const int32_t* edof, const int32
  * Mohr-Coulomb plans with row incidences: list the row units (a row, or the x and y rows of a node
  * with the same columns and elements), so that assembly reads incidences and positions once for two
  * rows.  HOST pointers, the same values as the descriptor's device arrays: inc_ptr [n_free+1], inc,
- * pos (pitem: [items][32] bytes), indptr, indices; read during the call only.  Without this call, and with FNE_EUNSUPPORTED (rows
- * longer than 254 entries), every row is a unit of its own.  Allocates the list once (freed by
- * fne_plan_destroy).  Part of the scatter build
+ * pos (pitem: [items][32] bytes), indptr, indices; read during the call only.  Without this call, with
+ * FNE_EUNSUPPORTED (rows longer than 254 entries) and with fewer than three quarters of the rows in such
+ * pairs the plan assembles row by row.  Allocates the list once (freed by fne_plan_destroy).  Part of
+ * the scatter build
  * (core/petsc/reordered_element_base.py:1464-1534).
  */
 int fne_plan_build_row_units(fne_plan* plan, const int32_t* inc_ptr, const uint32_t* inc, const unsigned char* pos,

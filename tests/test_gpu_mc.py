@@ -106,6 +106,49 @@ class _SingleRows(SlopeStabilityReorderedElementAssembler):
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
 @pytest.mark.parametrize("degree,h,order", [
+    (4, 10.0, "odd"),  # a y component constrained by itself: the last batch has one row
+    (4, 3.0, "block_xyz"),
+    (4, 3.0, "apart"),  # the x rows, then the y rows
+    (2, 1.3, "block_morton"),
+    (2, 1.6, "apart"),
+])
+def test_rows_without_units_match_the_oracle(require_gpu, degree, h, order, precision):
+    """The row-by-row form: plans without row units, and orderings that leave no pairs to list.  Tolerances
+    of the tests above."""
+    p, adj = mc_params(h=h, degree=degree, lam=1.5)
+    kw = {"reorder_mode": order}
+    if order == "odd":
+        keep = np.delete(np.arange(p["freedofs"].size), 101)
+        p, adj, kw = dict(p, freedofs=np.asarray(p["freedofs"])[keep]), adj.tocsr()[keep][:, keep], {}
+    free = np.asarray(p["freedofs"])
+    assert (free.size % 2 == 1) == (order == "odd")
+    if order == "apart":
+        kw = {"perm_override": np.argsort(free % 2, kind="stable")}
+    cls = SlopeStabilityReorderedElementAssembler if order == "apart" else _SingleRows
+    asm = cls(p, None, adj, hessian_precision=precision, **kw)
+    lay = asm.layout
+    u = _state(p, lay, 6)
+    ref = assembly.assemble("mc", p, u)
+    x = asm.create_vec(u[lay.perm])
+    g, y = x.duplicate(), x.duplicate()
+    asm.A.data.fill_(float("nan"))  # every entry is written
+    e = float(asm.energy_grad_hessian_device(x.t, g.t).item())
+    H = asm.A.to_scipy()[lay.iperm][:, lay.iperm]
+    assert abs(e - ref["e"]) <= 1e-12 * abs(ref["e"])
+    assert np.abs(g.array[lay.iperm] - ref["g"]).max() <= 1e-11 * np.abs(ref["g"]).max()
+    assert abs(H - ref["h"]).max() <= (1e-10 if precision == "fp64" else 3e-5) * abs(ref["h"]).max()
+    v = asm.A.data.clone()
+    asm.A.data.fill_(float("nan"))
+    asm.hessian_device(x.t)
+    assert torch.equal(asm.A.data, v)
+    asm.hvp_device(x.t, x.t, y.t)
+    want = ref["h"] @ u
+    assert np.abs(y.array[lay.iperm] - want).max() <= 1e-10 * np.abs(want).max()
+    asm.cleanup()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("degree,h,order", [
     (4, 10.0, "block_morton"),  # fewer elements than a block's wavefronts take
     (4, 4.0, "block_morton"),
     (4, 2.2, "block_xyz"),  # rows of a node together
