@@ -744,7 +744,7 @@ __global__ __launch_bounds__(kBlock) void mc_unit_gather_kernel(fne_plan_desc d,
     HT o[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int i = min(max(i0 + j * kL, 0), n - 1);
+      const int i = max(min(i0 + j * kL, n - 1), 0);  // (a row without entries reads one and stores none)
       o[j] = i < w.len ? buf[i].x : buf[i - w.len].y;
     }
 #pragma unroll

@@ -7,6 +7,7 @@ largest entry (FP32 MFMA accumulation over 2 n_q = 38 products).
 
 import numpy as np
 import pytest
+import scipy.sparse as sp
 import torch
 
 from fenics_nonlinear_energies_amd.problems.slope_stability import SlopeStabilityReorderedElementAssembler
@@ -145,6 +146,37 @@ def test_rows_without_units_match_the_oracle(require_gpu, degree, h, order, prec
     want = ref["h"] @ u
     assert np.abs(y.array[lay.iperm] - want).max() <= 1e-10 * np.abs(want).max()
     asm.cleanup()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("degree", [4, 2])
+@pytest.mark.parametrize("cls", [SlopeStabilityReorderedElementAssembler, _SingleRows])
+def test_free_node_without_elements(require_gpu, cls, degree, precision):
+    """A free node that no element names has CSR rows without entries: nothing is read or stored for them,
+    the other rows are those of the mesh without it, and its gradient is minus its load."""
+    p, adj = mc_params(h=5.0, degree=degree, lam=1.2)
+    n, nt = p["freedofs"].size, p["nodes"].shape[0]
+    q = dict(p, nodes=np.vstack((p["nodes"], [[60.0, 60.0]])), freedofs=np.append(p["freedofs"], [2 * nt, 2 * nt + 1]),
+             force=np.append(p["force"], [3.0, -2.0]), u_0=np.append(p["u_0"], [0.0, 0.0]))
+    adj2 = sp.block_diag((adj, sp.coo_matrix((2, 2))))
+    asm = cls(q, None, adj2, hessian_precision=precision)
+    lay = asm.layout
+    lens = np.diff(lay.indptr)[lay.iperm]
+    assert np.all(lens[n:] == 0) and np.all(lens[:n] > 0)
+    ref_asm = cls(p, None, adj)
+    u = _state(p, ref_asm.layout, 3)
+    ref = assembly.assemble("mc", p, u)
+    x = asm.create_vec(np.append(u, [0.3, -0.1])[lay.perm])
+    g = x.duplicate()
+    asm.A.data.fill_(float("nan"))
+    asm.energy_grad_hessian_device(x.t, g.t)
+    H = asm.A.to_scipy()[lay.iperm][:, lay.iperm][:n, :n]
+    assert abs(H - ref["h"]).max() <= (1e-10 if precision == "fp64" else 3e-5) * abs(ref["h"]).max()
+    got = g.array[lay.iperm]
+    assert np.abs(got[:n] - ref["g"]).max() <= 1e-11 * np.abs(ref["g"]).max()
+    assert got[n:].tolist() == [-3.0, 2.0]
+    asm.cleanup()
+    ref_asm.cleanup()
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
