@@ -403,6 +403,36 @@ def test_spd_inverse_is_as_accurate_as_lapack(require_gpu, n, cond):
     assert err <= 2.0 * n * np.finfo(float).eps * cond
 
 
+@pytest.mark.parametrize("coarse", ["host", "device"])
+def test_setup_after_a_failed_one(require_gpu, coarse):
+    """A set-up on an operator with a NaN raises; the next one, on the same object with finite values, leaves
+    the hierarchy and the cycle of a new object bit for bit."""
+    import torch
+
+    from fenics_nonlinear_energies_amd import amg
+
+    p, adj, _ = build_plaplace_problem(24)
+    asm = PLaplaceReorderedElementAssembler(p, None, adj)
+    asm.assemble_hessian(asm.create_vec(np.random.default_rng(2).random(asm.layout.n_free)))
+    r = torch.as_tensor(np.random.default_rng(3).standard_normal(asm.layout.n_free)).cuda()
+
+    def result(pc):
+        pc.setup(asm.A)
+        z = torch.empty_like(r)
+        pc.apply(r, z)
+        return [z] + [t for L in pc.levels for t in (L["P64"].data, L["Ac64"].data, L["wd"], L["wcheb"])]
+
+    pc = amg.SmoothedAggregationPC(max_coarse=30, coarse_factor=coarse)
+    good = asm.A.data.clone()
+    asm.A.data[asm.A.nnz // 2] = float("nan")
+    with pytest.raises(FloatingPointError):
+        pc.setup(asm.A)
+    asm.A.data.copy_(good)
+    got, ref = result(pc), result(amg.SmoothedAggregationPC(max_coarse=30, coarse_factor=coarse))
+    assert all(torch.equal(a, b) and torch.isfinite(a).all() for a, b in zip(got, ref))
+    asm.cleanup()
+
+
 def _host_levels(pc, A0):
     """Operators of every level read back from the device (FP64 masters)."""
     import scipy.sparse as sp

@@ -177,3 +177,25 @@ def test_fused_energy_is_the_separate_one_near_rest(require_gpu, dims, amp):
     print("near rest", dims, amp, e, fused - e, flush=True)
     assert np.isfinite(e) and abs(fused - e) <= 4 * np.finfo(float).eps * abs(e)
     asm.cleanup()
+
+
+@pytest.mark.parametrize("cls", [HEReorderedElementAssembler, _RowGather])
+def test_energy_of_a_beam_with_an_inverted_element(require_gpu, cls):
+    """Admissible states have a finite energy, the same in the fused and the separate call; with det F < 0
+    in one element it is NaN (ln J) without |det F| and finite with it."""
+    p, adj, u0 = build_beam_problem(12, 3, 3)
+    u = _state(p, u0, 5, amp=2e-4)
+    for turned in (False, True):
+        v = u.copy()
+        if turned:  # one node moved through its neighbours' faces
+            v[3 * (u.size // 6):][:3] += [0.2, 0.0, 0.0]
+        for absdet in (False, True):
+            asm = cls(p, None, adj, use_abs_det=absdet)
+            x = asm.create_vec(v[asm.layout.perm])
+            g = x.duplicate()
+            both = [float(asm.energy_device(x.t).item()), float(asm.energy_grad_hessian_device(x.t, g.t).item())]
+            if turned and not absdet:
+                assert np.isnan(both).all()
+            else:
+                assert np.isfinite(both).all() and abs(both[0] - both[1]) <= 4 * np.finfo(float).eps * abs(both[0])
+            asm.cleanup()

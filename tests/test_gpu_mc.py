@@ -150,6 +150,37 @@ def test_rows_without_units_match_the_oracle(require_gpu, degree, h, order, prec
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
 @pytest.mark.parametrize("degree", [4, 2])
+@pytest.mark.parametrize("points", [20, 21])  # the last of the shorter K range, and the longer one
+def test_quadrature_of_20_and_21_points(require_gpu, points, degree, precision):
+    """The 19-point rule with its last points split in two halves of their weight integrates the same:
+    the oracle's results, within the tolerances of the tests above."""
+    p, adj = mc_params(h=4.0, degree=degree, lam=1.5)
+    nq = p["wq"].size
+    split = np.arange(nq - (points - nq), nq)
+    take = np.append(np.arange(nq), split)
+    w = p["wq"].copy()
+    w[split] *= 0.5
+    q = dict(p, xq=p["xq"][take], wq=w[take], phi=p["phi"][:, take], dhat=p["dhat"][take])
+    assert q["wq"].size == points
+    asm = SlopeStabilityReorderedElementAssembler(q, None, adj, hessian_precision=precision)
+    lay = asm.layout
+    u = _state(p, lay, 7)
+    ref = assembly.assemble("mc", p, u)
+    x = asm.create_vec(u[lay.perm])
+    g, y = x.duplicate(), x.duplicate()
+    e = float(asm.energy_grad_hessian_device(x.t, g.t).item())
+    H = asm.A.to_scipy()[lay.iperm][:, lay.iperm]
+    assert abs(e - ref["e"]) <= 1e-12 * abs(ref["e"])
+    assert np.abs(g.array[lay.iperm] - ref["g"]).max() <= 1e-11 * np.abs(ref["g"]).max()
+    assert abs(H - ref["h"]).max() <= (1e-10 if precision == "fp64" else 3e-5) * abs(ref["h"]).max()
+    asm.hvp_device(x.t, x.t, y.t)
+    want = ref["h"] @ u
+    assert np.abs(y.array[lay.iperm] - want).max() <= 1e-10 * np.abs(want).max()
+    asm.cleanup()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("degree", [4, 2])
 @pytest.mark.parametrize("cls", [SlopeStabilityReorderedElementAssembler, _SingleRows])
 def test_free_node_without_elements(require_gpu, cls, degree, precision):
     """A free node that no element names has CSR rows without entries: nothing is read or stored for them,
