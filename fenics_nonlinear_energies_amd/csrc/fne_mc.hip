@@ -210,11 +210,9 @@ template <> struct Pair<double> {
 __device__ __forceinline__ float mc_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double mc_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
-// blocks of the element kernel, each with `rounds` rounds of consecutive elements; by_rows: element
-// matrices row by row, for plans without row units
+// blocks of the element kernel, each with `rounds` rounds of consecutive elements
 struct McBlocks {
   int rounds = 1, all = 1;
-  bool by_rows = false;
 };
 
 // LDS of one wavefront
@@ -230,8 +228,9 @@ struct McWaveLds {
 
 // Values of an element matrix in the scratch, [n][m][j][i]: rows (n, i), columns (m, j).  The node rows
 // of P4 have 16 columns: 256 B (FP32) or 512 B at multiples of that, so that the row gather reads two
-// lines of 128 B for each instead of 2.75 (32,000 elements, assembly 140 -> 127 us).  With by_rows a row
-// (n, i) is kMcNodeRow / 2 values in the order of its columns.
+// lines of 128 B for each instead of 2.75 (32,000 elements, assembly 140 -> 127 us).  Plans without
+// row units store row (n, i) as kMcNodeRow / 2 values in the order of its columns instead (BY_ROWS: a
+// branch at run time spills two registers more, 98,000 elements 370 -> 376 us).
 template <int NN>
 constexpr int kMcNodeRow = 4 * (NN == 15 ? 16 : NN);
 template <int NN>
@@ -254,7 +253,7 @@ constexpr int kMcMatrix = NN * kMcNodeRow<NN>;
 // 98,000 elements 221 -> 154 us (matrix units busy 60, VALU 60 of it, 376 MB stored); P2 FP64, 21,978
 // elements, Hessian alone 65 -> 39 us, gradient alone 11.8 -> 10.8; product with a direction, P4,
 // 32,000 elements 46 -> 22 us.
-template <int NN, int NS, typename HT, bool WE, bool WG, bool WH, bool HV>
+template <int NN, int NS, typename HT, bool WE, bool WG, bool WH, bool HV, bool BY_ROWS>
 __global__ __launch_bounds__(kBlock, WH && sizeof(HT) == 8 && (WG || (NN == 15 && NS == 11)) ? 3 : 4) void mc_elem_kernel(
     fne_plan_desc d, McConst k, const double* __restrict__ x, const double* __restrict__ dvals,
     const double* __restrict__ f, const double* __restrict__ vin, EnergySum energy,
@@ -460,7 +459,7 @@ __global__ __launch_bounds__(kBlock, WH && sizeof(HT) == 8 && (WG || (NN == 15 &
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               const int row = Vec4<HT>::row(kk, r);  // 2 n + i
-              const int to = B.by_rows ? (row & 1) * (kMcNodeRow<NN> / 2) + c15 : c15 * 2 + (row & 1);
+              const int to = BY_ROWS ? (row & 1) * (kMcNodeRow<NN> / 2) + c15 : c15 * 2 + (row & 1);
               if (row < NL) H[(row >> 1) * kMcNodeRow<NN> + to] = acc[r];
             }
           }
@@ -483,13 +482,15 @@ __global__ __launch_bounds__(kBlock, WH && sizeof(HT) == 8 && (WG || (NN == 15 &
 #pragma unroll
           for (int r = 0; r < 4; ++r) {  // column 15 is zero
             const int n = Vec4<HT>::row(kk, r);
-            if (n < NN && !B.by_rows) {
-              V4 v = {axx[r], ayx[r], axy[r], ayy[r]};
-              *reinterpret_cast<V4*>(H + n * kMcNodeRow<NN> + c15 * 4) = v;
-            } else if (n < NN) {
-              HT2* to = reinterpret_cast<HT2*>(H + n * kMcNodeRow<NN>) + c15;
-              to[0] = HT2{axx[r], axy[r]};
-              to[kMcNodeRow<NN> / 4] = HT2{ayx[r], ayy[r]};
+            if (n < NN) {
+              if constexpr (BY_ROWS) {
+                HT2* to = reinterpret_cast<HT2*>(H + n * kMcNodeRow<NN>) + c15;
+                to[0] = HT2{axx[r], axy[r]};
+                to[kMcNodeRow<NN> / 4] = HT2{ayx[r], ayy[r]};
+              } else {
+                V4 v = {axx[r], ayx[r], axy[r], ayy[r]};
+                *reinterpret_cast<V4*>(H + n * kMcNodeRow<NN> + c15 * 4) = v;
+              }
             }
           }
         }
@@ -856,8 +857,8 @@ template <int NN>
 int launch_mc(fne_plan* plan, FneOp op, const FneCall& c) {
   const fne_plan_desc& d = plan->d;
   const int ne = d.n_elem;
-  McBlocks B = mc_blocks(ne);
-  B.by_rows = plan->units.n_unit == 0 && op != kOpElementEval;
+  const McBlocks B = mc_blocks(ne);
+  const bool by_rows = plan->units.n_unit == 0;
   const int nb = B.all;
   if (nb > plan->n_partials) {
     fne_set_error("energy reduction scratch too small");
@@ -870,19 +871,27 @@ int launch_mc(fne_plan* plan, FneOp op, const FneCall& c) {
   const EnergySum energy = fne_energy_sum(plan, op, nb, c.out);
   double* gb = plan->mc_g;
   void* hb = plan->mc_h;
-#define MC_ELEM_NS(NS, HT, E, G, H, FV, EV)                                                                      \
-  hipLaunchKernelGGL((mc_elem_kernel<NN, NS, HT, E, G, H, false>), dim3(nb), dim3(kBlock), 0, c.stream, d, k, c.x, \
+#define MC_ELEM_GO(NS, HT, E, G, H, R, FV, EV)                                                                      \
+  hipLaunchKernelGGL((mc_elem_kernel<NN, NS, HT, E, G, H, false, R>), dim3(nb), dim3(kBlock), 0, c.stream, d, k, c.x, \
                      c.dvals, FV, (const double*)nullptr, energy, EV, gb, (HT*)hb, B)
   // NS: products of four K rows that cover 2 n_q
-#define MC_ELEM(HT, E, G, H, FV, EV)            \
+#define MC_ELEM_R(HT, E, G, H, R, FV, EV)       \
   do {                                          \
     if (d.nq <= 20)                             \
-      MC_ELEM_NS(10, HT, E, G, H, FV, EV);      \
+      MC_ELEM_GO(10, HT, E, G, H, R, FV, EV);   \
     else                                        \
-      MC_ELEM_NS(11, HT, E, G, H, FV, EV);      \
+      MC_ELEM_GO(11, HT, E, G, H, R, FV, EV);   \
+  } while (0)
+  // (only matrices are stored in two ways)
+#define MC_ELEM(HT, E, G, H, FV, EV)            \
+  do {                                          \
+    if (H && by_rows)                           \
+      MC_ELEM_R(HT, E, G, H, H, FV, EV);        \
+    else                                        \
+      MC_ELEM_R(HT, E, G, H, false, FV, EV);    \
   } while (0)
   if (op == kOpElementEval) {
-    MC_ELEM(double, false, true, true, (const double*)nullptr, c.e_out);
+    MC_ELEM_R(double, false, true, true, false, (const double*)nullptr, c.e_out);
     FNE_LAUNCH_CHECK();
     if (c.ge_out || c.he_out) {
       hipLaunchKernelGGL(mc_element_out_kernel<NN>, dim3((ne + kBlock - 1) / kBlock), dim3(kBlock), 0, c.stream,
@@ -920,7 +929,8 @@ int launch_mc(fne_plan* plan, FneOp op, const FneCall& c) {
     MC_ELEM(double, true, false, false, c.f, none);
   }
 #undef MC_ELEM
-#undef MC_ELEM_NS
+#undef MC_ELEM_R
+#undef MC_ELEM_GO
   FNE_LAUNCH_CHECK();
   if (want_e) {
     const int rc = fne_finalize_energy(plan, nb, c.out, c.stream);
@@ -1039,7 +1049,7 @@ int launch_mc_aux(fne_plan* plan, const double* x, const double* dvals, const do
   if (v) {
     const double* none = nullptr;
 #define MC_HVP(NS)                                                                                                 \
-  hipLaunchKernelGGL((mc_elem_kernel<NN, NS, double, false, true, false, true>), grid, dim3(kBlock), 0, stream, d, k, \
+  hipLaunchKernelGGL((mc_elem_kernel<NN, NS, double, false, true, false, true, false>), grid, dim3(kBlock), 0, stream, d, k, \
                      x, dvals, none, v, EnergySum{}, (double*)nullptr, plan->mc_g, (double*)nullptr, B)
     if (d.nq <= 20)
       MC_HVP(10);
