@@ -159,8 +159,8 @@ def _spgemm(a_indptr, a_indices, a_data, b: _DevMat, b_data: torch.Tensor, c: _D
 
 
 def _lanczos_work_len(n: int, code: int) -> int:
-    """Doubles of ``fne_lanczos_max``'s work array (``fne_lanczos_work_len``)."""
-    return 6 * n + 512 + 128 + 8 + (n * (((code >> 8) & 0xFF) or 8) + 255) // 256
+    """Doubles of ``fne_lanczos_max``'s work array."""
+    return int(native.lib().fne_lanczos_work_len(n, code))
 
 
 def _spgemm_smoothed(a_indptr, a_indices, a_data, b: _DevMat, c: _DevMat, w: torch.Tensor):
@@ -317,7 +317,7 @@ class SmoothedAggregationPC:
         ``pmg.py``); aggregation continues below the last of them with ``coarse_near_nullspace``
         (rows of the coarsest fixed level; default: the near-nullspace injected through the
         transfers' unit rows).  ``coarse_factor``: where the coarsest operator's dense FP64 inverse
-        is computed at set-up, "host" (LAPACK) or "device" (the GPU's dense solvers, no host
+        is computed at set-up, "host" (LAPACK) or "device" (``fne_spd_inverse``, no host
         round trip); the cycle applies it on the device either way.  The two agree to rounding;
         the inexact Newton paths built on them can differ by an iteration or two."""
         if smoother not in ("jacobi", "chebyshev"):
@@ -441,15 +441,14 @@ class SmoothedAggregationPC:
         self._coarse_n = nc
         # first use of the dense solvers of the coarse inverse at the coarse size (library
         # loading, thread pools, device solver handles), here in the symbolic phase rather than in
-        # whichever numeric set-up first needs them: a definite operator (Cholesky) and an
-        # indefinite one (the eigendecomposition fallback)
+        # whichever numeric set-up first needs them: LAPACK with a definite operator (Cholesky) and an
+        # indefinite one (the eigendecomposition); on the device only the fallback of fne_spd_inverse
         warm = np.diag(np.linspace(1.0, 2.0, nc))
         warm_indef = warm.copy()
         warm_indef[0, 0] = -1.0
         if self.coarse_factor == "device" and torch.device(device).type == "cuda":
             rows = np.repeat(np.arange(nc, dtype=np.int64), np.diff(A_pat.indptr))
             self._coarse_flat = torch.as_tensor(rows * nc + A_pat.indices.astype(np.int64)).to(device)
-            coarse_inverse_device(torch.as_tensor(warm, device=device))
             coarse_inverse_device(torch.as_tensor(warm_indef, device=device))
         else:
             coarse_inverse(warm)

@@ -205,7 +205,7 @@ class ReorderedElementAssemblerBase:
         reference passes them): ``mg_levels_ksp_type`` ("chebyshev", the default as in PCGAMG,
         or "richardson" = damped Jacobi sweeps) and ``mg_levels_ksp_max_it`` (steps per level and
         side, 2 by default); and this build's ``mg_coarse_factor`` ("host": LAPACK, the default,
-        or "device": the GPU's dense solvers) for the coarsest level's inverse.  Other options
+        or "device": ``fne_spd_inverse``) for the coarsest level's inverse.  Other options
         have no counterpart on this solver stack and are ignored."""
         opts = {str(k).lstrip("-"): v for k, v in dict(pc_options or {}).items()}
         kind = str(opts.get("mg_levels_ksp_type", "chebyshev")).lower()
