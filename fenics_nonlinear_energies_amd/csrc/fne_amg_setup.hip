@@ -7,9 +7,11 @@
 // them per set-up and three host reads when written as vector operations.  Here a Lanczos step is
 // two launches (the scalars stay on the device as per-block partial sums that the next launch adds up
 // itself), a level's copies and permutations are one each, and the dense inverse is one launch per 32
-// columns.  Everything is deterministic: sums are taken in a fixed order.
-// Set-up and solve of the 383x383 p-Laplace system (three levels above 286 unknowns, 10 CG iterations):
-// 6.48 -> 3.12 ms, of which kernels 5.31 -> 3.16.
+// columns and one more.  Everything is deterministic: sums are taken in a fixed order.
+// Assembly, set-up and solve of the 383x383 p-Laplace system (three levels above 286 unknowns, 10 CG
+// iterations), pass after pass: 6.48 -> 3.12 ms by this file, 2.20 with the cycle's passes of fne_amg.hip.
+// The set-up alone, waited for: 383x383 p-Laplace 4.53 -> 0.89 ms, 320x16x16 beam with six rigid-body
+// modes 16.1 -> 8.6, P4 slope by p-multigrid (128,080 unknowns) 6.28 -> 1.32.
 #include "fne_common.h"
 
 #include <algorithm>
@@ -122,7 +124,7 @@ __global__ __launch_bounds__(kLanThreads) void lanczos_update_kernel(int n, cons
 
 // Largest eigenvalue of the symmetric tridiagonal (alpha, beta) by multisection: the leading minors of
 // x - T are all positive exactly where x is above every eigenvalue (T scaled to its bound, so that
-// the minors stay in range; products instead of the pivots' quotients, 17 -> 5 us).  64 points per
+// the minors stay in range; products instead of the pivots' quotients, 17 -> 10 us in a kernel trace).  64 points per
 // round, so 6 bits each; 11 rounds.  out = {max(lambda, 1e-300), 1 if every coefficient is finite else 0}.
 __global__ __launch_bounds__(kLanThreads) void lanczos_eig_kernel(int k, const double* __restrict__ alpha,
                                                                   const double* __restrict__ beta,

@@ -282,8 +282,8 @@ void fne_set_error(const std::string& msg) { g_last_error = msg; }
 
 // Workgroups up to which an energy's launch adds its own partial sums up (EnergySum): the release of
 // each arrival writes its XCD's L2 back, some 70 ns one after the other, against 3 to 5 us for a
-// launch of finalize_pairs_kernel (10 workgroups of the 32x32 Ginzburg-Landau grid 10.6 -> 9.1 us,
-// energy alone 7.5 -> 4.6; 128 workgroups 7.6 -> 9.5).
+// launch of finalize_pairs_kernel (32x32 Ginzburg-Landau grid: the 5 workgroups of the fused call 10.3 ->
+// 9.1 us, the 4 of the energy alone 7.5 -> 4.6; an energy of 128 workgroups 7.6 -> 9.5).
 static bool energy_in_launch(int nblocks) {
   constexpr int kEnergyInLaunch = 32;
   return nblocks <= kEnergyInLaunch;

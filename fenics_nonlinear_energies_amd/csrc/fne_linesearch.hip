@@ -6,7 +6,7 @@
 // points and their values, the best point so far and the next alpha to evaluate, so the host enqueues
 // the whole search and synchronises once at the end.  A point is two launches, the energy's partial
 // sums and golden_point_kernel (fne_golden_search); both are bound by latency (4.7 and 3.8 us on the
-// 160x8x8 beam, 24 points 232 to 251 us; four launches per point enqueued one by one took 404 to 438).
+// 160x8x8 beam, 24 points 210 to 256 us; four launches per point enqueued one by one took 404 to 461).
 // fne_golden_trial and fne_golden_step are the same steps for energies that the caller evaluates.
 // The arithmetic and the order of every comparison are the reference's (same points, same
 // tie-breaking), so the chosen alpha is the one the host search would choose from the same energies.

@@ -396,14 +396,14 @@ int fne_hvp_tet(fne_plan* plan, const double* x, const double* dvals, const doub
 // both nodes are in the patch it also writes the transposed block of (j, i).  Eight threads per node
 // sum the diagonal block.  Every CSR value is written once, by one thread; no atomics, so results
 // are bitwise reproducible.  Elements on patch borders are evaluated by every patch that touches
-// them (2.3 times each on the beam), which costs less than a pass over memory.  The gradient goes
+// them (2.2 times each on the 160x8x8 beam, 2.3 on 320x16x16), which costs less than a pass over memory.  The gradient goes
 // through the same LDS before the states do.  Sums are FP64 in both precisions (an FP32 value is
 // rounded once: 2.6e-8 from the exact Hessian, 6.4e-8 with the row gather's FP32 sums).
 // What bounds it: latency.  A workgroup lives ~18k cycles, of which 6.6k are the element phase (two
 // dependent gathers and ~350 FP64 operations), 6k the blocks (LDS reads at random slots), 2k the
 // energy's compensated sum; HBM moves under 2 TB/s.
 // Fused call, before (element matrices + row gather + separate energy) and after, us:
-//   160x8x8 FP64 61.2 -> 20, 320x16x16 FP32 318 -> 70.
+//   160x8x8 FP64 61.5 -> 16.7, 320x16x16 FP32 318 -> 62.4 (back to back, with the final sum).
 // Slot stride 26 doubles (52 words): 16 consecutive slots start in 16 bank groups.
 // ---------------------------------------------------------------------------------------------
 namespace {
